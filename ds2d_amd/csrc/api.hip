@@ -92,7 +92,7 @@ struct ds2d_ctx {
     int log_every = 0;      // CG solvers print the residual to stderr every this many iterations (0: never)
     int use_graph = 0;  // capture time loops into one hipGraph per loop
     int per_launch = 0; // plain Born/adjoint: shots per time loop (0: all)
-    int fwd_two = 0;    // autotuned: mode 2 runs the two-kernel step instead of the fused one
+    int fwd_two = 0;    // autotuned: mode 2 runs the two-kernel step (1) or the tiles of two steps (2) instead of the march
     int acou_fused = -1;  // fused Born/adjoint steps: -1 auto, 0 never, 1 whenever eligible
     int src_fp64 = 1;     // reference-compat gradient: background and first-order Born field in FP64
     std::vector<int> shot_status;  // per shot of the last reference-compat gradient: 1 = left out (non-finite)
@@ -310,6 +310,17 @@ int stats_end(ds2d_ctx* h, ds2d_stats* out, long long cell_updates, long long la
     if (out) *out = h->last;
     return 0;
 }
+
+// Compute units of the device (256 on the MI355X when the query fails).
+int device_cus() {
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess || ncu < kPlanXcds) ncu = 256;
+    return ncu;
+}
+
+// Rounds of tiles beyond which the two-kernel step is faster anyway (2.2 M
+// cells: 47 against 40 us a step), so the autotuner does not time them.
+constexpr long long TILE_MAX_ROUNDS = 16;
 
 int check_h(ds2d_ctx* h) {
     if (!h) return fail(DS2D_EINVAL, "null handle");
@@ -788,9 +799,23 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         if (S.boundary == 0 && S.pml >= NOP)
             pml_cells += (double)(S.nxp - 2 * NOP) * (S.nzp - 2 * NOP) -
                          (double)(S.nxp - 2 * S.pml + 1) * (S.nzp - 2 * S.pml + 1);
+    // Tiles of two steps a launch (kernels_tile.hip): when the autotuner picked
+    // them, or untuned on batches of up to eight rounds of tiles.  There a
+    // launch takes 12 us a round for two steps against 47-85 us a step for the
+    // untuned march of 64 columns (1.07 M cells, 5.6 rounds: 33 against 85 us
+    // a step with the PML); from about twelve rounds on the march is as fast.
+    TilePlan tp{};
+    bool tile = false;
+    if (mode == 2 && n <= FUSED_MAX_CELLS) {
+        std::vector<int> nxp;
+        for (const SlotDesc& q : B.slots) nxp.push_back(q.nxp);
+        tp = plan_tiles(nxp, sh.nzp, device_cus());
+        const bool untuned = !h->fwd_two && !h->chunk_w && !h->chunk_t && !h->chunk_d && h->tblock == 1;
+        tile = h->fwd_two == 2 ? tp.rounds <= TILE_MAX_ROUNDS : untuned && tp.rounds <= 8;
+    }
     long long launches = 0;
     StepSampler smp;
-    if ((rc = smp.init(nt))) return rc;
+    if (!tile && (rc = smp.init(nt))) return rc;
     if (mode == 0) {
         Strain none{nullptr, nullptr, nullptr, nullptr};
         stats_loop_begin(h);
@@ -809,8 +834,8 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         // split layout, per padded cell: v reads 10 writes 6; s reads 12 writes 9
         bytes_v = (double)B.total_cells * 16 * 4;
         bytes_s = (double)B.total_cells * 21 * 4;
-    } else if (mode == 2 && !h->fwd_two && n <= FUSED_MAX_CELLS) {
-        // single fused kernel per step, ping-pong state
+    } else if (mode == 2 && (tile || !h->fwd_two) && n <= FUSED_MAX_CELLS) {
+        // fused kernels, ping-pong state
         float* par;
         int* rmap;
         if ((rc = h->fbuf("fpar", (size_t)n * 3, &par)) || (rc = h->fbuf("rmap", B.total_rmap, &rmap))) return rc;
@@ -824,13 +849,15 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         const int T = h->chunk_t > 0 ? h->chunk_t : 256;
         const int D = h->chunk_d == 4 ? 4 : 2;
         const int rows = T - 2 * FUSED_HALO;
-        for (int s = 0; s < nshots; ++s)
-            for (int x0 = 0; x0 < B.slots[s].nxp; x0 += W)
-                for (int z0 = 0; z0 < B.slots[s].nzp; z0 += rows)
-                    ch.push_back(ChunkDesc{s, x0, std::min(x0 + W, B.slots[s].nxp), z0});
-        ChunkDesc* d_ch;
-        if ((rc = h->fbuf("chunks", ch.size(), &d_ch))) return rc;
-        HIP_TRY(hipMemcpyAsync(d_ch, ch.data(), ch.size() * sizeof(ChunkDesc), hipMemcpyHostToDevice, st));
+        ChunkDesc* d_ch = nullptr;
+        if (!tile) {
+            for (int s = 0; s < nshots; ++s)
+                for (int x0 = 0; x0 < B.slots[s].nxp; x0 += W)
+                    for (int z0 = 0; z0 < B.slots[s].nzp; z0 += rows)
+                        ch.push_back(ChunkDesc{s, x0, std::min(x0 + W, B.slots[s].nxp), z0});
+            if ((rc = h->fbuf("chunks", ch.size(), &d_ch))) return rc;
+            HIP_TRY(hipMemcpyAsync(d_ch, ch.data(), ch.size() * sizeof(ChunkDesc), hipMemcpyHostToDevice, st));
+        }
         auto mk = [&](const EField& A, const EField& Bf) {
             FusedArgs q{};
             q.A = A.vx;  // alloc_efield: 15 fields of n floats from vx on
@@ -845,6 +872,31 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
             return q;
         };
         const FusedArgs even = mk(f, g2), odd = mk(g2, f);
+        if (tile) {
+            std::vector<TileDesc> tiles;
+            for (const SlotDesc& q : B.slots)
+                for (int x0 = NOP; x0 < q.nxp - NOP; x0 += tp.cols)
+                    for (int z0 = NOP; z0 < q.nzp - NOP; z0 += TILE_ROWS)
+                        tiles.push_back(TileDesc{q.off, q.rec_off, x0, z0, q.nxp, q.nzp, q.boundary == 0 ? q.pml : 0,
+                                                 q.isx, q.isz, q.igz, q.rmap_off, {0, 0, 0}});
+            TileDesc* d_tiles;
+            if ((rc = h->fbuf("tiles", tiles.size(), &d_tiles))) return rc;
+            HIP_TRY(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(TileDesc), hipMemcpyHostToDevice, st));
+            int k = 0;
+            auto pair = [&](int it) {
+                launch_tile_steps(st, sh, (k & 1) ? odd : even, d_tiles, (int)tiles.size(), rmap, it,
+                                  std::min(2, nt - it), tp.kind, B.any_pml);
+                ++k;
+            };
+            stats_loop_begin(h);
+            if ((rc = run_steps(h, 0, (nt + 1) / 2, 2, pair))) return rc;
+            stats_loop_end(h);
+            // reported per time step (ds2d_get_time_block is 1 here): the one-step figure of the march, and
+            // half of what a launch of two steps must move (state and parameters once)
+            launches = nt;
+            bytes_v = (double)B.total_cells * 13 * 4 + pml_cells * 12 * 4;
+            blocked = bytes_v / 2;
+        } else
         if (h->tblock == 2 && nt >= 2) {
             // temporal blocking of depth 2: steps (it, it+1) per launch; an odd
             // last step runs the single-step kernel on its own chunk list
@@ -860,11 +912,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
                     nxv[s] = B.slots[s].nxp;
                     nzv[s] = B.slots[s].nzp;
                 }
-                int ncu = 0;
-                if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess ||
-                    ncu < kPlanXcds)
-                    ncu = 256;
-                const int cpx = ncu / kPlanXcds;
+                const int cpx = device_cus() / kPlanXcds;
                 std::vector<int> key{W, rows2, cpx, h->chunk_plan};
                 key.insert(key.end(), nxv.begin(), nxv.end());
                 key.insert(key.end(), nzv.begin(), nzv.end());
@@ -1084,9 +1132,10 @@ int ds2d_autotune_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, int nst
     int rc;
     if ((rc = check_h(h))) return rc;
     struct Cand {
-        int w, t, d, tb;  // x width (0: two-kernel step), lanes, prefetch columns, time steps per launch
+        int w, t, d, tb;  // x width (0: no march), lanes, prefetch columns, time steps per launch
+        int two = 0;      // without a march: 1 the two-kernel step, 2 the tiles of two steps
     };
-    static const Cand cand[] = {{0, 0, 0, 1},     {32, 256, 2, 1},  {64, 256, 2, 1},  {64, 256, 4, 1},
+    static const Cand cand[] = {{0, 0, 0, 1, 1},  {32, 256, 2, 1},  {64, 256, 2, 1},  {64, 256, 4, 1},
                                 {128, 256, 4, 1}, {64, 512, 4, 1},  {64, 768, 2, 1},  {64, 768, 4, 1},
                                 {128, 768, 4, 1}, {64, 704, 4, 1},  {112, 704, 4, 1}, {160, 704, 4, 1},
                                 {64, 704, 2, 2},  {128, 704, 2, 2}};
@@ -1120,6 +1169,12 @@ int ds2d_autotune_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, int nst
             cands.push_back(Cand{lo, 704, 2, 2});
         }
     }
+    {
+        std::vector<int> nxp;
+        for (int i = 0; i < nshots; ++i) nxp.push_back(shots[i].nx + 2 * h->g.pml);
+        if (plan_tiles(nxp, h->g.allnz + 2 * h->g.pml, device_cus()).rounds <= TILE_MAX_ROUNDS)
+            cands.push_back(Cand{0, 0, 0, 1, 2});
+    }
     Cand best{64, 256, 2, 1};
     double bt = 1e300;
     const int keep_w = h->chunk_w, keep_t = h->chunk_t, keep_d = h->chunk_d, keep_two = h->fwd_two,
@@ -1127,7 +1182,7 @@ int ds2d_autotune_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, int nst
     h->use_graph = 0;  // candidates are timed as direct launches (a short capture would time its instantiation)
     for (const Cand& c : cands) {
         if (c.tb == 2 && nsteps < 2) continue;
-        h->fwd_two = c.w == 0;
+        h->fwd_two = c.two;
         h->chunk_w = c.w;
         h->chunk_t = c.t;
         h->chunk_d = c.d;
@@ -1152,7 +1207,7 @@ int ds2d_autotune_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, int nst
         }
     }
     h->use_graph = keep_graph;
-    h->fwd_two = best.w == 0;
+    h->fwd_two = best.two;
     h->chunk_w = best.w;
     h->chunk_t = best.t;
     h->chunk_d = best.d;

@@ -1,5 +1,7 @@
 // Host-side launchers of the DS2D gfx950 kernels.
 #pragma once
+#include <vector>
+
 #include "common.hpp"
 
 namespace ds2d {
@@ -307,5 +309,28 @@ bool fused2_threads_ok(int threads);
 void launch_fused2_step(hipStream_t st, const BatchShape& b, const FusedArgs& a, float* scratch,
                         const ChunkDesc* chunks, int nchunks, const int* rmap, int it, int threads, int depth,
                         bool pml);
+
+// --- elastic step on tiles, two time steps per launch (kernels_tile.hip) ----
+// One tile: all that a workgroup needs of its window (one 64-byte load).
+struct TileDesc {
+    long long off, rec_off;
+    int x0, z0;     // first owned column and row
+    int nxp, nzp;
+    int pml;        // frame width of a PML window, 0 with the random boundary
+    int isx, isz, igz;
+    int rmap_off;
+    int pad[3];
+};
+constexpr int TILE_HALO = 16, TILE_ROWS = 64 - 2 * TILE_HALO, TILE_KINDS = 4;
+struct TilePlan {
+    int kind, cols;    // tile and its owned columns
+    long long rounds;  // rounds of one workgroup per CU
+    float us;          // estimate of one launch
+};
+// The tile whose rounds of the chip cost least for windows of nxp columns and nzp rows.
+TilePlan plan_tiles(const std::vector<int>& nxp, int nzp, int ncu);
+// Steps it .. it + ns - 1 (ns 1 or 2), state A -> B.
+void launch_tile_steps(hipStream_t st, const BatchShape& b, const FusedArgs& a, const TileDesc* tiles, int ntiles,
+                       const int* rmap, int it, int ns, int kind, bool pml);
 
 }  // namespace ds2d

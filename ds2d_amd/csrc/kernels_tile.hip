@@ -1,0 +1,341 @@
+// Elastic forward step for batches too small to fill the chip with x-marching
+// workgroups (gfx950): two time steps per launch on two-dimensional tiles,
+// batched over uneven shot windows.
+//
+// Scheme, arithmetic, damping strips, source and recorder are those of the
+// fused step (born.cu:215-349, FD2DGPU.cu:2039-2049, 355-365).
+//
+// What bounds a small batch is the length of a launch, not its traffic: a
+// workgroup that marches 64 columns has 80 columns in series (82 us a step on
+// one 141x101 padded window, 84 us on 291x141), and a launch per half step
+// costs two launches (8.4-10.8 us a step).  Here every cell of a tile is loaded
+// at once and a launch takes two steps, one wave per column of 64 rows: the
+// state stays in registers, x neighbours come from LDS, z neighbours from the
+// lanes beside (wave shifts), so a half step is one LDS exchange and about 60
+// vector operations a column.  Each step spends four columns and rows on each
+// side on the velocity and four on the stress, so a tile owns all but its 16
+// outer ones.  Measured per launch on 291x141 with the PML: 4.4 us for the
+// loads and stores alone, 9.2 us for two steps (4.6 us a step against 84 and
+// 10.8); with the random boundary 7.0 us (3.5 a step).  Three steps a launch
+// would leave 16 of 64 rows owned and cost more than the saved launch.
+// Columns are dealt to the waves in turn (column = unit * waves + wave), which
+// keeps all SIMDs busy as the active columns shrink from half step to half
+// step; contiguous columns, whose x taps would partly come from registers,
+// measured the same on one round and 10 % slower over several.
+#include "common.hpp"
+#include "kernels.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace ds2d {
+
+namespace {
+
+// The value of the next (previous) lane of the wave: the cell below (above).
+__device__ __forceinline__ float next_z(float f) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float prev_z(float f) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float taps(float a1, float b1, float a2, float b2, float a3, float b3, float a4, float b4) {
+    return DS2D_C1 * (a1 - b1) + DS2D_C2 * (a2 - b2) + DS2D_C3 * (a3 - b3) + DS2D_C4 * (a4 - b4);
+}
+// Forward and backward half-point differences along z.
+__device__ __forceinline__ float dplus_z(float f) {
+    const float p1 = next_z(f), p2 = next_z(p1), p3 = next_z(p2), p4 = next_z(p3);
+    const float m1 = prev_z(f), m2 = prev_z(m1), m3 = prev_z(m2);
+    return taps(p1, f, p2, m1, p3, m2, p4, m3);
+}
+__device__ __forceinline__ float dminus_z(float f) {
+    const float p1 = next_z(f), p2 = next_z(p1), p3 = next_z(p2);
+    const float m1 = prev_z(f), m2 = prev_z(m1), m3 = prev_z(m2), m4 = prev_z(m3);
+    return taps(f, m1, p1, m2, p2, m3, p3, m4);
+}
+
+// Weight of the cell at offset d in a forward half-point difference.
+__device__ __forceinline__ float src_tap(int d) {
+    return d == 1 ? DS2D_C1 : d == 2 ? DS2D_C2 : d == 3 ? DS2D_C3 : d == 4 ? DS2D_C4 :
+           d == 0 ? -DS2D_C1 : d == -1 ? -DS2D_C2 : d == -2 ? -DS2D_C3 : d == -3 ? -DS2D_C4 : 0.f;
+}
+
+}  // namespace
+
+template <int K, int NW, bool PML>
+__global__ __launch_bounds__(NW * 64) void k_tile_steps(FusedArgs a, const TileDesc* __restrict__ tiles, int ntiles,
+                                                        int per_xcd, const int* __restrict__ rmap, float idx,
+                                                        float idz, float dt, int nt, int it, int ns) {
+    constexpr int RX = K * NW, RZ = 64, HALO = TILE_HALO;
+    const int b = blockIdx.x;
+    const int ch = (b % 8) * per_xcd + b / 8;
+    if (ch >= ntiles) return;
+    const TileDesc T = tiles[ch];
+    // four spare rows on each side, so that the x taps of every row stay inside
+    __shared__ float lds[4][(RX + 8) * RZ];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto row = [&](int k) { return k * NW + wv; };  // column of the tile, uniform over the wave
+    auto at = [&](int f, int k) { return &lds[f][(row(k) + 4) * RZ + lane]; };
+    const int z = T.z0 - HALO + lane, ix0 = T.x0 - HALO;
+    const bool zu = z >= NOP && z < T.nzp - NOP;
+    const bool zd = PML && T.pml > 0 && (z < T.pml || z > T.nzp - T.pml);
+    const bool zown = lane >= HALO && lane < RZ - HALO && zu;
+    const long long n = a.n;
+
+    // Each component as the sum of two parts.  In a damped cell they are its x
+    // and z splits, which are what its window's strips store (the sum alone with
+    // one split would round the other one off at every step); elsewhere the
+    // first is the component.
+    float vx[K], vz[K], xx[K], zz[K], xz[K], vxb[K], vzb[K], xxb[K], zzb[K], xzb[K];
+    float bx[K], lam[K], mu[K], ex[K], ez[K];
+    auto row_upd = [&](int k) { const int ix = ix0 + row(k); return ix >= NOP && ix < T.nxp - NOP; };
+    auto row_damp = [&](int k) { const int ix = ix0 + row(k); return T.pml > 0 && (ix < T.pml || ix > T.nxp - T.pml); };
+    auto cell = [&](int k) { return (uint32_t)(T.off + (long long)(ix0 + row(k)) * T.nzp + z); };
+    const bool near4 = lane >= 4 && lane < RZ - 4, near8 = lane >= 8 && lane < RZ - 8;
+    bool damped = PML && __any(zd);  // whether any cell of this wave is
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        vx[k] = vz[k] = xx[k] = zz[k] = xz[k] = vxb[k] = vzb[k] = xxb[k] = zzb[k] = xzb[k] = 0.f;
+        bx[k] = lam[k] = mu[k] = ex[k] = ez[k] = 0.f;
+        const int r = row(k);
+        damped = damped || (PML && row_damp(k));
+        if (row_upd(k) && zu) {
+            const uint32_t c = cell(k);
+            const bool dmp = PML && (zd || row_damp(k));
+            xx[k] = (a.A + (dmp ? 9 : 2) * n)[c];
+            xz[k] = (a.A + (dmp ? 13 : 4) * n)[c];
+            zz[k] = (a.A + (dmp ? 11 : 3) * n)[c];
+            if (dmp) {
+                xxb[k] = (a.A + 10 * n)[c];
+                xzb[k] = (a.A + 14 * n)[c];
+                zzb[k] = (a.A + 12 * n)[c];
+            }
+            if (r >= 4 && r < RX - 4 && near4) {
+                vx[k] = (a.A + (dmp ? 5 : 0) * n)[c];
+                vz[k] = (a.A + (dmp ? 7 : 1) * n)[c];
+                bx[k] = a.par[c];
+                if (dmp) {
+                    vxb[k] = (a.A + 6 * n)[c];
+                    vzb[k] = (a.A + 8 * n)[c];
+                    ex[k] = a.dampx[c];
+                    ez[k] = a.dampz[c];
+                }
+                if (r >= 8 && r < RX - 8 && near8) {
+                    lam[k] = (a.par + n)[c];
+                    mu[k] = (a.par + 2 * n)[c];
+                }
+            }
+        }
+    }
+    // traces of the wave's columns: lane k holds column k's (-1: none)
+    int rec = -1;
+    if (T.igz >= T.z0 && T.igz < T.z0 + RZ - 2 * HALO && lane < K) {
+        const int ix = ix0 + lane * NW + wv;
+        if (ix >= NOP && ix < T.nxp - NOP) rec = rmap[T.rmap_off + ix];
+    }
+    const float w0 = a.wav[it], w1 = ns > 1 ? a.wav[it + 1] : 0.f;
+    // weight of the source in the z derivative of this lane's row
+    const float cz_src = src_tap(T.isz - z);
+    float d1[K], r2[K], d3[K], r4[K];
+    if (PML && damped) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            d1[k] = 1.f - dt * ex[k] / 2;
+            r2[k] = __builtin_amdgcn_rcpf(1.f + dt * ex[k] / 2);
+            d3[k] = 1.f - dt * ez[k] / 2;
+            r4[k] = __builtin_amdgcn_rcpf(1.f + dt * ez[k] / 2);
+        }
+    }
+
+    // One step that leaves out the MV outer columns and rows in the velocity and four more in the stress.
+    auto velocity = [&](auto mvc, auto dc, float w, int step) {
+        constexpr int MV = decltype(mvc)::value;
+        constexpr bool DAMP = decltype(dc)::value;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int r = row(k);
+            const float *X = at(0, k), *Z = at(1, k);
+            float x[7], e[7];
+#pragma unroll
+            for (int i = 0; i < 7; ++i) {
+                x[i] = X[(i < 3 ? i - 3 : i - 2) * RZ];
+                e[i] = Z[(i < 4 ? i - 4 : i - 3) * RZ];
+            }
+            const bool all = k * NW >= MV && k * NW + NW <= RX - MV;
+            if (!all && (r < MV || r >= RX - MV)) continue;
+            const float txz = DAMP ? xz[k] + xzb[k] : xz[k];
+            float ax = taps(x[3], DAMP ? xx[k] + xxb[k] : xx[k], x[4], x[2], x[5], x[1], x[6], x[0]);
+            const float ez_ = taps(txz, e[3], e[4], e[2], e[5], e[1], e[6], e[0]);
+            const float bz = dminus_z(txz);
+            float cz = dplus_z(DAMP ? zz[k] + zzb[k] : zz[k]);
+            // the source sample, present in this step's velocity only
+            const int dx = T.isx - ix0 - r;
+            if ((unsigned)(dx + 3) < 8u) {
+                if (z == T.isz) ax += w * src_tap(dx);
+                if (dx == 0) cz += w * cz_src;
+            }
+            const bool u = zu && row_upd(k);
+            const float nx = vx[k] + bx[k] * (ax * idx + bz * idz);
+            const float nz = vz[k] + bx[k] * (ez_ * idx + cz * idz);
+            if (DAMP) {
+                const bool d = zd || row_damp(k);
+                const float ux = (d1[k] * vx[k] + bx[k] * idx * ax) * r2[k];
+                const float uz = (d3[k] * vxb[k] + bx[k] * idz * bz) * r4[k];
+                const float wx = (d1[k] * vz[k] + bx[k] * idx * ez_) * r2[k];
+                const float wz = (d3[k] * vzb[k] + bx[k] * idz * cz) * r4[k];
+                vx[k] = !u ? 0.f : d ? ux : nx;
+                vxb[k] = u && d ? uz : 0.f;
+                vz[k] = !u ? 0.f : d ? wx : nz;
+                vzb[k] = u && d ? wz : 0.f;
+            } else {
+                vx[k] = u ? nx : 0.f;
+                vz[k] = u ? nz : 0.f;
+            }
+            const int tr = __builtin_amdgcn_readlane(rec, k);
+            if (tr >= 0 && z == T.igz && r >= HALO && r < RX - HALO) {
+                const size_t o = (size_t)T.rec_off + (size_t)tr * nt + step;
+                a.rec_z[o] = DAMP ? vz[k] + vzb[k] : vz[k];
+                a.rec_x[o] = DAMP ? vx[k] + vxb[k] : vx[k];
+            }
+        }
+    };
+    auto stress = [&](auto msc, auto dc) {
+        constexpr int MS = decltype(msc)::value;
+        constexpr bool DAMP = decltype(dc)::value;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int r = row(k);
+            const float *X = at(2, k), *Z = at(3, k);
+            float x[7], e[7];
+#pragma unroll
+            for (int i = 0; i < 7; ++i) {
+                x[i] = X[(i < 4 ? i - 4 : i - 3) * RZ];
+                e[i] = Z[(i < 3 ? i - 3 : i - 2) * RZ];
+            }
+            const bool all = k * NW >= MS && k * NW + NW <= RX - MS;
+            if (!all && (r < MS || r >= RX - MS)) continue;
+            const float tvx = DAMP ? vx[k] + vxb[k] : vx[k], tvz = DAMP ? vz[k] + vzb[k] : vz[k];
+            const float dvx = taps(tvx, x[3], x[4], x[2], x[5], x[1], x[6], x[0]) * idx;
+            const float dvzx = taps(e[3], tvz, e[4], e[2], e[5], e[1], e[6], e[0]) * idx;
+            const float dvz = dminus_z(tvz) * idz, dvxz = dplus_z(tvx) * idz;
+            const float l = lam[k], m = mu[k], l2m = l + 2 * m;
+            const bool u = zu && row_upd(k);
+            const float nxx = xx[k] + (l2m * dvx + l * dvz);
+            const float nzz = zz[k] + (l * dvx + l2m * dvz);
+            const float nxz = xz[k] + m * (dvzx + dvxz);
+            if (DAMP) {
+                const bool d = zd || row_damp(k);
+                const float a1 = (d1[k] * xx[k] + l2m * dvx) * r2[k];
+                const float a2 = (d3[k] * xxb[k] + l * dvz) * r4[k];
+                const float b1 = (d1[k] * zz[k] + l * dvx) * r2[k];
+                const float b2 = (d3[k] * zzb[k] + l2m * dvz) * r4[k];
+                const float e1 = (d1[k] * xz[k] + m * dvzx) * r2[k];
+                const float e2 = (d3[k] * xzb[k] + m * dvxz) * r4[k];
+                xx[k] = !u ? 0.f : d ? a1 : nxx;
+                xxb[k] = u && d ? a2 : 0.f;
+                zz[k] = !u ? 0.f : d ? b1 : nzz;
+                zzb[k] = u && d ? b2 : 0.f;
+                xz[k] = !u ? 0.f : d ? e1 : nxz;
+                xzb[k] = u && d ? e2 : 0.f;
+            } else {
+                xx[k] = u ? nxx : 0.f;
+                zz[k] = u ? nzz : 0.f;
+                xz[k] = u ? nxz : 0.f;
+            }
+        }
+    };
+    auto publish = [&](int f, const float* p, const float* pb, const float* q, const float* qb) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            *at(f, k) = PML ? p[k] + pb[k] : p[k];
+            *at(f + 1, k) = PML ? q[k] + qb[k] : q[k];
+        }
+        __syncthreads();
+    };
+    auto one_step = [&](auto mvc, float w, int step) {
+        constexpr int MV = decltype(mvc)::value;
+        publish(0, xx, xxb, xz, xzb);
+        if (PML && damped)
+            velocity(mvc, std::true_type{}, w, step);
+        else
+            velocity(mvc, std::false_type{}, w, step);
+        publish(2, vx, vxb, vz, vzb);
+        if (PML && damped)
+            stress(std::integral_constant<int, MV + 4>{}, std::true_type{});
+        else
+            stress(std::integral_constant<int, MV + 4>{}, std::false_type{});
+    };
+    if (ns > 1) {
+        one_step(std::integral_constant<int, 4>{}, w0, it);
+        one_step(std::integral_constant<int, 12>{}, w1, it + 1);
+    } else {
+        one_step(std::integral_constant<int, 12>{}, w0, it);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int r = row(k);
+        if (!zown || !row_upd(k) || r < HALO || r >= RX - HALO) continue;
+        const uint32_t c = cell(k);
+        if (PML && (zd || row_damp(k))) {
+            const float part[10] = {vx[k], vxb[k], vz[k], vzb[k], xx[k], xxb[k], zz[k], zzb[k], xz[k], xzb[k]};
+#pragma unroll
+            for (int f = 0; f < 10; ++f) (a.B + (5 + f) * n)[c] = part[f];
+        } else {
+            a.B[c] = vx[k] + vxb[k];
+            (a.B + n)[c] = vz[k] + vzb[k];
+            (a.B + 2 * n)[c] = xx[k] + xxb[k];
+            (a.B + 3 * n)[c] = zz[k] + zzb[k];
+            (a.B + 4 * n)[c] = xz[k] + xzb[k];
+        }
+    }
+}
+
+// Columns per wave and waves of the four tiles, and what one round of one
+// workgroup per CU costs per launch of two steps (us, PML windows; measured
+// on 251x101 windows, 1 to 26 of them).
+struct TileKind {
+    int k, nw;
+    float us;
+};
+static const TileKind kTiles[TILE_KINDS] = {{3, 14, 9.2f}, {4, 12, 10.2f}, {4, 14, 12.1f}, {5, 12, 12.5f}};
+
+TilePlan plan_tiles(const std::vector<int>& nxp, int nzp, int ncu) {
+    TilePlan best{0, 0, 0, 0.f};
+    const long long zt = (std::max(nzp - 2 * NOP, 0) + TILE_ROWS - 1) / TILE_ROWS;
+    for (int v = 0; v < TILE_KINDS; ++v) {
+        const int cols = kTiles[v].k * kTiles[v].nw - 2 * TILE_HALO;
+        long long t = 0;
+        for (int w : nxp) t += (std::max(w - 2 * NOP, 0) + cols - 1) / cols * zt;
+        const long long rounds = (t + ncu - 1) / ncu;
+        const float us = rounds * kTiles[v].us;
+        if (v == 0 || us < best.us) best = TilePlan{v, cols, rounds, us};
+    }
+    return best;
+}
+
+void launch_tile_steps(hipStream_t st, const BatchShape& b, const FusedArgs& a, const TileDesc* tiles, int ntiles,
+                       const int* rmap, int it, int ns, int kind, bool pml) {
+    const int per_xcd = (ntiles + 7) / 8;
+    const float idx = 1.f / b.dx, idz = 1.f / b.dz;
+#define DS2D_TILE_LAUNCH(K, NW, MM)                                                                           \
+    hipLaunchKernelGGL((k_tile_steps<K, NW, MM>), dim3(per_xcd * 8), dim3(NW * 64), 0, st, a, tiles, ntiles,  \
+                       per_xcd, rmap, idx, idz, b.dt, b.nt, it, ns)
+#define DS2D_TILE_KIND(V, K, NW)                   \
+    case V:                                        \
+        if (pml)                                   \
+            DS2D_TILE_LAUNCH(K, NW, true);         \
+        else                                       \
+            DS2D_TILE_LAUNCH(K, NW, false);        \
+        break;
+    switch (kind) {
+        DS2D_TILE_KIND(0, 3, 14)
+        DS2D_TILE_KIND(1, 4, 12)
+        DS2D_TILE_KIND(2, 4, 14)
+        DS2D_TILE_KIND(3, 5, 12)
+    }
+#undef DS2D_TILE_KIND
+#undef DS2D_TILE_LAUNCH
+}
+
+}  // namespace ds2d

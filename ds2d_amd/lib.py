@@ -287,7 +287,7 @@ class Solver:
 
     def autotune(self, shots, nsteps=100):
         """Pick the forward step's tile for this batch; returns (width, threads, depth, ms);
-        width 0 means the two-kernel step won."""
+        width 0 means a step without a march won (two kernels, or tiles of two steps per launch)."""
         w, t, d = C.c_int(0), C.c_int(0), C.c_int(0)
         ms = C.c_double(0)
         _check(self.lib.ds2d_autotune_forward(self.h, len(shots), _shots_array(shots), nsteps, C.byref(w),

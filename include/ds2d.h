@@ -157,8 +157,11 @@ int ds2d_calculate_alpha(ds2d_t* h, int nshots, const ds2d_shot* shots, const fl
 int ds2d_forward(ds2d_t* h, float* rec_z, float* rec_x);
 /* Batched forward modelling of many uneven windows.  Records concatenated in
  * shot order, each [ntr_s][nt].  mode: 0 = reference split-field kernels,
- * 1 = two fast kernels per step (unsplit interior), 2 = one fused kernel per
- * step (or what ds2d_autotune_forward picked). */
+ * 1 = two fast kernels per step (unsplit interior), 2 = fused kernels: what
+ * ds2d_autotune_forward picked or ds2d_set_chunk / ds2d_set_time_block fixed,
+ * else tiles of two steps per launch for batches that would not fill the
+ * device with marching workgroups (their stats are per time step), and one
+ * march per step for the others. */
 int ds2d_batch_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z, float* rec_x,
                        int mode, ds2d_stats* stats);
 /* Tile of the fused kernel: x-chunk width (0 = default 64), workgroup size
@@ -166,8 +169,9 @@ int ds2d_batch_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec
  * default 256) and prefetch depth (columns of operands in flight, 2 or 4;
  * 0 = 2; two steps per launch always run with 2); and an autotuner that times
  * nsteps per candidate on this batch -- the fused kernel at several tiles,
- * one or two time steps per launch, and the two-kernel step (reported as
- * width 0) -- and keeps the fastest for mode 2.  No reference counterpart
+ * one or two time steps per launch, and the kernels without a march (the
+ * two-kernel step and, for small batches, the tiles of two steps; both are
+ * reported as width 0) -- and keeps the fastest for mode 2.  No reference counterpart
  * (new capability). */
 int ds2d_set_chunk(ds2d_t* h, int width, int threads, int depth);
 /* Time steps per launch of the fused elastic forward (mode 2): 1, or 2 =
