@@ -525,21 +525,16 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     const BatchShape& sh = B.shape;
     const long long n = B.total_cells;
     hipStream_t st = h->st;
-    EFieldT<TB> bg, b;
-    EField b2, bk, bb;
+    GradFields<TB> F{};
+    EFieldT<TB>&bg = F.bg, &b = F.b;
+    EField &b2 = F.b2, &bk = F.bk, &bb = F.bb;
     Med m;
-    Strain sg, sb;
     const char* tg = sizeof(TB) == 8 ? "bg64" : "bg";
     const char* tb = sizeof(TB) == 8 ? "b64" : "b";
     if ((rc = alloc_efield(h, tg, n, bg)) || (rc = alloc_efield(h, tb, n, b)) ||
         (rc = alloc_efield(h, "b2", n, b2)) || (rc = alloc_efield(h, "bk", n, bk)) ||
         (rc = alloc_efield(h, "bb", n, bb)) || (rc = alloc_med(h, n, m)))
         return rc;
-    float* strain;
-    if ((rc = h->fbuf("strain", (size_t)n * 8, &strain))) return rc;
-    HIP_TRY(hipMemsetAsync(strain, 0, (size_t)n * 8 * 4, st));
-    sg = Strain{strain, strain + n, strain + 2 * n, strain + 3 * n};
-    sb = Strain{strain + 4 * n, strain + 5 * n, strain + 6 * n, strain + 7 * n};
     const size_t R = std::max<long long>(B.total_rec, 1);
     float *rs, *obs;
     if ((rc = h->fbuf("recs", R * 4, &rs)) || (rc = h->fbuf("obs", R * 2, &obs))) return rc;
@@ -552,34 +547,58 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     float* win;
     if ((rc = h->fbuf("win7", (size_t)W * 7, &win))) return rc;
     HIP_TRY(hipMemsetAsync(win, 0, (size_t)W * 7 * 4, st));
-    TB *e_bvx = nullptr, *e_bvz = nullptr, *e_cvx = nullptr, *e_cvz = nullptr;
+    // column -> a trace that records it, trace -> the next one on its column (a column may have several)
+    std::vector<int> map(std::max<long long>(B.total_rmap, 1), -1), next(std::max<size_t>(B.rix.size(), 1), -1);
+    for (const SlotDesc& S : B.slots)
+        for (int r = 0; r < S.ntr; ++r) {
+            int& head = map[S.rmap_off + B.rix[S.rix_off + r]];
+            next[S.rix_off + r] = head;
+            head = r;
+        }
+    int *d_map, *d_next;
+    if ((rc = h->fbuf("gmap", map.size(), &d_map)) || (rc = h->fbuf("gnext", next.size(), &d_next))) return rc;
+    HIP_TRY(hipMemcpyAsync(d_map, map.data(), map.size() * 4, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(d_next, next.data(), next.size() * 4, hipMemcpyHostToDevice, st));
+    const int nt = h->g.nt;
+    GradArgs ga{};
+    ga.n = n;
+    ga.total_edge = B.total_edge;
+    ga.wstride = W;
+    ga.dt = sh.dt;
+    ga.dx = sh.dx;
+    ga.dz = sh.dz;
+    ga.nt = nt;
+    ga.wav = h->d_wav;
+    ga.rmap = d_map;
+    ga.rnext = d_next;
+    ga.rs_z = rs_z;
+    ga.rs_x = rs_x;
+    ga.rs2_z = rs2_z;
+    ga.rs2_x = rs2_x;
+    ga.w7 = win;
+    F.lvx = bg.vx;
+    F.lvz = bg.vz;
+    if (full) {
+        // strains of bg, two sets of products of bk, one of bb, the Born adjoint's modulus
+        float* prod;
+        if ((rc = h->fbuf("gradprod", (size_t)n * 13, &prod))) return rc;
+        HIP_TRY(hipMemsetAsync(prod, 0, (size_t)n * 13 * 4, st));
+        ga.g = prod;
+        ga.wk = prod + 3 * n;
+        ga.pk = prod + 6 * n;
+        ga.wb = prod + 9 * n;
+        ga.cs = prod + 12 * n;
+    }
     if (edges) {
-        TB* e;
-        if ((rc = h->fbuf(sizeof(TB) == 8 ? "edges64" : "edges", (size_t)B.total_edge * 4, &e))) return rc;
-        e_bvx = e; e_bvz = e + B.total_edge; e_cvx = e + 2 * B.total_edge; e_cvz = e + 3 * B.total_edge;
+        TB* lv;
+        if ((rc = h->fbuf(sizeof(TB) == 8 ? "edges64" : "edges", (size_t)B.total_edge * 4, &F.edges)) ||
+            (rc = h->fbuf(sizeof(TB) == 8 ? "edgev64" : "edgev", (size_t)n * 2, &lv)))
+            return rc;
+        F.lvx = lv;
+        F.lvz = lv + n;
     }
     launch_setup(st, sh, setup_args(h, true), m);
-    const int nt = h->g.nt;
-    for (int it = 0; it < nt; ++it) {
-        launch_inject_src(st, sh, bg.txx, bg.tzz, h->d_wav, it);
-        launch_ref_v(st, sh, bg, m, 1.f, 0);
-        launch_ref_s(st, sh, bg, m, sg, 1.f, 0);
-        launch_born_src(st, sh, bg.vx, bg.vz, b, m, 1.f);
-        launch_ref_v(st, sh, b, m, 1.f, 0);
-        launch_ref_s(st, sh, b, m, sg, 1.f, 0);
-        if (second) {
-            launch_born_src(st, sh, b.vx, b.vz, b2, m, 1.f);
-            launch_ref_v(st, sh, b2, m, 1.f, 0);
-            launch_ref_s(st, sh, b2, m, sg, 1.f, 0);
-            launch_record(st, sh, b.vz, b.vx, rs_z, rs_x, b2.vz, b2.vx, rs2_z, rs2_x, it);
-        } else {
-            launch_record(st, sh, b.vz, b.vx, rs_z, rs_x, (const float*)nullptr, nullptr, nullptr, nullptr, it);
-        }
-        if (edges) {
-            launch_edge_io(st, sh, bg.vx, bg.vz, e_bvx, e_bvz, it, 1);
-            launch_edge_io(st, sh, b.vx, b.vz, e_cvx, e_cvz, it, 1);
-        }
-    }
+    launch_grad_forward<TB>(st, sh, F, m, ga, second);
     // scatter_add (FD2DGPU.cu:3143-3149): s = 1*s + s2
     if (second) {
         launch_axpby(st, rs_z, rs2_z, B.total_rec, 1.f, 1.f);
@@ -624,24 +643,7 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
             }
         }
     }
-    for (int it = nt - 1; it >= 0; --it) {
-        if (B.any_pml) {
-            launch_edge_io(st, sh, bg.vx, bg.vz, e_bvx, e_bvz, it, 0);
-            launch_edge_io(st, sh, b.vx, b.vz, e_cvx, e_cvz, it, 0);
-        }
-        launch_ref_s(st, sh, bg, m, sg, -1.f, 1);
-        launch_ref_v(st, sh, bg, m, -1.f, 1);
-        launch_ref_s(st, sh, b, m, sb, -1.f, 1);
-        launch_born_src(st, sh, bg.vx, bg.vz, b, m, 1.f);
-        launch_ref_v(st, sh, b, m, -1.f, 1);
-        launch_inject_res(st, sh, bk.vz, bk.vx, rs_z, rs_x, it);
-        launch_adj_s(st, sh, bk, m, -1.f);
-        launch_adj_v(st, sh, bk, m, -1.f);
-        launch_adj_v(st, sh, bb, m, -1.f);
-        launch_born_adj(st, sh, bk, bb, m, -1.f);
-        launch_adj_s(st, sh, bb, m, -1.f);
-        launch_image(st, sh, sg, sb, bk, bb, bg, m, win, W);
-    }
+    launch_grad_backward<TB>(st, sh, F, m, ga);
     const long long A = (long long)h->g.allnx * h->g.allnz;
     launch_slot_nonfinite(st, sh, win, W, 7, 1, d_bad);
     launch_gather(st, sh, win, W, h->d_grad7, A, 7, h->g.allnx, h->g.allnz, d_bad);
@@ -817,17 +819,16 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
     StepSampler smp;
     if (!tile && (rc = smp.init(nt))) return rc;
     if (mode == 0) {
-        Strain none{nullptr, nullptr, nullptr, nullptr};
         stats_loop_begin(h);
         for (int it = 0; it < nt; ++it) {
             const bool tk = smp.take(it);
             launch_inject_src(st, sh, f.txx, f.tzz, h->d_wav, it);
             if (tk) smp.mark(st, 0);
-            launch_ref_v(st, sh, f, m, 1.f, 0);
+            launch_ref_v(st, sh, f, m);
             if (tk) smp.mark(st, 1);
-            launch_ref_s(st, sh, f, m, none, 1.f, 0);
+            launch_ref_s(st, sh, f, m);
             if (tk) smp.mark(st, 2);
-            launch_record(st, sh, f.vz, f.vx, rz, rx, nullptr, nullptr, nullptr, nullptr, it);
+            launch_record(st, sh, f.vz, f.vx, rz, rx, it);
         }
         stats_loop_end(h);
         launches = (long long)nt;
@@ -2632,7 +2633,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
         if (tk) smp.mark(st, 1);
         launch_rot_p(st, sh, f, m, 1.f);
         if (tk) smp.mark(st, 2);
-        launch_record(st, sh, f.vz, f.vx, rs, rs + R, nullptr, nullptr, nullptr, nullptr, it);
+        launch_record(st, sh, f.vz, f.vx, rs, rs + R, it);
     }
     stats_loop_end(h);
     if ((rc = stats_end(h, stats, padded_cells(B) * nt, nt, 0))) return rc;
@@ -2724,25 +2725,24 @@ int ds2d_decomp_rtm(ds2d_t* h, int nshots, const ds2d_shot* shots, int kind, con
     float *VP = vps, *VS = vps + n;
     HIP_TRY(hipMemsetAsync(vps, 0, (size_t)n * 2 * 4, st));
     HIP_TRY(hipMemsetAsync(win, 0, (size_t)W * 4, st));
-    const Strain none{nullptr, nullptr, nullptr, nullptr};
     stats_begin(h);
     stats_loop_begin(h);
     for (int it = 0; it < nt; ++it) {
         launch_inject_src(st, sh, f.txx, f.tzz, h->d_wav, it);
-        launch_ref_v(st, sh, f, m, 1.f, 0);
+        launch_ref_v(st, sh, f, m);
         launch_helmholtz(st, sh, f.vx, f.vz, VP, VS);
         launch_decomp(st, sh, kind, VP, VS, f, hist + (size_t)it * W * K, nullptr, 1);
-        launch_ref_s(st, sh, f, m, none, 1.f, 0);
+        launch_ref_s(st, sh, f, m);
     }
     // receiver side from rest; step nt-1 is not imaged (its backward slot is never written)
     HIP_TRY(hipMemsetAsync(f.vx, 0, (size_t)n * 15 * 4, st));
     HIP_TRY(hipMemsetAsync(vps, 0, (size_t)n * 2 * 4, st));
     for (int it = nt - 1; it >= 0; --it) {
         launch_assign_rec(st, sh, f.txx, f.tzz, dz, it);
-        launch_ref_v(st, sh, f, m, 1.f, 0);
+        launch_ref_v(st, sh, f, m);
         launch_helmholtz(st, sh, f.vx, f.vz, VP, VS);
         if (it < nt - 1) launch_decomp(st, sh, kind, VP, VS, f, hist + (size_t)it * W * K, win, 0);
-        launch_ref_s(st, sh, f, m, none, 1.f, 0);
+        launch_ref_s(st, sh, f, m);
     }
     stats_loop_end(h);
     if ((rc = stats_end(h, nullptr, padded_cells(B) * nt * 2, 0, 0))) return rc;

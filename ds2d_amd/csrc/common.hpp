@@ -46,11 +46,6 @@ struct EFieldT {
 using EField = EFieldT<float>;
 using EFieldD = EFieldT<double>;
 
-// Strain outputs of the reconstruction stress kernels (vx_gx, vz_gz, vx_gz, vz_gx).
-struct Strain {
-    float *gx_vx, *gz_vz, *gz_vx, *gx_vz;
-};
-
 // Per-cell medium of the padded window.
 struct Med {
     float *vp, *vs, *rho, *lam, *mu, *dampx, *dampz, *dmp, *dms;

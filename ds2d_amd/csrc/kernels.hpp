@@ -17,37 +17,37 @@ struct BatchShape {
 };
 
 // --- reference-compatible elastic kernels (kernels_ref.hip) ---------------
-// Overloads on EFieldD run the wavefield in FP64 (the source-side fields of
-// the reference-compat gradient); media, strains and records stay FP32.
-void launch_ref_v(hipStream_t st, const BatchShape& b, EField f, Med m, float dir, int recon);
-void launch_ref_v(hipStream_t st, const BatchShape& b, EFieldD f, Med m, float dir, int recon);
-void launch_ref_s(hipStream_t st, const BatchShape& b, EField f, Med m, Strain s, float dir, int recon);
-void launch_ref_s(hipStream_t st, const BatchShape& b, EFieldD f, Med m, Strain s, float dir, int recon);
-void launch_adj_v(hipStream_t st, const BatchShape& b, EField f, Med m, float dir);
-void launch_adj_s(hipStream_t st, const BatchShape& b, EField f, Med m, float dir);
-void launch_born_src(hipStream_t st, const BatchShape& b, const float* vx, const float* vz, EField tgt, Med m,
-                     float dir);
-void launch_born_src(hipStream_t st, const BatchShape& b, const double* vx, const double* vz, EFieldD tgt, Med m,
-                     float dir);
-void launch_born_src(hipStream_t st, const BatchShape& b, const double* vx, const double* vz, EField tgt, Med m,
-                     float dir);
-void launch_born_adj(hipStream_t st, const BatchShape& b, EField src, EField tgt, Med m, float dir);
+void launch_ref_v(hipStream_t st, const BatchShape& b, EField f, Med m);
+void launch_ref_s(hipStream_t st, const BatchShape& b, EField f, Med m);
 void launch_inject_src(hipStream_t st, const BatchShape& b, float* txx, float* tzz, const float* wav, int it);
-void launch_inject_src(hipStream_t st, const BatchShape& b, double* txx, double* tzz, const float* wav, int it);
 void launch_record(hipStream_t st, const BatchShape& b, const float* vz, const float* vx, float* rz, float* rx,
-                   const float* vz2, const float* vx2, float* rz2, float* rx2, int it);
-void launch_record(hipStream_t st, const BatchShape& b, const double* vz, const double* vx, float* rz, float* rx,
-                   const float* vz2, const float* vx2, float* rz2, float* rx2, int it);
-void launch_inject_res(hipStream_t st, const BatchShape& b, float* vz, float* vx, const float* rz, const float* rx,
-                       int it);
-void launch_edge_io(hipStream_t st, const BatchShape& b, float* fa, float* fb, float* ea, float* eb, int it,
-                    int save);
-void launch_edge_io(hipStream_t st, const BatchShape& b, double* fa, double* fb, double* ea, double* eb, int it,
-                    int save);
-void launch_image(hipStream_t st, const BatchShape& b, Strain sg, Strain sb, EField bk, EField bb, EField bg, Med m,
-                  float* w7, long long wstride);
-void launch_image(hipStream_t st, const BatchShape& b, Strain sg, Strain sb, EField bk, EField bb, EFieldD bg, Med m,
-                  float* w7, long long wstride);
+                   int it);
+
+// --- reference ELSRTM gradient (kernels_grad.hip) ---------------------------
+// TB is the precision of the two source-side wavefields.
+template <typename TB>
+struct GradFields {
+    EFieldT<TB> bg, b;
+    EField b2, bk, bb;
+    TB *lvx, *lvz;   // bg velocity with the edge bands of the coming step (bg.vx, bg.vz themselves without PML windows)
+    TB* edges;       // edge bands of bg vx, vz, b vx, vz (total_edge each), or null
+};
+struct GradArgs {
+    long long n, total_edge, wstride;
+    float dt, dx, dz;
+    int nt;
+    const float* wav;
+    const int *rmap, *rnext;          // column -> a trace, trace -> the next on its column (-1: none)
+    float *rs_z, *rs_x, *rs2_z, *rs2_x;
+    float *g, *wk, *pk, *wb, *cs;     // bg strains, products of bk (two sets) and bb, 3 arrays of n each; 2 mu (-dms)
+    float* w7;                        // window images pp, ps, illum, b_pp, b_ps, b2_pp, b2_ps
+};
+// Forward steps of bg, b and (second) b2 with records and edge bands.
+template <typename TB>
+void launch_grad_forward(hipStream_t st, const BatchShape& b, const GradFields<TB>& F, Med m, const GradArgs& a,
+                         bool second);
+template <typename TB>
+void launch_grad_backward(hipStream_t st, const BatchShape& b, const GradFields<TB>& F, Med m, const GradArgs& a);
 
 // --- setup and reductions (kernels_setup.hip) ------------------------------
 struct SetupArgs {
