@@ -14,13 +14,13 @@
 #include <cstring>
 #include <map>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "../../include/ds2d.h"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "chunk_plan.hpp"
+#include "wave.hpp"
 #include "unet.hpp"
 
 using namespace ds2d;
@@ -93,11 +93,9 @@ struct ds2d_ctx {
     int use_graph = 0;  // capture time loops into one hipGraph per loop
     int per_launch = 0; // plain Born/adjoint: shots per time loop (0: all)
     int fwd_two = 0;    // autotuned: mode 2 runs the two-kernel step (1) or the tiles of two steps (2) instead of the march
-    int acou_fused = -1;  // fused Born/adjoint steps: -1 auto, 0 never, 1 whenever eligible
+    int acou_fused = -1;  // fused acoustic steps in the resident-history passes (0: per-cell kernels)
     int src_fp64 = 1;     // reference-compat gradient: background and first-order Born field in FP64
     std::vector<int> shot_status;  // per shot of the last reference-compat gradient: 1 = left out (non-finite)
-    // (cells, slots, shots per launch) -> 0 per-cell kernels, else fused x width
-    std::map<std::tuple<long long, int, int>, int> acou_tuned;
 
     ~ds2d_ctx() {
         for (auto& kv : ws)
@@ -1281,6 +1279,7 @@ namespace {
 
 struct AcouWS {
     AcouFieldD bg;              // FP64 background
+    double* bg2 = nullptr;      // its second state in the fused background pass (3 n doubles)
     AcouField bn, lm;
     AcouField bn2, lm2;         // second state of the fused (ping-pong) Born / adjoint steps
     AcouMed m;
@@ -1292,34 +1291,31 @@ struct AcouWS {
     bool store = false;
     bool fused = false;         // store mode with the fused one-launch-per-step kernels
     int* rmap = nullptr;        // column -> trace of every slot (-1: none)
-    ChunkDesc* chunks = nullptr;
-    std::vector<std::pair<int, int>> gchunks;  // per launch group: first chunk, count
-    bool tune = false;          // choose per-cell vs fused (and the x width) at the first Born pass
+    AcouTile* tiles = nullptr;
+    std::vector<std::pair<int, int>> groups;   // per launch group: first tile, count
     long long n = 0, R = 0, W = 0;
 };
 
-constexpr int ACOU_CHUNK_W = 64, ACOU_THREADS = 256, ACOU_TUNE_STEPS = 48;
-
-// Chunk list of the fused acoustic steps for x width W (per launch group).
-int acou_build_chunks(ds2d_ctx* h, const Batch& B, AcouWS& w, int W) {
-    if (W < 1 || W > ACOU_FUSED_MAX_W) return fail(DS2D_EINVAL, "fused acoustic x width %d outside [1, %d]", W,
-                                                   ACOU_FUSED_MAX_W);
-    std::vector<ChunkDesc> ch;
+// Tiles of the fused acoustic steps, per launch group.
+int acou_build_tiles(ds2d_ctx* h, const Batch& B, AcouWS& w) {
+    std::vector<AcouTile> t;
     const int ns = (int)B.slots.size();
     const int gs = h->per_launch > 0 ? std::min(h->per_launch, ns) : ns;
-    const int rows = ACOU_THREADS - 16;
-    w.gchunks.clear();
+    w.groups.clear();
     for (int s0 = 0; s0 < ns; s0 += gs) {
-        const int first = (int)ch.size();
-        for (int s = s0; s < std::min(ns, s0 + gs); ++s)
-            for (int x0 = 0; x0 < B.slots[s].nxp; x0 += W)
-                for (int z0 = 0; z0 < B.slots[s].nzp; z0 += rows)
-                    ch.push_back(ChunkDesc{s, x0, std::min(x0 + W, B.slots[s].nxp), z0});
-        w.gchunks.push_back({first, (int)ch.size() - first});
+        const int first = (int)t.size();
+        for (int s = s0; s < std::min(ns, s0 + gs); ++s) {
+            const SlotDesc& q = B.slots[s];
+            for (int x0 = NOP; x0 < q.nxp - NOP; x0 += ACOU_TILE_COLS)
+                for (int z0 = NOP; z0 < q.nzp - NOP; z0 += WAVE_ROWS)
+                    t.push_back(AcouTile{q.off, q.rec_off, q.hist_off, x0, z0, q.nxp, q.nzp, q.nx, q.nz, q.pml, q.isx,
+                                         q.isz, q.igz, q.rmap_off, 0});
+        }
+        w.groups.push_back({first, (int)t.size() - first});
     }
     int rc;
-    if ((rc = h->fbuf("achunks", ch.size(), &w.chunks))) return rc;
-    HIP_TRY(hipMemcpyAsync(w.chunks, ch.data(), ch.size() * sizeof(ChunkDesc), hipMemcpyHostToDevice, h->st));
+    if ((rc = h->fbuf("atiles", t.size(), &w.tiles))) return rc;
+    HIP_TRY(hipMemcpyAsync(w.tiles, t.data(), t.size() * sizeof(AcouTile), hipMemcpyHostToDevice, h->st));
     return 0;
 }
 
@@ -1357,27 +1353,14 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
     if ((rc = h->fbuf("armap", std::max<long long>(B.total_rmap, 1), &w.rmap))) return rc;
     HIP_TRY(hipMemsetAsync(w.rmap, 0xff, B.total_rmap * 4, h->st));
     launch_fast_rmap(h->st, B.shape, w.rmap);
-    // fused Born / adjoint steps: store mode, 32-bit byte offsets within a field; the choice
-    // (per-cell kernels or fused at some x width) is timed once per batch geometry
-    w.fused = false;
-    w.tune = false;
-    if (w.store && n <= FUSED_MAX_CELLS && h->acou_fused != 0) {
-        int width = h->acou_fused > 1 ? h->acou_fused : ACOU_CHUNK_W;
-        if (h->acou_fused < 0) {
-            auto it = h->acou_tuned.find({n, (int)B.slots.size(), h->per_launch});
-            if (it == h->acou_tuned.end()) {
-                w.tune = true;
-                width = 0;
-            } else {
-                width = it->second;
-            }
-        }
-        if (width > 0) {
-            w.fused = true;
-            if ((rc = acou_build_chunks(h, B, w, width))) return rc;
-        }
+    // fused steps: store mode, 32-bit cell indices within a field (from one window to the largest batches
+    // faster than the per-cell kernels: 5.3 against 8 us a step on 331x181, 33 against 92 on 3.2 M cells)
+    w.fused = w.store && n <= FUSED_MAX_CELLS && h->acou_fused != 0;
+    if (w.fused && h->fbuf("acoubg2", (size_t)n * 3, &w.bg2)) {  // no room for the second background state
+        w.fused = false;
+        (void)hipGetLastError();
     }
-    return 0;
+    return w.fused ? acou_build_tiles(h, B, w) : 0;
 }
 AcouFusedArgs acou_fused_args(ds2d_ctx* h, AcouWS& w, const AcouField& A, const AcouField& Bf) {
     AcouFusedArgs q{};
@@ -1430,98 +1413,33 @@ std::vector<BatchShape> launch_groups(const ds2d_ctx* h, const Batch& B) {
 // Forward pass from rest.  do_bg: propagate the background (storing its
 // increment when w.store); otherwise the Born field reads the stored
 // increment.  Records: w.rec (bg), w.rec2 (born).
-void acou_fwd(ds2d_ctx* h, const Batch& B, AcouWS& w, bool do_bg, bool do_born, bool rec_bg);
-
-// Autotuner of the resident-history Born pass: time ACOU_TUNE_STEPS steps of
-// the per-cell kernels and of the fused step at several x widths, keep the
-// fastest for this batch geometry (cached in the handle).
-void acou_tune(ds2d_ctx* h, const Batch& B, AcouWS& w) {
-    hipStream_t st = h->st;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return;
-    const int steps = std::min(h->g.nt, ACOU_TUNE_STEPS);
-    auto time_pass = [&](int width) -> float {
-        (void)hipMemsetAsync(w.bn.vx, 0, (size_t)w.n * 3 * 4, st);
-        if (width > 0 && acou_build_chunks(h, B, w, width)) return 1e30f;
-        (void)hipEventRecord(e0, st);
-        if (width == 0) {
-            for (const BatchShape& sh : launch_groups(h, B))
-                for (int it = 0; it < steps; ++it) {
-                    launch_acou_v(st, sh, w.bg, w.bn, w.m, h->d_wav, it, 1.f, 0, 1);
-                    launch_acou_p(st, sh, w.bg, w.bn, w.m, w.hist, nullptr, w.rec2, it, 0, 1, 2, w.rmap);
-                }
-        } else {
-            AcouFusedArgs even = acou_fused_args(h, w, w.bn, w.bn2), odd = acou_fused_args(h, w, w.bn2, w.bn);
-            even.rec = odd.rec = w.rec2;
-            for (size_t gi = 0; gi < w.gchunks.size(); ++gi)
-                for (int it = 0; it < steps; ++it)
-                    launch_acou_born_fused(st, B.shape, (it & 1) ? odd : even, w.chunks + w.gchunks[gi].first,
-                                           w.gchunks[gi].second, w.rmap, it, ACOU_THREADS);
-        }
-        (void)hipEventRecord(e1, st);
-        float ms = 1e30f;
-        if (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return 1e30f;
-        return ms;
-    };
-    // widths 16, 32, 64 and those whose chunk count just fills 1, 2 or 3 rounds of one workgroup per CU
-    std::vector<int> widths = {16, 32, 64};
-    int ncu = 0;
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0) == hipSuccess && ncu > 0) {
-        const int rows = ACOU_THREADS - 16;
-        int max_nxp = 16;
-        for (const SlotDesc& S : B.slots) max_nxp = std::max(max_nxp, S.nxp);
-        auto nchunks = [&](int W) {
-            long long k = 0;
-            for (const SlotDesc& S : B.slots) k += (long long)((S.nxp + W - 1) / W) * ((S.nzp + rows - 1) / rows);
-            return k;
-        };
-        for (int R = 1; R <= 3; ++R) {
-            int lo = 8, hi = std::min(max_nxp, ACOU_FUSED_MAX_W);  // smallest W with nchunks(W) <= R * ncu
-            if (nchunks(hi) > (long long)R * ncu) continue;
-            while (lo < hi) {
-                const int mid = (lo + hi) / 2;
-                if (nchunks(mid) <= (long long)R * ncu)
-                    hi = mid;
-                else
-                    lo = mid + 1;
-            }
-            if (std::find(widths.begin(), widths.end(), lo) == widths.end()) widths.push_back(lo);
-        }
-    }
-    int best = 0;
-    float bt = time_pass(0);
-    for (int width : widths) {
-        const float t = time_pass(width);
-        if (t < bt) {
-            bt = t;
-            best = width;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    h->acou_tuned[{w.n, (int)B.slots.size(), h->per_launch}] = best;
-    w.fused = best > 0 && acou_build_chunks(h, B, w, best) == 0;
-}
-
 void acou_fwd(ds2d_ctx* h, const Batch& B, AcouWS& w, bool do_bg, bool do_born, bool rec_bg) {
     hipStream_t st = h->st;
-    if (w.tune && !do_bg && do_born && !rec_bg) {
-        w.tune = false;
-        acou_tune(h, B, w);
+    if (w.fused && w.store && !rec_bg) {
+        // the background pass fills the history, the Born pass reads it: one fused launch per step each;
+        // chunk lists hold absolute slot indices: launch with the whole slot table
+        if (do_bg) {
+            (void)hipMemsetAsync(w.bg.vx, 0, (size_t)w.n * 3 * 8, st);
+            (void)hipMemsetAsync(w.bg2, 0, (size_t)w.n * 3 * 8, st);
+            for (const std::pair<int, int>& gc : w.groups) {
+                double *a = w.bg.vx, *b = w.bg2;
+                for (int it = 0; it < h->g.nt; ++it, std::swap(a, b))
+                    launch_acou_bg_tile(st, B.shape, a, b, w.n, w.m, w.hist, h->d_wav, w.tiles + gc.first, gc.second, it);
+            }
+        }
+        if (do_born) {
+            (void)hipMemsetAsync(w.bn.vx, 0, (size_t)w.n * 3 * 4, st);
+            (void)hipMemsetAsync(w.bn2.vx, 0, (size_t)w.n * 3 * 4, st);
+            AcouFusedArgs even = acou_fused_args(h, w, w.bn, w.bn2), odd = acou_fused_args(h, w, w.bn2, w.bn);
+            even.rec = odd.rec = w.rec2;
+            for (const std::pair<int, int>& gc : w.groups)
+                for (int it = 0; it < h->g.nt; ++it)
+                    launch_acou_born_tile(st, B.shape, (it & 1) ? odd : even, w.tiles + gc.first, gc.second, w.rmap, it);
+        }
+        return;
     }
     (void)hipMemsetAsync(w.bg.vx, 0, (size_t)w.n * 3 * 8, st);
     (void)hipMemsetAsync(w.bn.vx, 0, (size_t)w.n * 3 * 4, st);
-    if (w.fused && !do_bg && do_born && !rec_bg) {
-        // Born field only, from the resident history: one fused launch per step
-        AcouFusedArgs even = acou_fused_args(h, w, w.bn, w.bn2), odd = acou_fused_args(h, w, w.bn2, w.bn);
-        even.rec = odd.rec = w.rec2;
-        // chunk lists hold absolute slot indices: launch with the whole slot table
-        for (size_t gi = 0; gi < w.gchunks.size(); ++gi)
-            for (int it = 0; it < h->g.nt; ++it)
-                launch_acou_born_fused(st, B.shape, (it & 1) ? odd : even, w.chunks + w.gchunks[gi].first,
-                                       w.gchunks[gi].second, w.rmap, it, ACOU_THREADS);
-        return;
-    }
     const int hmode = do_bg ? (w.store ? 1 : 0) : 2;
     for (const BatchShape& sh : launch_groups(h, B))
         for (int it = 0; it < h->g.nt; ++it) {
@@ -1539,13 +1457,14 @@ void acou_bwd(ds2d_ctx* h, const Batch& B, AcouWS& w) {
     (void)hipMemsetAsync(w.lm.vx, 0, (size_t)w.n * 3 * 4, st);
     (void)hipMemsetAsync(w.grad_pad, 0, (size_t)w.n * 4, st);
     if (w.fused) {
+        (void)hipMemsetAsync(w.lm2.vx, 0, (size_t)w.n * 3 * 4, st);
         AcouFusedArgs even = acou_fused_args(h, w, w.lm, w.lm2), odd = acou_fused_args(h, w, w.lm2, w.lm);
         even.grad = odd.grad = w.grad_pad;
         even.res = odd.res = w.rec2;
-        for (size_t gi = 0; gi < w.gchunks.size(); ++gi)
+        launch_acou_inj(st, B.shape, w.lm.p, w.rec2, h->g.nt - 1);
+        for (const std::pair<int, int>& gc : w.groups)
             for (int it = h->g.nt - 1, k = 0; it >= 0; --it, ++k)
-                launch_acou_adj_fused(st, B.shape, (k & 1) ? odd : even, w.chunks + w.gchunks[gi].first,
-                                      w.gchunks[gi].second, w.rmap, it, ACOU_THREADS);
+                launch_acou_adj_tile(st, B.shape, (k & 1) ? odd : even, w.tiles + gc.first, gc.second, w.rmap, it);
         return;
     }
     for (const BatchShape& sh : launch_groups(h, B)) {

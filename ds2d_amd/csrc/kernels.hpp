@@ -115,7 +115,7 @@ void launch_acou_adj_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouF
 void launch_acou_adj_v(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField lam, AcouMed m,
                        const float* wav, int it, int do_bg, const int* rmap, const float* res);
 struct ChunkDesc;
-// Fused plain acoustic steps (kernels_acoustic_fused.hip): state A -> B, each
+// Fused plain acoustic steps (kernels_acoustic_tile.hip): state A -> B, each
 // 3 fields (vx, vz, p) of n floats from the base pointer.
 struct AcouFusedArgs {
     const float* A;
@@ -128,11 +128,22 @@ struct AcouFusedArgs {
     const float* res;        // adjoint step: residual records
     float ax, az;            // dt/dx, dt/dz
 };
-bool acou_fused_threads_ok(int threads);
-void launch_acou_born_fused(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const ChunkDesc* chunks,
-                            int nchunks, const int* rmap, int it, int threads);
-void launch_acou_adj_fused(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const ChunkDesc* chunks,
-                           int nchunks, const int* rmap, int it, int threads);
+// One tile of the fused acoustic steps: all that a workgroup needs of its window.
+struct AcouTile {
+    long long off, rec_off, hist_off;
+    int x0, z0;  // first owned column and row
+    int nxp, nzp, nx, nz, pml;
+    int isx, isz, igz, rmap_off;
+    int pad;
+};
+constexpr int ACOU_TILE_COLS = 16;  // owned columns (of WAVE_ROWS rows)
+void launch_acou_born_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+                           int ntiles, const int* rmap, int it);
+void launch_acou_adj_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+                          int ntiles, const int* rmap, int it);
+// FP64 background step A -> B (3 fields of n doubles), increment into the history.
+void launch_acou_bg_tile(hipStream_t st, const BatchShape& b, const double* A, double* B, long long n, AcouMed m,
+                         float* hist, const float* wav, const AcouTile* tiles, int ntiles, int it);
 void launch_acou_ref_step(hipStream_t st, const BatchShape& b, float* px, float* pz, float* p, float* vx, float* vz,
                           const float* k, const float* rho, const float* damp, const float* wav, int sxnum,
                           float* rec, int it);
@@ -291,8 +302,7 @@ constexpr long long FUSED_MAX_CELLS = (1LL << 30) - (1LL << 20);
 // FUSED_HALO rows above and below its block are loaded to feed the z taps,
 // so it owns threads - 2*FUSED_HALO rows.
 constexpr int FUSED_HALO = 8;
-// Widest x chunk of the fused acoustic steps (the adjoint stages the
-// receiver residuals of its chunk's columns in LDS).
+// Largest x width that ds2d_set_fused accepts.
 constexpr int ACOU_FUSED_MAX_W = 1024;
 bool fused_threads_ok(int threads);
 // depth: columns of operands in flight per lane (2 or 4)

@@ -24,43 +24,12 @@
 // measured the same on one round and 10 % slower over several.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "wave.hpp"
 
 #include <algorithm>
 #include <type_traits>
 
 namespace ds2d {
-
-namespace {
-
-// The value of the next (previous) lane of the wave: the cell below (above).
-__device__ __forceinline__ float next_z(float f) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float prev_z(float f) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float taps(float a1, float b1, float a2, float b2, float a3, float b3, float a4, float b4) {
-    return DS2D_C1 * (a1 - b1) + DS2D_C2 * (a2 - b2) + DS2D_C3 * (a3 - b3) + DS2D_C4 * (a4 - b4);
-}
-// Forward and backward half-point differences along z.
-__device__ __forceinline__ float dplus_z(float f) {
-    const float p1 = next_z(f), p2 = next_z(p1), p3 = next_z(p2), p4 = next_z(p3);
-    const float m1 = prev_z(f), m2 = prev_z(m1), m3 = prev_z(m2);
-    return taps(p1, f, p2, m1, p3, m2, p4, m3);
-}
-__device__ __forceinline__ float dminus_z(float f) {
-    const float p1 = next_z(f), p2 = next_z(p1), p3 = next_z(p2);
-    const float m1 = prev_z(f), m2 = prev_z(m1), m3 = prev_z(m2), m4 = prev_z(m3);
-    return taps(f, m1, p1, m2, p2, m3, p3, m4);
-}
-
-// Weight of the cell at offset d in a forward half-point difference.
-__device__ __forceinline__ float src_tap(int d) {
-    return d == 1 ? DS2D_C1 : d == 2 ? DS2D_C2 : d == 3 ? DS2D_C3 : d == 4 ? DS2D_C4 :
-           d == 0 ? -DS2D_C1 : d == -1 ? -DS2D_C2 : d == -2 ? -DS2D_C3 : d == -3 ? -DS2D_C4 : 0.f;
-}
-
-}  // namespace
 
 template <int K, int NW, bool PML>
 __global__ __launch_bounds__(NW * 64) void k_tile_steps(FusedArgs a, const TileDesc* __restrict__ tiles, int ntiles,
@@ -136,7 +105,7 @@ __global__ __launch_bounds__(NW * 64) void k_tile_steps(FusedArgs a, const TileD
     }
     const float w0 = a.wav[it], w1 = ns > 1 ? a.wav[it + 1] : 0.f;
     // weight of the source in the z derivative of this lane's row
-    const float cz_src = src_tap(T.isz - z);
+    const float cz_src = src_tap<float>(T.isz - z);
     float d1[K], r2[K], d3[K], r4[K];
     if (PML && damped) {
 #pragma unroll
@@ -172,7 +141,7 @@ __global__ __launch_bounds__(NW * 64) void k_tile_steps(FusedArgs a, const TileD
             // the source sample, present in this step's velocity only
             const int dx = T.isx - ix0 - r;
             if ((unsigned)(dx + 3) < 8u) {
-                if (z == T.isz) ax += w * src_tap(dx);
+                if (z == T.isz) ax += w * src_tap<float>(dx);
                 if (dx == 0) cz += w * cz_src;
             }
             const bool u = zu && row_upd(k);

@@ -451,8 +451,8 @@ class Solver:
         return pp.reshape(self.allnx, self.allnz), ps.reshape(self.allnx, self.allnz), res, st.as_dict()
 
     def set_fused(self, mode):
-        """Fused Born/adjoint steps of the resident-history passes: -1 auto (timed), 0 never,
-        1 always (x width 64), k in [8, 1024] always with x width k."""
+        """Fused background/Born/adjoint steps of the resident-history passes: 0 never, else whenever they fit
+        (-1, 1 and x widths in [8, 1024] are the same: the tiles have a fixed width)."""
         _check(self.lib.ds2d_set_fused(self.h, int(mode)))
 
     def set_stop(self, target):

@@ -318,11 +318,10 @@ int ds2d_elsrtm_learned(ds2d_t* h, ds2d_unet_t* u, int nshots, const ds2d_shot* 
  * batched launch, the default; 1 = one shot after another as the reference's
  * per-rank shot loop does).  Applies to the plain Born/adjoint/CG entries. */
 int ds2d_set_batch(ds2d_t* h, int shots_per_launch);
-/* Resident-history Born and adjoint passes as one fused launch per step
- * (x-marching workgroups): -1 = auto (default: the per-cell kernels and the
- * fused step at several x widths are timed once per batch geometry), 0 =
- * never (per-cell kernels), 1 = always (x width 64), k in [8, 1024] = always,
- * with x width k. */
+/* Resident-history background, Born and adjoint passes as one fused launch
+ * per step: -1 = whenever they fit (default), 0 = never (per-cell kernels),
+ * 1 or an x width in [8, 1024] = as -1 (the steps run on tiles of a fixed
+ * width). */
 int ds2d_set_fused(ds2d_t* h, int mode);
 /* Stop rule of the CG solvers (ds2d_lsrtm_cg, ds2d_lsrtm_learned,
  * ds2d_elsrtm_cg, ds2d_elsrtm_learned): return after the first iteration
