@@ -81,8 +81,7 @@ struct ds2d_ctx {
     int chunk_d = 0;    // fused-kernel prefetch depth in columns (2 or 4; 0: default 2)
     int tblock = 1;     // fused elastic forward: time steps per launch (1 or 2)
     int chunk_plan = 1; // two steps per launch: balanced chunk plan when it simulates faster (0: fixed width)
-    int eb_fused = 1;   // elastic Born forward pass: one fused launch per step (0: k_eb_v + k_eb_s)
-    int eb_w = 0, eb_t = 0;  // its x-chunk width and workgroup lanes (0: defaults 64, 256)
+    int eb_fused = 1;   // elastic Born passes: one fused launch per step (0: the per-cell kernels)
     int rot_fused = 1;  // rotation forward: one fused launch per step (0: k_rot_v + k_rot_p)
     int last_plan = 0;  // the last two-step launch list: 1 balanced, 0 fixed width
     std::vector<int> plan_key;         // batch shape of the cached two-step chunk list
@@ -1072,10 +1071,8 @@ int ds2d_set_fused_born(ds2d_t* h, int on, int width, int threads) {
     int rc;
     if ((rc = check_h(h))) return rc;
     if (width < 0 || (width > 0 && width < 8)) return fail(DS2D_EINVAL, "chunk width must be 0 or >= 8");
-    if (threads != 0 && !eb_fused_threads_ok(threads)) return fail(DS2D_EINVAL, "threads must be 0, 256 or 512");
+    if (threads != 0 && threads != 256 && threads != 512) return fail(DS2D_EINVAL, "threads must be 0, 256 or 512");
     h->eb_fused = on ? 1 : 0;
-    h->eb_w = width;
-    h->eb_t = threads;
     return 0;
 }
 
@@ -1718,11 +1715,11 @@ struct EbWS {
     bool store = false;
     int* rmap = nullptr;
     long long n = 0, R = 0, W = 0, H = 0;
-    // fused forward step: second state (10 n) and chunk lists per launch group
+    // fused steps: second state (10 n; null: per-cell kernels) and tiles per launch group
     float* alt = nullptr;
-    ChunkDesc* chunks = nullptr;
-    std::vector<std::pair<int, int>> gchunks;
-    int threads = 256;
+    EbTile* tiles = nullptr;
+    bool wide = false;
+    std::vector<std::pair<int, int>> groups;  // first tile, count
     StepSampler* smp = nullptr;  // when set, the fused forward launches are timed (sampled steps)
 };
 
@@ -1784,33 +1781,65 @@ int eb_prepare(ds2d_ctx* h, const Batch& B, const float* pp_dev, const float* ps
     if ((rc = h->fbuf("ebrmap", std::max<long long>(B.total_rmap, 1), &w.rmap))) return rc;
     HIP_TRY(hipMemsetAsync(w.rmap, 0xff, B.total_rmap * 4, h->st));
     launch_fast_rmap(h->st, B.shape, w.rmap);
-    // fused forward step (32-bit byte offsets within a field: n < 2^30 cells)
+    // fused steps (32-bit cell indices within a field); when the second state does
+    // not fit, the per-cell kernels (one state) run instead
     w.alt = nullptr;
     if (h->eb_fused && n < (1LL << 30)) {
-        const int W = h->eb_w > 0 ? h->eb_w : 64;
-        w.threads = eb_fused_threads_ok(h->eb_t) ? h->eb_t : 256;
-        const int rows = w.threads - 2 * FUSED_HALO;
-        std::vector<ChunkDesc> ch;
-        w.gchunks.clear();
+        std::vector<int> nxp;
+        for (const SlotDesc& q : B.slots) nxp.push_back(q.nxp);
+        const EbTiles tp = plan_eb_tiles(nxp, B.shape.nzp);
+        w.wide = tp.wide;
+        std::vector<EbTile> t;
+        w.groups.clear();
         const int ns = (int)B.slots.size();
         const int gs = h->per_launch > 0 ? std::min(h->per_launch, ns) : ns;  // the groups of launch_groups
         for (int s0 = 0; s0 < ns; s0 += gs) {
-            const int first = (int)ch.size();
-            for (int s = s0; s < std::min(ns, s0 + gs); ++s)
-                for (int x0 = 0; x0 < B.slots[s].nxp; x0 += W)
-                    for (int z0 = 0; z0 < B.slots[s].nzp; z0 += rows)
-                        ch.push_back(ChunkDesc{s - s0, x0, std::min(x0 + W, B.slots[s].nxp), z0});
-            w.gchunks.push_back({first, (int)ch.size() - first});
+            const int first = (int)t.size();
+            for (int s = s0; s < std::min(ns, s0 + gs); ++s) {
+                const SlotDesc& q = B.slots[s];
+                for (int x0 = NOP; x0 < q.nxp - NOP; x0 += tp.cols)
+                    for (int z0 = NOP; z0 < q.nzp - NOP; z0 += WAVE_ROWS)
+                        t.push_back(EbTile{q.off, q.rec_off, q.hist_off, x0, z0, q.nxp, q.nzp, q.nx, q.nz, q.pml, q.isx,
+                                           q.isz, q.igz, q.rmap_off, 0});
+            }
+            w.groups.push_back({first, (int)t.size() - first});
         }
-        if ((rc = h->fbuf("ebchunks", ch.size(), &w.chunks))) return rc;
-        HIP_TRY(hipMemcpyAsync(w.chunks, ch.data(), ch.size() * sizeof(ChunkDesc), hipMemcpyHostToDevice, h->st));
-        // the second state; when it does not fit, the per-cell kernels (one state) run instead
+        if ((rc = h->fbuf("ebtiles", t.size(), &w.tiles))) return rc;
+        HIP_TRY(hipMemcpyAsync(w.tiles, t.data(), t.size() * sizeof(EbTile), hipMemcpyHostToDevice, h->st));
         if (h->fbuf("eborn2", (size_t)n * 10, &w.alt)) {
             w.alt = nullptr;
             (void)hipGetLastError();
         }
     }
     return 0;
+}
+
+// Steps 0 .. nt-1 of the background and / or the scattered field, one fused
+// launch each, state ping-ponged between the workspace (bg then bn, 10 n
+// floats) and w.alt; a background's final state ends in the workspace, where
+// the adjoint pass expects it.
+void eb_tile_steps(ds2d_ctx* h, const Batch& B, EbWS& w, bool do_bg, bool do_bn, int hmode) {
+    hipStream_t st = h->st;
+    const int nt = h->g.nt;
+    (void)hipMemsetAsync(w.alt, 0, (size_t)w.n * 10 * 4, st);
+    int g = 0;
+    for (const std::pair<int, int>& gc : w.groups) {
+        float *a = w.bg.vx, *b = w.alt;
+        for (int it = 0; it < nt; ++it, std::swap(a, b)) {
+            const EbFusedArgs q{a, b, w.n, w.m, w.hist, w.H, do_bn ? w.rec : nullptr, do_bn ? w.rec + w.R : nullptr};
+            const bool tk = w.smp && g == 0 && w.smp->take(it);
+            if (tk) w.smp->mark(st, 0);
+            launch_eb_tile(st, B.shape, q, w.tiles + gc.first, gc.second, w.wide, w.rmap, h->wav[it], it, do_bg, do_bn,
+                           hmode);
+            if (tk) {
+                w.smp->mark(st, 1);
+                w.smp->mark(st, 2);
+            }
+        }
+        ++g;
+    }
+    if (do_bg && (nt & 1))
+        (void)hipMemcpyAsync(w.bg.vx, w.alt, (size_t)w.n * (do_bn ? 10 : 5) * 4, hipMemcpyDeviceToDevice, st);
 }
 
 // Forward pass from rest into w.rec (z then x).  do_bg: propagate the
@@ -1820,29 +1849,8 @@ void eb_fwd(ds2d_ctx* h, const Batch& B, EbWS& w, bool do_bg) {
     hipStream_t st = h->st;
     (void)hipMemsetAsync(w.bg.vx, 0, (size_t)w.n * 10 * 4, st);  // bg + bn
     const int hmode = do_bg ? (w.store ? 1 : 0) : 2;
-    if (do_bg && w.alt) {
-        // one fused launch per step, state ping-ponged between the workspace
-        // (bg then bn, 10 n floats) and w.alt; the final state goes back to
-        // the workspace, where the adjoint pass expects it
-        const int nt = h->g.nt;
-        int g = 0;
-        for (const BatchShape& sh : launch_groups(h, B)) {
-            const std::pair<int, int> gc = w.gchunks[g++];
-            float *a = w.bg.vx, *b = w.alt;
-            for (int it = 0; it < nt; ++it) {
-                EbFusedArgs q{a, b, w.n, w.m, w.hist, w.H, w.rec, w.rec + w.R};
-                const bool tk = w.smp && g == 1 && w.smp->take(it);
-                if (tk) w.smp->mark(st, 0);
-                launch_eb_fused(st, sh, q, w.chunks + gc.first, gc.second, w.rmap, h->wav[it], 1.f, it, hmode,
-                                w.threads);
-                if (tk) {
-                    w.smp->mark(st, 1);
-                    w.smp->mark(st, 2);
-                }
-                std::swap(a, b);
-            }
-        }
-        if (nt & 1) (void)hipMemcpyAsync(w.bg.vx, w.alt, (size_t)w.n * 10 * 4, hipMemcpyDeviceToDevice, st);
+    if (w.alt) {
+        eb_tile_steps(h, B, w, do_bg, true, hmode);
         return;
     }
     for (const BatchShape& sh : launch_groups(h, B))
@@ -1856,6 +1864,10 @@ void eb_fwd(ds2d_ctx* h, const Batch& B, EbWS& w, bool do_bg) {
 void eb_bg(ds2d_ctx* h, const Batch& B, EbWS& w) {
     hipStream_t st = h->st;
     (void)hipMemsetAsync(w.bg.vx, 0, (size_t)w.n * 5 * 4, st);
+    if (w.alt) {
+        eb_tile_steps(h, B, w, true, false, w.store ? 1 : 0);
+        return;
+    }
     for (const BatchShape& sh : launch_groups(h, B))
         for (int it = 0; it < h->g.nt; ++it) {
             launch_eb_v(st, sh, w.bg, w.bn, w.m.rho, h->wav[it], 1.f, 1, 0);
@@ -1869,6 +1881,7 @@ void eb_bg(ds2d_ctx* h, const Batch& B, EbWS& w) {
 void eb_bwd(ds2d_ctx* h, const Batch& B, EbWS& w) {
     hipStream_t st = h->st;
     (void)hipMemsetAsync(w.lm.vx, 0, (size_t)w.n * 12 * 4, st);  // lm + gpp + gps + adjoint products
+    if (w.alt) (void)hipMemsetAsync(w.alt, 0, (size_t)w.n * 10 * 4, st);
     const int nt = h->g.nt, undo = w.store ? 0 : 1;
     int g = 0;
     for (const BatchShape& sh : launch_groups(h, B)) {
@@ -1880,13 +1893,13 @@ void eb_bwd(ds2d_ctx* h, const Batch& B, EbWS& w) {
         if (w.alt) {
             // one fused launch per step: adjoint state (and the background when
             // it is reversed) ping-ponged between the workspace and w.alt
-            const std::pair<int, int> gc = w.gchunks[g++];
+            const std::pair<int, int> gc = w.groups[g++];
             float *alm = w.lm.vx, *abg = w.bg.vx, *blm = w.alt, *bbg = w.alt + 5 * w.n;
             for (int it = nt - 2; it >= 0; --it) {
                 EbAdjArgs q{alm, abg, blm, bbg, w.n, w.m, w.store ? w.hist : nullptr, w.H, w.gpp, w.gps,
                             w.res, w.res + w.R};
-                launch_eb_adj_fused(st, sh, q, w.chunks + gc.first, gc.second, w.rmap, h->wav[it + 1], it, it + 1,
-                                    undo != 0, w.threads);
+                launch_eb_adj_tile(st, sh, q, w.tiles + gc.first, gc.second, w.wide, w.rmap, h->wav[it + 1], it, it + 1,
+                                   undo != 0);
                 std::swap(alm, blm);
                 if (undo) std::swap(abg, bbg);
             }

@@ -178,10 +178,9 @@ struct EbMed {
 struct EbAux {
     float *wa, *wb, *wc, *ux, *uz;
 };
-// One fused forward step of the pair (kernels_eborn_fused.hip): A and B hold
+// One fused forward step of the pair (kernels_eborn_tile.hip): A and B hold
 // 10 fields of n floats each (background vx vz txx tzz txz, then the
-// scattered five); A is read, B written.  hist_mode 1 stores the background
-// strains as k_eb_s does (0: none).
+// scattered five); A is read, B written.
 struct EbFusedArgs {
     const float* A;
     float* B;
@@ -200,10 +199,6 @@ void launch_eb_v(hipStream_t st, const BatchShape& b, EbField bg, EbField born, 
 void launch_eb_s(hipStream_t st, const BatchShape& b, EbField bg, EbField born, EbMed m, float* hist,
                  long long hstride, int it, float sign, int do_bg, int do_born, int hist_mode, const int* rmap,
                  float* rec_z, float* rec_x);
-// Chunks as the fused elastic step's (rows of a block: threads - 2*FUSED_HALO);
-// threads 256 or 512.  The result equals launch_eb_v + launch_eb_s with
-// do_bg = do_born = 1 up to FP32 rounding (FMA contraction).
-bool eb_fused_threads_ok(int threads);
 // One fused step of the rotation scheme (kernels_rot_fused.hip): A and B hold
 // 8 fields of n floats (theta omega vpx vpz vsx vsz, then theta_x omega_x of
 // the damping cells); records of vz, vx through the column -> trace map.
@@ -231,10 +226,18 @@ struct EbAdjArgs {
     float *gpp, *gps;
     const float *res_z, *res_x;
 };
-void launch_eb_adj_fused(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const struct ChunkDesc* chunks,
-                         int nchunks, const int* rmap, float w, int it, int it_inj, bool undo, int threads);
-void launch_eb_fused(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const struct ChunkDesc* chunks,
-                     int nchunks, const int* rmap, float w, float sign, int it, int hist_mode, int threads);
+using EbTile = AcouTile;
+struct EbTiles {
+    bool wide;
+    int cols;  // owned columns of a tile (of WAVE_ROWS rows)
+};
+EbTiles plan_eb_tiles(const std::vector<int>& nxp, int nzp);
+// Forward step of the background, the scattered field or both: equal to
+// launch_eb_v + launch_eb_s bit for bit, with the same hist_mode.
+void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const EbTile* tiles, int ntiles,
+                    bool wide, const int* rmap, float w, int it, bool do_bg, bool do_bn, int hist_mode);
+void launch_eb_adj_tile(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const EbTile* tiles, int ntiles,
+                        bool wide, const int* rmap, float w, int it, int it_inj, bool undo);
 // Adjoint step: k_eb_adj_v (receiver injection of step it_inj, -1 none, and the
 // transpose of the stress update), then k_eb_adj_s (transpose of the velocity
 // update and the gradient of step it; strains from hist, or from bg when

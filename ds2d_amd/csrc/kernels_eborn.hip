@@ -18,6 +18,7 @@
 // by reversing the background.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "eborn_math.hpp"
 
 namespace ds2d {
 
@@ -43,11 +44,11 @@ __device__ __forceinline__ bool cell_u(const SlotDesc& S, Cell& t) {
 // difference axis.  plus: sum c_i (f(i) - f(1-i)); minus: sum c_i (f(i-1) - f(-i)).
 template <typename F>
 __device__ __forceinline__ float dplus(F f) {
-    return DS2D_C1 * (f(1) - f(0)) + DS2D_C2 * (f(2) - f(-1)) + DS2D_C3 * (f(3) - f(-2)) + DS2D_C4 * (f(4) - f(-3));
+    return ebm::diff8(f(1), f(0), f(2), f(-1), f(3), f(-2), f(4), f(-3));
 }
 template <typename F>
 __device__ __forceinline__ float dminus(F f) {
-    return DS2D_C1 * (f(0) - f(-1)) + DS2D_C2 * (f(1) - f(-2)) + DS2D_C3 * (f(2) - f(-3)) + DS2D_C4 * (f(3) - f(-4));
+    return ebm::diff8(f(0), f(-1), f(1), f(-2), f(2), f(-3), f(3), f(-4));
 }
 // operand k cells away along x (stride s) or z (stride 1) of array a at cell c
 #define EB_X(a) [&](int k) { return (a)[c + (long long)k * s]; }
@@ -60,15 +61,6 @@ __device__ __forceinline__ bool hist_at(const SlotDesc& S, int ix, int iz, int i
     if (lx < 0 || lx >= S.nx || lz < 0 || lz >= S.nz) return false;
     h = (size_t)S.hist_off + ((size_t)it * S.nx + lx) * S.nz + lz;
     return true;
-}
-
-// Background strains of the Born source at cell c (add_born_source's
-// vxx/dx, vzz/dz and vzx/dx + vxz/dz).
-__device__ __forceinline__ void strains(const EbField& f, long long c, long long s, float idx, float idz, float& exx,
-                                        float& ezz, float& exz) {
-    exx = dminus(EB_X(f.vx)) * idx;
-    ezz = dminus(EB_Z(f.vz)) * idz;
-    exz = dplus(EB_X(f.vz)) * idx + dplus(EB_Z(f.vx)) * idz;
 }
 
 }  // namespace
@@ -93,12 +85,12 @@ __global__ __launch_bounds__(256) void k_eb_v(EbField bg, EbField b, const float
             const long long j = c + k;
             return j == src ? bg.tzz[j] + w : bg.tzz[j];
         };
-        bg.vx[c] += sign * (br * ax * dplus(txx) + br * az * dminus(EB_Z(bg.txz)));
-        bg.vz[c] += sign * (br * ax * dminus(EB_X(bg.txz)) + br * az * dplus(tzz));
+        bg.vx[c] += sign * ebm::two(br * ax, dplus(txx), br * az, dminus(EB_Z(bg.txz)));
+        bg.vz[c] += sign * ebm::two(br * ax, dminus(EB_X(bg.txz)), br * az, dplus(tzz));
     }
     if (do_b) {
-        b.vx[c] += br * ax * dplus(EB_X(b.txx)) + br * az * dminus(EB_Z(b.txz));
-        b.vz[c] += br * ax * dminus(EB_X(b.txz)) + br * az * dplus(EB_Z(b.tzz));
+        b.vx[c] += ebm::two(br * ax, dplus(EB_X(b.txx)), br * az, dminus(EB_Z(b.txz)));
+        b.vz[c] += ebm::two(br * ax, dminus(EB_X(b.txz)), br * az, dplus(EB_Z(b.tzz)));
     }
 }
 
@@ -114,19 +106,19 @@ __global__ __launch_bounds__(256) void k_eb_s(EbField bg, EbField b, EbMed m, fl
     Cell t;
     if (!cell_u(S, t)) return;
     const long long c = (long long)t.c, s = S.nzp;
-    const float l = m.lam[c], mu = m.mu[c], l2m = l + 2 * mu;
+    const ebm::Moduli q(m.lam[c], m.mu[c]);
     size_t h = 0;
     const bool inside = hist_at(S, t.ix, t.iz, it, h);
     float exx = 0.f, ezz = 0.f, exz = 0.f;
     if (do_bg) {
         const float dvx = dminus(EB_X(bg.vx)), dvz = dminus(EB_Z(bg.vz));
         const float dvxz = dplus(EB_Z(bg.vx)), dvzx = dplus(EB_X(bg.vz));
-        bg.txx[c] += sign * (ax * l2m * dvx + az * l * dvz);
-        bg.tzz[c] += sign * (ax * l * dvx + az * l2m * dvz);
-        bg.txz[c] += sign * (mu * (ax * dvzx + az * dvxz));
+        bg.txx[c] += sign * ebm::inc_xx(q, ax, az, dvx, dvz);
+        bg.tzz[c] += sign * ebm::inc_zz(q, ax, az, dvx, dvz);
+        bg.txz[c] += sign * ebm::inc_xz(q, ax, az, dvzx, dvxz);
         exx = dvx * idx;
         ezz = dvz * idz;
-        exz = dvzx * idx + dvxz * idz;
+        exz = ebm::two(dvzx, idx, dvxz, idz);
         if (hist_mode == 1 && inside) {
             hist[h] = exx;
             hist[h + hstride] = ezz;
@@ -140,15 +132,10 @@ __global__ __launch_bounds__(256) void k_eb_s(EbField bg, EbField b, EbMed m, fl
     if (do_b) {
         const float dvx = dminus(EB_X(b.vx)), dvz = dminus(EB_Z(b.vz));
         const float dvxz = dplus(EB_Z(b.vx)), dvzx = dplus(EB_X(b.vz));
-        float txx = b.txx[c] + ax * l2m * dvx + az * l * dvz;
-        float tzz = b.tzz[c] + ax * l * dvx + az * l2m * dvz;
-        float txz = b.txz[c] + mu * (ax * dvzx + az * dvxz);
-        if (inside) {
-            const float mp = -m.dmp[c], ms = -m.dms[c];
-            txx += 2 * l2m * mp * exx + 2 * (l2m * mp - 2 * mu * ms) * ezz;
-            tzz += 2 * (l2m * mp - 2 * mu * ms) * exx + 2 * l2m * mp * ezz;
-            txz += 2 * mu * ms * exz;
-        }
+        float txx = b.txx[c] + ebm::inc_xx(q, ax, az, dvx, dvz);
+        float tzz = b.tzz[c] + ebm::inc_zz(q, ax, az, dvx, dvz);
+        float txz = b.txz[c] + ebm::inc_xz(q, ax, az, dvzx, dvxz);
+        if (inside) ebm::born_source(q, m.dmp[c], m.dms[c], exx, ezz, exz, txx, tzz, txz);
         b.txx[c] = txx;
         b.tzz[c] = tzz;
         b.txz[c] = txz;
@@ -187,8 +174,8 @@ __global__ __launch_bounds__(256) void k_eb_adj_v(EbField lm, EbAux x, EbField b
             const long long j = c + k;
             return j == src ? bg.tzz[j] + w : bg.tzz[j];
         };
-        bg.vx[c] += -(br * ax * dplus(txx) + br * az * dminus(EB_Z(bg.txz)));
-        bg.vz[c] += -(br * ax * dminus(EB_X(bg.txz)) + br * az * dplus(tzz));
+        bg.vx[c] -= ebm::two(br * ax, dplus(txx), br * az, dminus(EB_Z(bg.txz)));
+        bg.vz[c] -= ebm::two(br * ax, dminus(EB_X(bg.txz)), br * az, dplus(tzz));
     }
     float ix_ = 0.f, iz_ = 0.f;
     if (it_inj >= 0 && t.iz == S.igz) {
@@ -199,8 +186,8 @@ __global__ __launch_bounds__(256) void k_eb_adj_v(EbField lm, EbAux x, EbField b
             iz_ = res_z[o];
         }
     }
-    const float vx = lm.vx[c] + ix_ - (ax * dplus(EB_X(x.wa)) + az * dminus(EB_Z(x.wc)));
-    const float vz = lm.vz[c] + iz_ - (az * dplus(EB_Z(x.wb)) + ax * dminus(EB_X(x.wc)));
+    const float vx = lm.vx[c] + ix_ - ebm::two(ax, dplus(EB_X(x.wa)), az, dminus(EB_Z(x.wc)));
+    const float vz = lm.vz[c] + iz_ - ebm::two(az, dplus(EB_Z(x.wb)), ax, dminus(EB_X(x.wc)));
     lm.vx[c] = vx;
     lm.vz[c] = vz;
     x.ux[c] = br * vx;
@@ -221,16 +208,16 @@ __global__ __launch_bounds__(256) void k_eb_adj_s(EbField lm, EbAux x, EbField b
     Cell t;
     if (!cell_u(S, t)) return;
     const long long c = (long long)t.c, s = S.nzp;
-    const float txx = lm.txx[c] - ax * dminus(EB_X(x.ux));
-    const float tzz = lm.tzz[c] - az * dminus(EB_Z(x.uz));
-    const float txz = lm.txz[c] - (az * dplus(EB_Z(x.ux)) + ax * dplus(EB_X(x.uz)));
+    const float txx = ebm::fma_(-ax, dminus(EB_X(x.ux)), lm.txx[c]);
+    const float tzz = ebm::fma_(-az, dminus(EB_Z(x.uz)), lm.tzz[c]);
+    const float txz = lm.txz[c] - ebm::two(az, dplus(EB_Z(x.ux)), ax, dplus(EB_X(x.uz)));
     lm.txx[c] = txx;
     lm.tzz[c] = tzz;
     lm.txz[c] = txz;
-    const float l = m.lam[c], mu = m.mu[c], l2m = l + 2 * mu;
-    x.wa[c] = l2m * txx + l * tzz;
-    x.wb[c] = l * txx + l2m * tzz;
-    x.wc[c] = mu * txz;
+    const ebm::Moduli q(m.lam[c], m.mu[c]);
+    x.wa[c] = ebm::two(q.l2m, txx, q.l, tzz);
+    x.wb[c] = ebm::two(q.l2m, tzz, q.l, txx);
+    x.wc[c] = q.mu * txz;
     size_t h;
     const bool inside = hist_at(S, t.ix, t.iz, it, h);
     float exx = 0.f, ezz = 0.f, exz = 0.f;
@@ -245,16 +232,18 @@ __global__ __launch_bounds__(256) void k_eb_adj_s(EbField lm, EbAux x, EbField b
         const float dvxz = dplus(EB_Z(bg.vx)), dvzx = dplus(EB_X(bg.vz));
         exx = dvx * idx;
         ezz = dvz * idz;
-        exz = dvzx * idx + dvxz * idz;
+        exz = ebm::two(dvzx, idx, dvxz, idz);
         if (undo) {
-            bg.txx[c] += -(ax * l2m * dvx + az * l * dvz);
-            bg.tzz[c] += -(ax * l * dvx + az * l2m * dvz);
-            bg.txz[c] += -(mu * (ax * dvzx + az * dvxz));
+            bg.txx[c] -= ebm::inc_xx(q, ax, az, dvx, dvz);
+            bg.tzz[c] -= ebm::inc_zz(q, ax, az, dvx, dvz);
+            bg.txz[c] -= ebm::inc_xz(q, ax, az, dvzx, dvxz);
         }
         if (!inside) return;
     }
-    gpp[c] += -2 * l2m * (exx + ezz) * (txx + tzz);
-    gps[c] += 4 * mu * (ezz * txx + exx * tzz) - 2 * mu * exz * txz;
+    float pp = gpp[c], ps = gps[c];
+    ebm::image(q, exx, ezz, exz, txx, tzz, txz, pp, ps);
+    gpp[c] = pp;
+    gps[c] = ps;
 }
 
 namespace {

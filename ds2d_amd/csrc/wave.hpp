@@ -39,7 +39,7 @@ __device__ __forceinline__ double prev_z(double f) {
 // c1 (a1 - b1) + c2 (a2 - b2) + c3 (a3 - b3) + c4 (a4 - b4)
 template <typename T>
 __device__ __forceinline__ T taps(T a1, T b1, T a2, T b2, T a3, T b3, T a4, T b4) {
-    return C8<T>::c1 * (a1 - b1) + C8<T>::c2 * (a2 - b2) + C8<T>::c3 * (a3 - b3) + C8<T>::c4 * (a4 - b4);
+    return fma(C8<T>::c4, a4 - b4, fma(C8<T>::c3, a3 - b3, fma(C8<T>::c2, a2 - b2, C8<T>::c1 * (a1 - b1))));
 }
 // Forward and backward half-point differences along z.
 template <typename T>
@@ -54,31 +54,11 @@ __device__ __forceinline__ T dminus_z(T f) {
     const T m1 = prev_z(f), m2 = prev_z(m1), m3 = prev_z(m2), m4 = prev_z(m3);
     return taps(f, m1, p1, m2, p2, m3, p3, m4);
 }
-// The same along x from a register queue q of columns j - 4 .. j + 4 (forward
-// differences read q[1..8] about q[4], backward ones q[0..7]).
-template <typename T>
-__device__ __forceinline__ T dplus_q(const T* q) {
-    return taps(q[5], q[4], q[6], q[3], q[7], q[2], q[8], q[1]);
-}
-template <typename T>
-__device__ __forceinline__ T dminus_q(const T* q) {
-    return taps(q[4], q[3], q[5], q[2], q[6], q[1], q[7], q[0]);
-}
 // Weight of the cell at offset d in a forward half-point difference.
 template <typename T>
 __device__ __forceinline__ T src_tap(int d) {
     return d == 1 ? C8<T>::c1 : d == 2 ? C8<T>::c2 : d == 3 ? C8<T>::c3 : d == 4 ? C8<T>::c4 :
            d == 0 ? -C8<T>::c1 : d == -1 ? -C8<T>::c2 : d == -2 ? -C8<T>::c3 : d == -3 ? -C8<T>::c4 : T(0);
-}
-
-// A copy in a register distinct from the source (early clobber).  A loaded
-// operand that enters an x queue stays live there for eight columns; copying
-// it lets the next prefetch reuse the load register, so the loop latch never
-// moves (and waits for) freshly loaded registers.
-__device__ __forceinline__ float fresh(float x) {
-    float r;
-    asm("v_mov_b32 %0, %1" : "=&v"(r) : "v"(x));
-    return r;
 }
 
 // Rows a wave owns: the velocity and the stress (or pressure) of a step each

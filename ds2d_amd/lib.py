@@ -264,7 +264,8 @@ class Solver:
         _check(self.lib.ds2d_set_chunk_plan(self.h, 1 if on else 0))
 
     def set_fused_born(self, on, width=0, threads=0):
-        """Elastic Born forward pass: one fused launch per step (True, default) or the two per-step kernels."""
+        """Elastic Born passes: one fused launch per step (True, default) or the two per-step kernels; the
+        width and the lanes are accepted without effect."""
         _check(self.lib.ds2d_set_fused_born(self.h, 1 if on else 0, int(width), int(threads)))
 
     def set_fused_rotation(self, on):
