@@ -258,8 +258,8 @@ def run_forward(a, cfg):
 
 def run_rot(a, cfg):
     """P/S-decoupled (theta/omega) forward modelling of the C3 windows: one
-    fused launch per step (velocity parts, then dilatation/rotation, in one
-    x-march), or with --no-fused-rot the two per-cell kernels per step."""
+    fused launch per step (velocity, then dilatation/rotation, on
+    tiles), or with --no-fused-rot the two per-cell kernels per step."""
     from ds2d_amd import Solver
     from ds2d_amd.lib import ricker
     wav = ricker(cfg["nt"], cfg["f0"], cfg["dt"])
@@ -286,7 +286,7 @@ def run_rot(a, cfg):
         "data": f"synthetic: seeded layered+faulted elastic model (seed {cfg['seed']}), vs = vp/1.73",
         "config": {"workload": cfg["desc"], "shots": len(cfg["shots"]), "nt": cfg["nt"], "cell_updates_per_step": cu,
                    "kernels": ("k_rot_v + k_rot_p per step (per-cell, reference layout of the rotation scheme)"
-                               if a.no_fused_rot else "k_rot_fused: one x-marching launch per step (unsplit "
+                               if a.no_fused_rot else "k_rot_tile: one launch per step on tiles (unsplit "
                                "theta/omega outside the damping strips)"),
                    "parallelism": "shots batched on one GPU"},
         "roofline": roofline(stats),
@@ -639,7 +639,7 @@ def run_c5(a):
                        "born_data_s": round(t_fwd, 2), "solvers": runs, "elastic_unet_training": train,
                        "note": "a step = one CG iteration over all shots; 1e-2 is not reached in this many "
                                "iterations (see resid)"},
-            # the fused forward step of the Born data pass (k_eb_fused, 100 B per padded cell and step)
+            # the fused forward step of the Born data pass (k_eb_tile, 100 B per padded cell and step)
             "roofline": roofline([stf]) if stf.get("kernel_avg_ms", 0) > 0 else None}
 
 
@@ -787,9 +787,9 @@ def main():
     out["device"] = {"arch": name, "cus": ncu, "hbm_gb": round(mem, 1)}
     traffic_json = a.traffic_json
     if a.workload == "rot" and traffic_json == TRAFFIC_JSON:  # the fused rotation step's own counters
-        traffic_json = None if a.no_fused_rot else os.path.join(ROOT, "profiles", "k_rot_fused_c3_traffic.json")
+        traffic_json = None if a.no_fused_rot else os.path.join(ROOT, "profiles", "k_rot_tile_c3_traffic.json")
     if a.workload == "c5" and traffic_json == TRAFFIC_JSON:  # the fused Born forward step's counters
-        traffic_json = None if a.no_fused_born else os.path.join(ROOT, "profiles", "k_eb_fused_c5_traffic.json")
+        traffic_json = None if a.no_fused_born else os.path.join(ROOT, "profiles", "k_eb_tile_c5_traffic.json")
     if traffic_json and os.path.exists(traffic_json) and out.get("roofline"):
         tr = json.load(open(traffic_json))
         cfgd = out.get("config", {})

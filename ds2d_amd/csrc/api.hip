@@ -1288,32 +1288,44 @@ struct AcouWS {
     bool store = false;
     bool fused = false;         // store mode with the fused one-launch-per-step kernels
     int* rmap = nullptr;        // column -> trace of every slot (-1: none)
-    AcouTile* tiles = nullptr;
+    StepTile* tiles = nullptr;
     std::vector<std::pair<int, int>> groups;   // per launch group: first tile, count
     long long n = 0, R = 0, W = 0;
 };
 
-// Tiles of the fused acoustic steps, per launch group.
-int acou_build_tiles(ds2d_ctx* h, const Batch& B, AcouWS& w) {
-    std::vector<AcouTile> t;
+// Tiles of cols owned columns, and the first and count of each group of per_group windows.
+int step_tiles(ds2d_ctx* h, const Batch& B, const char* name, int cols, int per_group, StepTile** tiles,
+               std::vector<std::pair<int, int>>& groups) {
+    std::vector<StepTile> t;
     const int ns = (int)B.slots.size();
-    const int gs = h->per_launch > 0 ? std::min(h->per_launch, ns) : ns;
-    w.groups.clear();
-    for (int s0 = 0; s0 < ns; s0 += gs) {
+    groups.clear();
+    for (int s0 = 0; s0 < ns; s0 += per_group) {
         const int first = (int)t.size();
-        for (int s = s0; s < std::min(ns, s0 + gs); ++s) {
+        for (int s = s0; s < std::min(ns, s0 + per_group); ++s) {
             const SlotDesc& q = B.slots[s];
-            for (int x0 = NOP; x0 < q.nxp - NOP; x0 += ACOU_TILE_COLS)
+            for (int x0 = NOP; x0 < q.nxp - NOP; x0 += cols)
                 for (int z0 = NOP; z0 < q.nzp - NOP; z0 += WAVE_ROWS)
-                    t.push_back(AcouTile{q.off, q.rec_off, q.hist_off, x0, z0, q.nxp, q.nzp, q.nx, q.nz, q.pml, q.isx,
-                                         q.isz, q.igz, q.rmap_off, 0});
+                    t.push_back(StepTile{q.off, q.rec_off, q.hist_off, x0, z0, q.nxp, q.nzp, q.nx, q.nz, q.pml, q.isx,
+                                         q.isz, q.igz, q.rmap_off, q.boundary == 0 ? q.pml : 0});
         }
-        w.groups.push_back({first, (int)t.size() - first});
+        groups.push_back({first, (int)t.size() - first});
     }
     int rc;
-    if ((rc = h->fbuf("atiles", t.size(), &w.tiles))) return rc;
-    HIP_TRY(hipMemcpyAsync(w.tiles, t.data(), t.size() * sizeof(AcouTile), hipMemcpyHostToDevice, h->st));
+    if ((rc = h->fbuf(name, t.size(), tiles))) return rc;
+    HIP_TRY(hipMemcpyAsync(*tiles, t.data(), t.size() * sizeof(StepTile), hipMemcpyHostToDevice, h->st));
     return 0;
+}
+
+// Windows of a launch group (launch_groups).
+int group_size(const ds2d_ctx* h, const Batch& B) {
+    const int ns = (int)B.slots.size();
+    return h->per_launch > 0 ? std::min(h->per_launch, ns) : ns;
+}
+
+std::vector<int> widths(const Batch& B) {
+    std::vector<int> w;
+    for (const SlotDesc& q : B.slots) w.push_back(q.nxp);
+    return w;
 }
 
 int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS& w) {
@@ -1357,7 +1369,7 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
         w.fused = false;
         (void)hipGetLastError();
     }
-    return w.fused ? acou_build_tiles(h, B, w) : 0;
+    return w.fused ? step_tiles(h, B, "atiles", ACOU_TILE_COLS, group_size(h, B), &w.tiles, w.groups) : 0;
 }
 AcouFusedArgs acou_fused_args(ds2d_ctx* h, AcouWS& w, const AcouField& A, const AcouField& Bf) {
     AcouFusedArgs q{};
@@ -1717,7 +1729,7 @@ struct EbWS {
     long long n = 0, R = 0, W = 0, H = 0;
     // fused steps: second state (10 n; null: per-cell kernels) and tiles per launch group
     float* alt = nullptr;
-    EbTile* tiles = nullptr;
+    StepTile* tiles = nullptr;
     bool wide = false;
     std::vector<std::pair<int, int>> groups;  // first tile, count
     StepSampler* smp = nullptr;  // when set, the fused forward launches are timed (sampled steps)
@@ -1785,27 +1797,9 @@ int eb_prepare(ds2d_ctx* h, const Batch& B, const float* pp_dev, const float* ps
     // not fit, the per-cell kernels (one state) run instead
     w.alt = nullptr;
     if (h->eb_fused && n < (1LL << 30)) {
-        std::vector<int> nxp;
-        for (const SlotDesc& q : B.slots) nxp.push_back(q.nxp);
-        const EbTiles tp = plan_eb_tiles(nxp, B.shape.nzp);
+        const StepTiles tp = plan_eb_tiles(widths(B), B.shape.nzp);
         w.wide = tp.wide;
-        std::vector<EbTile> t;
-        w.groups.clear();
-        const int ns = (int)B.slots.size();
-        const int gs = h->per_launch > 0 ? std::min(h->per_launch, ns) : ns;  // the groups of launch_groups
-        for (int s0 = 0; s0 < ns; s0 += gs) {
-            const int first = (int)t.size();
-            for (int s = s0; s < std::min(ns, s0 + gs); ++s) {
-                const SlotDesc& q = B.slots[s];
-                for (int x0 = NOP; x0 < q.nxp - NOP; x0 += tp.cols)
-                    for (int z0 = NOP; z0 < q.nzp - NOP; z0 += WAVE_ROWS)
-                        t.push_back(EbTile{q.off, q.rec_off, q.hist_off, x0, z0, q.nxp, q.nzp, q.nx, q.nz, q.pml, q.isx,
-                                           q.isz, q.igz, q.rmap_off, 0});
-            }
-            w.groups.push_back({first, (int)t.size() - first});
-        }
-        if ((rc = h->fbuf("ebtiles", t.size(), &w.tiles))) return rc;
-        HIP_TRY(hipMemcpyAsync(w.tiles, t.data(), t.size() * sizeof(EbTile), hipMemcpyHostToDevice, h->st));
+        if ((rc = step_tiles(h, B, "ebtiles", tp.cols, group_size(h, B), &w.tiles, w.groups))) return rc;
         if (h->fbuf("eborn2", (size_t)n * 10, &w.alt)) {
             w.alt = nullptr;
             (void)hipGetLastError();
@@ -2492,38 +2486,32 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
     if ((rc = smp.init(nt))) return rc;
     const long long n = B.total_cells;
     float* fa = nullptr;
-    // one fused launch per step needs two sets of 8 fields; when they do not
+    // one fused launch per step needs two sets of 6 fields; when they do not
     // fit, the per-cell kernels (12 fields) run instead
-    if (h->rot_fused && n < (1LL << 30) && h->fbuf("rotf", (size_t)n * 16, &fa)) {
+    if (h->rot_fused && n < (1LL << 30) && h->fbuf("rotf", (size_t)n * 12, &fa)) {
         fa = nullptr;
         (void)hipGetLastError();
     }
     if (fa) {
-        // one fused launch per step (64-column chunks, 256 lanes), state
-        // ping-ponged between two sets of 8 fields
+        // one fused launch per step on tiles, state ping-ponged between two sets of 6 fields
         int* rmap;
         if ((rc = h->fbuf("rmap", B.total_rmap, &rmap))) return rc;
-        HIP_TRY(hipMemsetAsync(fa, 0, (size_t)n * 16 * 4, st));
+        HIP_TRY(hipMemsetAsync(fa, 0, (size_t)n * 12 * 4, st));
         HIP_TRY(hipMemsetAsync(rmap, 0xff, B.total_rmap * 4, st));
         HIP_TRY(hipMemsetAsync(rs, 0, R * 2 * 4, st));
         launch_fast_rmap(st, sh, rmap);
-        const int W = 64, T = 256, rows = T - 2 * FUSED_HALO;
-        std::vector<ChunkDesc> ch;
-        for (int s = 0; s < nshots; ++s)
-            for (int x0 = 0; x0 < B.slots[s].nxp; x0 += W)
-                for (int z0 = 0; z0 < B.slots[s].nzp; z0 += rows)
-                    ch.push_back(ChunkDesc{s, x0, std::min(x0 + W, B.slots[s].nxp), z0});
-        ChunkDesc* d_ch;
-        if ((rc = h->fbuf("rotchunks", ch.size(), &d_ch))) return rc;
-        HIP_TRY(hipMemcpyAsync(d_ch, ch.data(), ch.size() * sizeof(ChunkDesc), hipMemcpyHostToDevice, st));
+        const StepTiles tp = plan_rot_tiles(widths(B), sh.nzp);
+        StepTile* tiles;
+        std::vector<std::pair<int, int>> gr;
+        if ((rc = step_tiles(h, B, "rottiles", tp.cols, nshots, &tiles, gr))) return rc;
         stats_begin(h);
         stats_loop_begin(h);
-        float *a = fa, *b = fa + 8 * n;
+        float *a = fa, *b = fa + 6 * n;
         for (int it = 0; it < nt; ++it) {
             const bool tk = smp.take(it);
             if (tk) smp.mark(st, 0);
             RotFusedArgs q{a, b, n, m.vp, m.vs, m.dampx, m.dampz, h->d_wav, rs, rs + R};
-            launch_rot_fused(st, sh, q, d_ch, (int)ch.size(), rmap, it, T, B.any_pml);
+            launch_rot_tile(st, sh, q, tiles, gr[0].second, tp.wide, rmap, it, B.any_pml);
             if (tk) {
                 smp.mark(st, 1);
                 smp.mark(st, 2);
@@ -2534,7 +2522,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
         if ((rc = stats_end(h, stats, padded_cells(B) * nt, nt, 0))) return rc;
         double kf, unused;
         smp.averages(&kf, &unused);
-        // per padded cell: theta, omega, 4 velocity parts, vp, vs in, 6 fields out (56 B); the damping cells
+        // per padded cell: theta, omega, vx, vz, vp, vs in, 4 fields out (40 B); the damping cells
         // add dampx, dampz and theta_x, omega_x read and written (24 B)
         h->last.kernel_avg_ms = kf;
         double pml_cells = 0;  // update-region cells of the damping strips (PML windows)
@@ -2542,7 +2530,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
             if (S.boundary == 0 && S.pml >= NOP)
                 pml_cells += (double)(S.nxp - 2 * NOP) * (S.nzp - 2 * NOP) -
                              (double)(S.nxp - 2 * S.pml + 1) * (S.nzp - 2 * S.pml + 1);
-        h->last.alg_bytes = (double)n * 14 * 4 + pml_cells * 6 * 4;
+        h->last.alg_bytes = (double)n * 10 * 4 + pml_cells * 6 * 4;
         h->last.aux_kernel_avg_ms = 0;
         h->last.aux_alg_bytes = 0;
         h->last.kernel_samples = smp.n;

@@ -128,22 +128,30 @@ struct AcouFusedArgs {
     const float* res;        // adjoint step: residual records
     float ax, az;            // dt/dx, dt/dz
 };
-// One tile of the fused acoustic steps: all that a workgroup needs of its window.
-struct AcouTile {
+// One tile of the kernels that take a step per launch (tile_lanes.hpp,
+// kernels_acoustic_tile.hip): all that a workgroup needs of its window.
+struct StepTile {
     long long off, rec_off, hist_off;
     int x0, z0;  // first owned column and row
     int nxp, nzp, nx, nz, pml;
     int isx, isz, igz, rmap_off;
-    int pad;
+    int damp;  // width of the damping strips (0: none)
 };
+// Width of the tiles by the size of the batch: narrow ones until wide ones
+// alone give eight to a CU.
+struct StepTiles {
+    bool wide;
+    int cols;  // owned columns of a tile (of WAVE_ROWS rows)
+};
+StepTiles plan_step_tiles(const std::vector<int>& nxp, int nzp, int narrow, int wide);
 constexpr int ACOU_TILE_COLS = 16;  // owned columns (of WAVE_ROWS rows)
-void launch_acou_born_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+void launch_acou_born_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const StepTile* tiles,
                            int ntiles, const int* rmap, int it);
-void launch_acou_adj_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+void launch_acou_adj_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const StepTile* tiles,
                           int ntiles, const int* rmap, int it);
 // FP64 background step A -> B (3 fields of n doubles), increment into the history.
 void launch_acou_bg_tile(hipStream_t st, const BatchShape& b, const double* A, double* B, long long n, AcouMed m,
-                         float* hist, const float* wav, const AcouTile* tiles, int ntiles, int it);
+                         float* hist, const float* wav, const StepTile* tiles, int ntiles, int it);
 void launch_acou_ref_step(hipStream_t st, const BatchShape& b, float* px, float* pz, float* p, float* vx, float* vz,
                           const float* k, const float* rho, const float* damp, const float* wav, int sxnum,
                           float* rec, int it);
@@ -199,9 +207,9 @@ void launch_eb_v(hipStream_t st, const BatchShape& b, EbField bg, EbField born, 
 void launch_eb_s(hipStream_t st, const BatchShape& b, EbField bg, EbField born, EbMed m, float* hist,
                  long long hstride, int it, float sign, int do_bg, int do_born, int hist_mode, const int* rmap,
                  float* rec_z, float* rec_x);
-// One fused step of the rotation scheme (kernels_rot_fused.hip): A and B hold
-// 8 fields of n floats (theta omega vpx vpz vsx vsz, then theta_x omega_x of
-// the damping cells); records of vz, vx through the column -> trace map.
+// One fused step of the rotation scheme (kernels_rot_tile.hip): A and B hold
+// 6 fields of n floats (theta omega vx vz, then theta_x omega_x of the damping
+// cells); records of vz, vx through the column -> trace map.
 struct RotFusedArgs {
     const float* A;
     float* B;
@@ -209,8 +217,9 @@ struct RotFusedArgs {
     const float *vp, *vs, *dampx, *dampz, *wav;
     float *rec_z, *rec_x;
 };
-void launch_rot_fused(hipStream_t st, const BatchShape& b, const RotFusedArgs& a, const struct ChunkDesc* chunks,
-                      int nchunks, const int* rmap, int it, int threads, bool pml);
+StepTiles plan_rot_tiles(const std::vector<int>& nxp, int nzp);
+void launch_rot_tile(hipStream_t st, const BatchShape& b, const RotFusedArgs& a, const StepTile* tiles, int ntiles,
+                     bool wide, const int* rmap, int it, bool pml);
 // One fused adjoint step (k_eb_adj_v with the residual of step it_inj, then
 // k_eb_adj_s of step it): adjoint state and background read from A, written
 // to B (5 fields each: vx vz txx tzz txz); gradients accumulated in place.
@@ -226,17 +235,12 @@ struct EbAdjArgs {
     float *gpp, *gps;
     const float *res_z, *res_x;
 };
-using EbTile = AcouTile;
-struct EbTiles {
-    bool wide;
-    int cols;  // owned columns of a tile (of WAVE_ROWS rows)
-};
-EbTiles plan_eb_tiles(const std::vector<int>& nxp, int nzp);
+StepTiles plan_eb_tiles(const std::vector<int>& nxp, int nzp);
 // Forward step of the background, the scattered field or both: equal to
 // launch_eb_v + launch_eb_s bit for bit, with the same hist_mode.
-void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const EbTile* tiles, int ntiles,
+void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const StepTile* tiles, int ntiles,
                     bool wide, const int* rmap, float w, int it, bool do_bg, bool do_bn, int hist_mode);
-void launch_eb_adj_tile(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const EbTile* tiles, int ntiles,
+void launch_eb_adj_tile(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const StepTile* tiles, int ntiles,
                         bool wide, const int* rmap, float w, int it, int it_inj, bool undo);
 // Adjoint step: k_eb_adj_v (receiver injection of step it_inj, -1 none, and the
 // transpose of the stress update), then k_eb_adj_s (transpose of the velocity

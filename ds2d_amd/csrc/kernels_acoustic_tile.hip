@@ -33,10 +33,10 @@ namespace {
 constexpr int NW = 8, K = ACOU_TILE_COLS / NW + 2 * WAVE_HALO / NW;
 struct Tile {
     static constexpr int RX = K * NW;
-    AcouTile T;
+    StepTile T;
     int lane, wv, z, ix0;
     bool zu, zown;
-    __device__ __forceinline__ bool init(const AcouTile* tiles, int ntiles, int per_xcd) {
+    __device__ __forceinline__ bool init(const StepTile* tiles, int ntiles, int per_xcd) {
         const int ch = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
         if (ch >= ntiles) return false;
         T = tiles[ch];
@@ -91,7 +91,7 @@ __device__ __forceinline__ void publish(R* f, int wv, int lane, const R (&v)[K])
 }  // namespace
 
 // Born step: v += (dt/d) b D+ p;  p += k (dt/dx D- vx + dt/dz D- vz) + 2 m dp_bg
-__global__ __launch_bounds__(NW * 64) void k_acou_born_tile(AcouFusedArgs a, const AcouTile* __restrict__ tiles,
+__global__ __launch_bounds__(NW * 64) void k_acou_born_tile(AcouFusedArgs a, const StepTile* __restrict__ tiles,
                                                             int ntiles, int per_xcd, const int* __restrict__ rmap,
                                                             int nt, int it) {
     __shared__ float lp[(K * NW + 8) * 64], lv[(K * NW + 8) * 64];
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(NW * 64) void k_acou_born_tile(AcouFusedArgs a, con
 //   lv += -(dt/d) D+ (k lp);  lp += -(dt/d) D- (b lv)   (k lp, b lv masked to the update region)
 // The residual of the next (earlier) step is added by the wave that stores a
 // receiver's lp, as k_acou_adj_v does; the first one's by launch_acou_inj.
-__global__ __launch_bounds__(NW * 64) void k_acou_adj_tile(AcouFusedArgs a, const AcouTile* __restrict__ tiles,
+__global__ __launch_bounds__(NW * 64) void k_acou_adj_tile(AcouFusedArgs a, const StepTile* __restrict__ tiles,
                                                            int ntiles, int per_xcd, const int* __restrict__ rmap,
                                                            int nt, int it) {
     __shared__ float lw[(K * NW + 8) * 64], lu[(K * NW + 8) * 64];
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(NW * 64) void k_acou_bg_tile(const double* __restri
                                                           long long n, const float* __restrict__ bu,
                                                           const float* __restrict__ kk, float* hist,
                                                           const float* __restrict__ wav,
-                                                          const AcouTile* __restrict__ tiles, int ntiles, int per_xcd,
+                                                          const StepTile* __restrict__ tiles, int ntiles, int per_xcd,
                                                           double ax, double az, int it) {
     __shared__ double lp[(K * NW + 8) * 64];
     Tile g;
@@ -268,20 +268,20 @@ __global__ __launch_bounds__(NW * 64) void k_acou_bg_tile(const double* __restri
     }
 }
 
-void launch_acou_born_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+void launch_acou_born_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const StepTile* tiles,
                            int ntiles, const int* rmap, int it) {
     const int per_xcd = (ntiles + 7) / 8;
     hipLaunchKernelGGL(k_acou_born_tile, dim3(per_xcd * 8), dim3(NW * 64), 0, st, a, tiles, ntiles, per_xcd, rmap,
                        b.nt, it);
 }
-void launch_acou_adj_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const AcouTile* tiles,
+void launch_acou_adj_tile(hipStream_t st, const BatchShape& b, const AcouFusedArgs& a, const StepTile* tiles,
                           int ntiles, const int* rmap, int it) {
     const int per_xcd = (ntiles + 7) / 8;
     hipLaunchKernelGGL(k_acou_adj_tile, dim3(per_xcd * 8), dim3(NW * 64), 0, st, a, tiles, ntiles, per_xcd, rmap,
                        b.nt, it);
 }
 void launch_acou_bg_tile(hipStream_t st, const BatchShape& b, const double* A, double* B, long long n, AcouMed m,
-                         float* hist, const float* wav, const AcouTile* tiles, int ntiles, int it) {
+                         float* hist, const float* wav, const StepTile* tiles, int ntiles, int it) {
     const int per_xcd = (ntiles + 7) / 8;
     hipLaunchKernelGGL(k_acou_bg_tile, dim3(per_xcd * 8), dim3(NW * 64), 0, st, A, B, n, m.b, m.k, hist, wav, tiles,
                        ntiles, per_xcd, (double)b.dt / (double)b.dx, (double)b.dt / (double)b.dz, it);

@@ -27,80 +27,21 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
-#include "wave.hpp"
+#include "tile_lanes.hpp"
 #include "eborn_math.hpp"
 
 namespace ds2d {
 
-namespace {
-
-template <int K, int NW>
-struct EbTileLanes {
-    static constexpr int RX = K * NW;
-    EbTile T;
-    int lane, wv, z, ix0;
-    bool zu, zown, zphys;
-    __device__ __forceinline__ bool init(const EbTile* tiles, int ntiles, int per_xcd) {
-        const int ch = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if (ch >= ntiles) return false;
-        T = tiles[ch];
-        lane = threadIdx.x & 63;
-        wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        z = T.z0 - WAVE_HALO + lane;
-        ix0 = T.x0 - WAVE_HALO;
-        zu = z >= NOP && z < T.nzp - NOP;
-        zown = zu && lane >= WAVE_HALO && lane < 64 - WAVE_HALO;
-        zphys = z >= T.pml && z < T.pml + T.nz;
-        return true;
-    }
-    __device__ __forceinline__ int row(int k) const { return k * NW + wv; }
-    __device__ __forceinline__ int col(int k) const { return ix0 + k * NW + wv; }
-    __device__ __forceinline__ bool row_upd(int k) const { return col(k) >= NOP && col(k) < T.nxp - NOP; }
-    __device__ __forceinline__ bool upd(int k) const { return zu && row_upd(k); }
-    __device__ __forceinline__ bool inside(int k, int m) const {
-        return (k * NW >= m || row(k) >= m) && (k * NW + NW <= RX - m || row(k) < RX - m);
-    }
-    __device__ __forceinline__ uint32_t cell(int k) const {
-        return (uint32_t)(T.off + (long long)col(k) * T.nzp + z);
-    }
-    __device__ __forceinline__ bool phys(int k) const { return zphys && col(k) >= T.pml && col(k) < T.pml + T.nx; }
-    __device__ __forceinline__ size_t hist(int k, int it) const {
-        return (size_t)T.hist_off + ((size_t)it * T.nx + (col(k) - T.pml)) * T.nz + (size_t)(z - T.pml);
-    }
-    __device__ __forceinline__ float dplus_x(const float* f, int k, float own) const {
-        const float* X = f + (row(k) + 4) * 64 + lane;
-        return ebm::diff8(X[64], own, X[128], X[-64], X[192], X[-128], X[256], X[-192]);
-    }
-    __device__ __forceinline__ float dminus_x(const float* f, int k, float own) const {
-        const float* X = f + (row(k) + 4) * 64 + lane;
-        return ebm::diff8(own, X[-64], X[64], X[-128], X[128], X[-192], X[192], X[-256]);
-    }
-    // v with the source sample on top in the source cell
-    __device__ __forceinline__ float with_source(int k, float v, float w) const {
-        return col(k) == T.isx && z == T.isz ? v + w : v;
-    }
-    __device__ __forceinline__ void put_source(float* f, const float (&v)[K], float w) const {
-#pragma unroll
-        for (int k = 0; k < K; ++k) f[(row(k) + 4) * 64 + lane] = with_source(k, v[k], w);
-    }
-    __device__ __forceinline__ void put(float* f, const float (&v)[K]) const {
-#pragma unroll
-        for (int k = 0; k < K; ++k) f[(row(k) + 4) * 64 + lane] = v[k];
-    }
-};
-
-}  // namespace
-
 // One forward step of the background (BG) and / or the scattered field (BN).
 // hist_mode 1 stores the background strains, 2 takes them from the history.
 template <int K, int NW, bool BG, bool BN>
-__global__ __launch_bounds__(NW * 64) void k_eb_tile(EbFusedArgs a, const EbTile* __restrict__ tiles, int ntiles,
+__global__ __launch_bounds__(NW * 64) void k_eb_tile(EbFusedArgs a, const StepTile* __restrict__ tiles, int ntiles,
                                                      int per_xcd, const int* __restrict__ rmap, float cax, float caz,
                                                      float idx, float idz, float w, int it, int nt, int hist_mode) {
     constexpr int NF = (BG ? 2 : 0) + (BN ? 2 : 0), FS = (K * NW + 8) * 64;
     __shared__ float lds[NF * FS];
     float *l0 = lds, *l1 = lds + FS, *l2 = lds + (BG ? 2 : 0) * FS, *l3 = l2 + FS;
-    EbTileLanes<K, NW> g;
+    TileLanes<K, NW> g;
     if (!g.init(tiles, ntiles, per_xcd)) return;
     const long long n = a.n;
     float gvx[K], gvz[K], gxx[K], gzz[K], gxz[K], svx[K], svz[K], sxx[K], szz[K], sxz[K], br[K], lam[K], mu[K];
@@ -246,14 +187,14 @@ __global__ __launch_bounds__(NW * 64) void k_eb_tile(EbFusedArgs a, const EbTile
 // k_eb_adj_s of step it).  UNDO: the background is taken one step back
 // alongside; otherwise the strains come from the history.
 template <int K, int NW, bool UNDO>
-__global__ __launch_bounds__(NW * 64) void k_eb_adj_tile(EbAdjArgs a, const EbTile* __restrict__ tiles, int ntiles,
+__global__ __launch_bounds__(NW * 64) void k_eb_adj_tile(EbAdjArgs a, const StepTile* __restrict__ tiles, int ntiles,
                                                          int per_xcd, const int* __restrict__ rmap, float cax,
                                                          float caz, float idx, float idz, float w, int it, int it_inj,
                                                          int nt) {
     constexpr int FS = (K * NW + 8) * 64;
     __shared__ float lds[(UNDO ? 4 : 2) * FS];
     float *l0 = lds, *l1 = lds + FS, *l2 = lds + (UNDO ? 2 : 0) * FS, *l3 = l2 + FS;
-    EbTileLanes<K, NW> g;
+    TileLanes<K, NW> g;
     if (!g.init(tiles, ntiles, per_xcd)) return;
     const long long n = a.n;
     const float *Al = a.Alm, *Ag = a.Abg;
@@ -389,15 +330,18 @@ __global__ __launch_bounds__(NW * 64) void k_eb_adj_tile(EbAdjArgs a, const EbTi
 
 static constexpr int kNW = 8;  // waves of a workgroup, and so columns per unit
 
-EbTiles plan_eb_tiles(const std::vector<int>& nxp, int nzp) {
-    const int wide = 6 * kNW - 2 * WAVE_HALO, narrow = 4 * kNW - 2 * WAVE_HALO;
+StepTiles plan_step_tiles(const std::vector<int>& nxp, int nzp, int narrow, int wide) {
     long long t = 0;
     for (int w : nxp)
         t += (long long)ceil_div(std::max(w - 2 * NOP, 0), wide) * ceil_div(std::max(nzp - 2 * NOP, 0), WAVE_ROWS);
-    return t >= 2048 ? EbTiles{true, wide} : EbTiles{false, narrow};
+    return t >= 2048 ? StepTiles{true, wide} : StepTiles{false, narrow};
 }
 
-void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const EbTile* tiles, int ntiles,
+StepTiles plan_eb_tiles(const std::vector<int>& nxp, int nzp) {
+    return plan_step_tiles(nxp, nzp, 4 * kNW - 2 * WAVE_HALO, 6 * kNW - 2 * WAVE_HALO);
+}
+
+void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, const StepTile* tiles, int ntiles,
                     bool wide, const int* rmap, float w, int it, bool do_bg, bool do_bn, int hist_mode) {
     const int per_xcd = (ntiles + 7) / 8;
     const float cax = b.dt / b.dx, caz = b.dt / b.dz, idx = 1.f / b.dx, idz = 1.f / b.dz;
@@ -420,7 +364,7 @@ void launch_eb_tile(hipStream_t st, const BatchShape& b, const EbFusedArgs& a, c
 #undef DS2D_EB_LAUNCH
 }
 
-void launch_eb_adj_tile(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const EbTile* tiles, int ntiles,
+void launch_eb_adj_tile(hipStream_t st, const BatchShape& b, const EbAdjArgs& a, const StepTile* tiles, int ntiles,
                         bool wide, const int* rmap, float w, int it, int it_inj, bool undo) {
     const int per_xcd = (ntiles + 7) / 8;
     const float cax = b.dt / b.dx, caz = b.dt / b.dz, idx = 1.f / b.dx, idz = 1.f / b.dz;

@@ -200,8 +200,8 @@ int ds2d_get_chunk_plan(ds2d_t* h, int* used);
  * capability). */
 int ds2d_set_fused_born(ds2d_t* h, int on, int width, int threads);
 /* Rotation-scheme forward modelling (ds2d_rot_forward): on (1, the default)
- * one fused launch per time step updates the velocity parts and theta /
- * omega (unsplit outside the damping strips); off (0) launches the per-cell
+ * one fused launch per time step on tiles updates the velocity (its P and S
+ * parts summed) and theta / omega (unsplit outside the damping strips); off (0) launches the per-cell
  * k_rot_v and k_rot_p of the reference layout.  No reference counterpart
  * (new capability). */
 int ds2d_set_fused_rotation(ds2d_t* h, int on);
