@@ -564,6 +564,14 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     ga.dt = sh.dt;
     ga.dx = sh.dx;
     ga.dz = sh.dz;
+    ga.kx = sh.dt / sh.dx;
+    ga.kz = sh.dt / sh.dz;
+    ga.ix = 1.f / sh.dx;
+    ga.iz = 1.f / sh.dz;
+    ga.kx64 = (double)sh.dt / sh.dx;
+    ga.kz64 = (double)sh.dt / sh.dz;
+    ga.ix64 = 1.0 / sh.dx;
+    ga.iz64 = 1.0 / sh.dz;
     ga.nt = nt;
     ga.wav = h->d_wav;
     ga.rmap = d_map;

@@ -35,6 +35,9 @@ struct GradFields {
 struct GradArgs {
     long long n, total_edge, wstride;
     float dt, dx, dz;
+    // dt/dx, dt/dz, 1/dx, 1/dz in both precisions
+    float kx, kz, ix, iz;
+    double kx64, kz64, ix64, iz64;
     int nt;
     const float* wav;
     const int *rmap, *rnext;          // column -> a trace, trace -> the next on its column (-1: none)

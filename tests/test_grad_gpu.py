@@ -55,6 +55,13 @@ def test_gradient_matches_oracle(allnx, allnz, pml, widths, boundaries, nt):
     assert abs(mf - omf) <= TOL * max(1.0, abs(omf))
 
 
+@pytest.mark.parametrize("boundary", [0, 1])
+@pytest.mark.parametrize("allnx,allnz", [(8, 56), (16, 57), (17, 55), (9, 112)])
+def test_gradient_at_the_edges_of_tiles(allnx, allnz, boundary):
+    """Update regions of exactly one and two tiles of 8 x 56 cells, one cell more and one less."""
+    test_gradient_matches_oracle(allnx, allnz, 4, [allnx], [boundary], 160)
+
+
 def test_born_records_of_traces_on_one_column():
     allnx, allnz, pml, nt = 40, 30, 20, 150
     vp, vs, _ = elastic_model(allnx, allnz, 21)
