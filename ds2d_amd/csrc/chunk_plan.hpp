@@ -4,8 +4,9 @@
 // window and one block of rows.  Its time is close to linear in the width:
 // on 128 windows of 440-1240 padded columns (2000x600 model, 704 lanes) a chunk
 // of w columns took 63 us + 2.80 us per column with the PML and 38 us + 1.90 us
-// with the random boundary, i.e. w plus 20-23 columns, the 12 + 12 columns of
-// the march outside the chunk.  One workgroup fits a CU (112 KB of LDS), so a
+// with the random boundary (at 1.36 and 0.92 ms a launch, 1.26 and 0.88 now),
+// i.e. w plus 20-23 columns, the 12 + 12 columns of the march outside the
+// chunk.  One workgroup fits a CU (135 KB of LDS), so a
 // launch is a list-scheduling problem: the k_fused2_step launch gives XCD x
 // the chunks [x*per, (x+1)*per) in order (block b runs chunk
 // (b % 8) * per + b / 8), and each of the XCD's CUs takes the next chunk

@@ -25,8 +25,19 @@
 // them back eight columns later.  The reading lane wrote the value itself
 // (program order), or a neighbouring workgroup whose halo overlaps wrote the
 // same bits (both compute it from the same inputs with the same code).
+//
+// What bounds the PML launch is the instruction stream of the one wave that
+// holds the damped rows, which every column's barrier waits for; the other
+// waves take their undamped columns with code that knows no damping.  On 128
+// windows of 440-1240 x 640 a launch takes 1.26 ms (1.39 with one code for all
+// waves; 0.88 with the random boundary, 0.92 before), 4.1 GB at 3.3 TB/s.  The
+// damping operands' round trip through memory is not the limit: kept in an
+// LDS ring instead, the launch took 3 % longer (the ring's own instructions),
+// and a higher priority for that wave changed nothing.
 #include "common.hpp"
 #include "kernels.hpp"
+
+#include <type_traits>
 
 namespace ds2d {
 
@@ -51,10 +62,11 @@ struct Col2 {
     float txx4, txz4;        // step-it stress of column j+4 (x-tap queues)
     float tzz, vx, vz, bx;   // step-it tzz, velocity and dt/rho of column j
     float lam, mu;           // moduli (x dt) of column j-4
-    int rec, rec2;           // traces recorded at column j (step it) and j-8 (step it+1)
-    // damping lanes only
-    float dxv, dzv, vxx, vzz;        // stage 1 velocity: damping, old vx_x, vz_z (column j)
-    float dxs, dzs, sxx, szz, sxz;   // stage 1 stress: damping, old txx_x, tzz_z, txz_x (column j-4)
+};
+// Stage 1 damping operands of march column j.
+struct Damp2 {
+    float dxv, dzv, vxx, vzz;        // velocity: damping, old vx_x, vz_z (column j)
+    float dxs, dzs, sxx, szz, sxz;   // stress: damping, old txx_x, tzz_z, txz_x (column j-4)
 };
 // Damping operands of stage 2 (loaded at the end of the previous column, in
 // flight across the barrier and stage 1: prefetching them two columns ahead
@@ -111,9 +123,10 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
 
     __shared__ float lds[2][8][T];
     // per-lane ring of stage 1's parameters (dt/rho of column j, moduli of
-    // column j-4): stage 2 reads them eight columns later instead of loading
-    // them again from memory
-    __shared__ float pring[8][3][T];
+    // column j-4) and of its tzz (column j-4): stage 2 reads them eight columns
+    // later instead of loading or carrying them (a register queue of tzz spills
+    // the damping code of 704 lanes, 168 registers each)
+    __shared__ float pring[8][4][T];
 
     const long long n = a.n;
     const float* Avx = a.A;
@@ -125,7 +138,6 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     const float* Plam = a.par + n;
     const float* Pmu = a.par + 2 * n;
     const uint32_t colb = (uint32_t)nzp * 4u;
-    const uint32_t zo4 = (uint32_t)(S.off + z) * 4u;
     const uint32_t zc4 = (uint32_t)(S.off + min(max(z, 0), nzp - 1)) * 4u;
     auto at = [](const float* p, uint32_t boff) -> float {
         return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + boff);
@@ -134,7 +146,7 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
         *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + boff) = v;
     };
     auto ld = [&](const float* p, int col) -> float {
-        return (zin && col >= 0 && col < nxp) ? at(p, zo4 + (uint32_t)col * colb) : 0.f;
+        return (zin && col >= 0 && col < nxp) ? at(p, zc4 + (uint32_t)col * colb) : 0.f;
     };
     auto ldc = [&](const float* p, int col) -> float {
         return at(p, zc4 + (uint32_t)min(max(col, 0), nxp - 1) * colb);
@@ -161,16 +173,13 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
         o.bx = ldc(Pbx, j);
         o.lam = ldc(Plam, j - 4);
         o.mu = ldc(Pmu, j - 4);
-        o.rec = o.rec2 = -1;
-        if (z == S.igz) {
-            if (j >= x0 && j < x1) o.rec = rmap[S.rmap_off + j];
-            if (j - 8 >= x0 && j - 8 < x1) o.rec2 = rmap[S.rmap_off + j - 8];
-        }
-        o.dxv = o.dzv = o.vxx = o.vzz = 0.f;
-        o.dxs = o.dzs = o.sxx = o.szz = o.sxz = 0.f;
-        if (PML && zupd) {
+        return o;
+    };
+    auto fetch_damp = [&](int j) {
+        Damp2 o{};
+        if (zupd) {
             if (inx(j) && (zdamp || damp_col2(S, j))) {
-                const uint32_t c = zo4 + (uint32_t)j * colb;
+                const uint32_t c = zc4 + (uint32_t)j * colb;
                 o.dxv = at(a.dampx, c);
                 o.dzv = at(a.dampz, c);
                 o.vxx = at(splitA(0), c);
@@ -178,7 +187,7 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
             }
             const int cs = j - 4;
             if (inx(cs) && (zdamp || damp_col2(S, cs))) {
-                const uint32_t c = zo4 + (uint32_t)cs * colb;
+                const uint32_t c = zc4 + (uint32_t)cs * colb;
                 o.dxs = at(a.dampx, c);
                 o.dzs = at(a.dampz, c);
                 o.sxx = at(splitA(4), c);
@@ -191,13 +200,11 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     // stage 2 damping operands of column j: the scratch holds what stage 1 of
     // this lane wrote eight (velocity) and eight (stress) columns earlier
     auto fetch_late = [&](int j) {
-        Late2 q;
-        q.dxv2 = q.dzv2 = q.vxx2 = q.vzz2 = 0.f;
-        q.dxs2 = q.dzs2 = q.sxx2 = q.szz2 = q.sxz2 = 0.f;
-        if (PML && zupd) {
+        Late2 q{};
+        if (zupd) {
             const int c2 = j - 8;
             if (l2v && inx(c2) && c2 >= x0 - 4 && c2 < x1 + 4 && (zdamp || damp_col2(S, c2))) {
-                const uint32_t c = zo4 + (uint32_t)c2 * colb;
+                const uint32_t c = zc4 + (uint32_t)c2 * colb;
                 q.dxv2 = at(a.dampx, c);
                 q.dzv2 = at(a.dampz, c);
                 q.vxx2 = at(scr(0), c);
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
             }
             const int c3 = j - 12;
             if (zown && inx(c3) && c3 >= x0 && c3 < x1 && (zdamp || damp_col2(S, c3))) {
-                const uint32_t c = zo4 + (uint32_t)c3 * colb;
+                const uint32_t c = zc4 + (uint32_t)c3 * colb;
                 q.dxs2 = at(a.dampx, c);
                 q.dzs2 = at(a.dampz, c);
                 q.sxx2 = at(scr(2), c);
@@ -221,10 +228,10 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     // (stress) or j-8+k (velocity) after the shift at column j
     float qxx[9], qxz[9], qzz[5], qvx[9], qvz[9];
     // stage 2 queues: step-it+1 stress s*[k] = column j-12+k, step-it+2 velocity w*[k] = column j-16+k
-    float sxx[9], sxz[9], szz[9], wvx[9], wvz[9];
+    float sxx[9], sxz[9], wvx[9], wvz[9];
     const int j0 = x0 - 12;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) pring[k][0][L] = pring[k][1][L] = pring[k][2][L] = 0.f;
+    for (int k = 0; k < 8; ++k) pring[k][0][L] = pring[k][1][L] = pring[k][2][L] = pring[k][3][L] = 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         qxx[k + 1] = ld(Atxx, j0 - 4 + k);
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
 #pragma unroll
     for (int k = 0; k < 4; ++k) qzz[k + 1] = ld(Atzz, j0 - 4 + k);
 #pragma unroll
-    for (int k = 0; k < 9; ++k) qvx[k] = qvz[k] = sxx[k] = sxz[k] = szz[k] = wvx[k] = wvz[k] = 0.f;
+    for (int k = 0; k < 9; ++k) qvx[k] = qvz[k] = sxx[k] = sxz[k] = wvx[k] = wvz[k] = 0.f;
 
     const float w1 = a.wav[it], w2 = a.wav[it + 1];
     auto tap = [&](int d) -> float {
@@ -261,11 +268,10 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     struct V2 {
         float vx, vz, sx, sz;  // new velocity, new splits vx_x, vz_z
     };
-    auto vel = [&](float ovx, float ovz, float ax, float ex, float bz, float cz, float bx, float dxv, float dzv,
+    auto vel = [&](auto dmp, float ovx, float ovz, float ax, float ex, float bz, float cz, float bx, float dxv, float dzv,
                    float pvxx, float pvzz, bool damped) -> V2 {
-        V2 r;
-        r.sx = r.sz = 0.f;
-        if (PML && __any(damped)) {
+        V2 r{};
+        if (decltype(dmp)::value && __any(damped)) {
             const float d1 = 1.f - dt * dxv / 2, r2 = __builtin_amdgcn_rcpf(1.f + dt * dxv / 2);
             const float d3 = 1.f - dt * dzv / 2, r4 = __builtin_amdgcn_rcpf(1.f + dt * dzv / 2);
             const float vxx = (d1 * pvxx + bx * idx * ax) * r2;
@@ -285,12 +291,11 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     struct S3 {
         float xx, zz, xz, sxx, szz, sxz;  // new stress and splits txx_x, tzz_z, txz_x
     };
-    auto str = [&](float txx, float tzz, float txz, float dvx, float dvzx, float dvz, float dvxz, float l, float mu,
+    auto str = [&](auto dmp, float txx, float tzz, float txz, float dvx, float dvzx, float dvz, float dvxz, float l, float mu,
                    float dxs, float dzs, float psxx, float pszz, float psxz, bool damped) -> S3 {
-        S3 r;
-        r.sxx = r.szz = r.sxz = 0.f;
+        S3 r{};
         const float l2m = l + 2 * mu;
-        if (PML && __any(damped)) {
+        if (decltype(dmp)::value && __any(damped)) {
             const float d1 = 1.f - dt * dxs / 2, r2 = __builtin_amdgcn_rcpf(1.f + dt * dxs / 2);
             const float d3 = 1.f - dt * dzs / 2, r4 = __builtin_amdgcn_rcpf(1.f + dt * dzs / 2);
             const float a1 = (d1 * psxx + l2m * dvx) * r2;
@@ -313,9 +318,20 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
         return r;
     };
 
-    auto column = [&](const int j, const Col2& o, const int p, Late2& q) {
+    // traces of 64 columns from x0 - 12 + 64 i on (-1: none), one per lane, and of those eight before
+    int rec1 = -1, rec2 = -1;
+    auto fetch_rec = [&](int j) {
+        const int c = j + (threadIdx.x & 63);
+        rec1 = c >= x0 && c < x1 ? rmap[S.rmap_off + c] : -1;
+        rec2 = c - 8 >= x0 && c - 8 < x1 ? rmap[S.rmap_off + c - 8] : -1;
+    };
+
+    // one march column; dmp: whether a cell of the wave is damped in it
+    auto column = [&](auto dmp, const int j, const Col2& o, const Damp2& d, const int p, Late2& q) {
+        constexpr bool D = decltype(dmp)::value;
         const int slot = j & 7;  // (j - 8) & 7 as well
         const float bx2 = pring[slot][0][L], lam2 = pring[slot][1][L], mu2 = pring[slot][2][L];
+        const float szz0 = pring[slot][3][L], szz4 = pring[slot ^ 4][3][L];
         pring[slot][0][L] = o.bx;
         pring[slot][1][L] = o.lam;
         pring[slot][2][L] = o.mu;
@@ -327,7 +343,6 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
             qvz[k] = qvz[k + 1];
             sxx[k] = sxx[k + 1];
             sxz[k] = sxz[k + 1];
-            szz[k] = szz[k + 1];
             wvx[k] = wvx[k + 1];
             wvz[k] = wvz[k + 1];
         }
@@ -342,7 +357,7 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
         lds[p][2][L] = qvx[4];  // vx, step it+1, column j-4
         lds[p][3][L] = qvz[4];  // vz, step it+1, column j-4
         lds[p][4][L] = sxz[4];  // txz, step it+1, column j-8
-        lds[p][5][L] = szz[4];  // tzz, step it+1, column j-8
+        lds[p][5][L] = szz4;  // tzz, step it+1, column j-8
         lds[p][6][L] = wvx[4];  // vx, step it+2, column j-12
         lds[p][7][L] = wvz[4];  // vz, step it+2, column j-12
         __syncthreads();
@@ -353,20 +368,21 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
             float ax = dxp(qxx), ex = dxm(qxz), bz = dzm(lds[p][0]), cz = dzp(lds[p][1]);
             if ((unsigned)(S.isx - j + 3) < 8u && z == S.isz) ax += w1 * tap(S.isx - j);
             if (j == S.isx) cz += w1 * tz;
-            const bool dv = PML && (zdamp || damp_col2(S, j));
-            const V2 r = vel(o.vx, o.vz, ax, ex, bz, cz, o.bx, o.dxv, o.dzv, o.vxx, o.vzz, dv);
+            const bool dv = D && (zdamp || damp_col2(S, j));
+            const V2 r = vel(dmp, o.vx, o.vz, ax, ex, bz, cz, o.bx, d.dxv, d.dzv, d.vxx, d.vzz, dv);
             nvx = r.vx;
             nvz = r.vz;
-            if (PML && dv && l2v && j >= x0 - 4 && j < x1 + 4) {
-                const uint32_t c = zo4 + (uint32_t)j * colb;
+            if (D && dv && l2v && j >= x0 - 4 && j < x1 + 4) {
+                const uint32_t c = zc4 + (uint32_t)j * colb;
                 st(scr(0), c, r.sx);
                 st(scr(1), c, r.sz);
             }
         }
         qvx[8] = nvx;
         qvz[8] = nvz;
-        if (zown && o.rec >= 0) {
-            const size_t q = (size_t)S.rec_off + (size_t)o.rec * nt + it;
+        const int tr1 = __builtin_amdgcn_readlane(rec1, (j - j0) & 63);
+        if (tr1 >= 0 && z == S.igz && zown) {
+            const size_t q = (size_t)S.rec_off + (size_t)tr1 * nt + it;
             a.rec_z[q] = nvz;
             a.rec_x[q] = nvx;
         }
@@ -380,38 +396,39 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
                 const float dvzx = dxp(qvz) * idx;
                 const float dvz = dzm(lds[p][3]) * idz;
                 const float dvxz = dzp(lds[p][2]) * idz;
-                const bool ds = PML && (zdamp || damp_col2(S, cs));
-                const S3 r = str(txx, tzz, txz, dvx, dvzx, dvz, dvxz, o.lam, o.mu, o.dxs, o.dzs, o.sxx, o.szz, o.sxz,
-                                 ds);
+                const bool ds = D && (zdamp || damp_col2(S, cs));
+                const S3 r = str(dmp, txx, tzz, txz, dvx, dvzx, dvz, dvxz, o.lam, o.mu, d.dxs, d.dzs, d.sxx, d.szz,
+                                 d.sxz, ds);
                 txx = r.xx;
                 tzz = r.zz;
                 txz = r.xz;
-                if (PML && ds && zown && cs >= x0 && cs < x1) {
-                    const uint32_t c = zo4 + (uint32_t)cs * colb;
+                if (D && ds && zown && cs >= x0 && cs < x1) {
+                    const uint32_t c = zc4 + (uint32_t)cs * colb;
                     st(scr(2), c, r.sxx);
                     st(scr(3), c, r.szz);
                     st(scr(4), c, r.sxz);
                 }
             }
             sxx[8] = txx;
-            szz[8] = tzz;
+            pring[slot][3][L] = tzz;
             sxz[8] = txz;
         }
 
         // ---- stage 2 velocity, column j-8 (step it+1 -> it+2)
         {
             const int c2 = j - 8;
+            const int tr2 = __builtin_amdgcn_readlane(rec2, (j - j0) & 63);
             float mvx = qvx[0], mvz = qvz[0];
             if (l2v && zupd && inx(c2)) {
                 float ax = dxp(sxx), ex = dxm(sxz), bz = dzm(lds[p][4]), cz = dzp(lds[p][5]);
                 if ((unsigned)(S.isx - c2 + 3) < 8u && z == S.isz) ax += w2 * tap(S.isx - c2);
                 if (c2 == S.isx) cz += w2 * tz;
-                const bool dv = PML && (zdamp || damp_col2(S, c2));
-                const V2 r = vel(mvx, mvz, ax, ex, bz, cz, bx2, q.dxv2, q.dzv2, q.vxx2, q.vzz2, dv);
+                const bool dv = D && (zdamp || damp_col2(S, c2));
+                const V2 r = vel(dmp, mvx, mvz, ax, ex, bz, cz, bx2, q.dxv2, q.dzv2, q.vxx2, q.vzz2, dv);
                 mvx = r.vx;
                 mvz = r.vz;
-                if (PML && dv && zown && c2 >= x0 && c2 < x1) {
-                    const uint32_t c = zo4 + (uint32_t)c2 * colb;
+                if (D && dv && zown && c2 >= x0 && c2 < x1) {
+                    const uint32_t c = zc4 + (uint32_t)c2 * colb;
                     st(splitB(0), c, r.sx);
                     st(splitB(3), c, r.sz);
                 }
@@ -419,11 +436,11 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
             wvx[8] = mvx;
             wvz[8] = mvz;
             if (zown && c2 >= x0 && c2 < x1) {
-                const uint32_t c = zo4 + (uint32_t)c2 * colb;
+                const uint32_t c = zc4 + (uint32_t)c2 * colb;
                 st(a.B, c, mvx);
                 st(a.B + n, c, mvz);
-                if (o.rec2 >= 0) {
-                    const size_t q = (size_t)S.rec_off + (size_t)o.rec2 * nt + it + 1;
+                if (tr2 >= 0 && z == S.igz) {
+                    const size_t q = (size_t)S.rec_off + (size_t)tr2 * nt + it + 1;
                     a.rec_z[q] = mvz;
                     a.rec_x[q] = mvx;
                 }
@@ -434,33 +451,33 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
         {
             const int c3 = j - 12;
             if (zown && c3 >= x0 && c3 < x1) {
-                float txx = sxx[0], tzz = szz[0], txz = sxz[0];
+                float txx = sxx[0], tzz = szz0, txz = sxz[0];
                 if (zupd && inx(c3)) {
                     const float dvx = dxm(wvx) * idx;
                     const float dvzx = dxp(wvz) * idx;
                     const float dvz = dzm(lds[p][7]) * idz;
                     const float dvxz = dzp(lds[p][6]) * idz;
-                    const bool ds = PML && (zdamp || damp_col2(S, c3));
-                    const S3 r = str(txx, tzz, txz, dvx, dvzx, dvz, dvxz, lam2, mu2, q.dxs2, q.dzs2, q.sxx2,
+                    const bool ds = D && (zdamp || damp_col2(S, c3));
+                    const S3 r = str(dmp, txx, tzz, txz, dvx, dvzx, dvz, dvxz, lam2, mu2, q.dxs2, q.dzs2, q.sxx2,
                                      q.szz2, q.sxz2, ds);
                     txx = r.xx;
                     tzz = r.zz;
                     txz = r.xz;
-                    if (PML && ds) {
-                        const uint32_t c = zo4 + (uint32_t)c3 * colb;
+                    if (D && ds) {
+                        const uint32_t c = zc4 + (uint32_t)c3 * colb;
                         st(splitB(4), c, r.sxx);
                         st(splitB(7), c, r.szz);
                         st(splitB(8), c, r.sxz);
                     }
                 }
-                const uint32_t c = zo4 + (uint32_t)c3 * colb;
+                const uint32_t c = zc4 + (uint32_t)c3 * colb;
                 st(a.B + 2 * n, c, txx);
                 st(a.B + 3 * n, c, tzz);
                 st(a.B + 4 * n, c, txz);
             }
         }
         // stage 2 damping operands of the next column, in flight across the barrier
-        q = fetch_late(j + 1);
+        if (D) q = fetch_late(j + 1);
     };
 
     // march columns [x0-12, x1+12) in passes of two columns, the operands of
@@ -468,12 +485,47 @@ __global__ __launch_bounds__(T) void k_fused2_step(FusedArgs a, float* __restric
     static_assert(PF == 2, "two steps per launch march with two columns in flight");
     const int jend = j0 + (x1 + 12 - j0 + 1) / 2 * 2;
     Col2 cA = fetch(j0), cB = fetch(j0 + 1);
-    Late2 q = fetch_late(j0);
-    for (int j = j0; j < jend; j += 2) {
-        column(j, cA, 0, q);
-        cA = fetch(j + 2);
-        column(j + 1, cB, 1, q);
-        cB = fetch(j + 3);
+    if constexpr (PML) {
+        // A wave without damped rows takes the columns of the middle with the code that knows no damping.
+        const bool zd = __any(zdamp && zupd);
+        auto damped_pair = [&](int j) {
+            return zd || (S.boundary == 0 && (j - 12 < S.pml || j + 1 > nxp - S.pml));
+        };
+        for (int j = j0; j < jend;) {
+            if (damped_pair(j)) {
+                Damp2 dA = fetch_damp(j), dB = fetch_damp(j + 1);
+                Late2 q = fetch_late(j);
+                do {
+                    if (((j - j0) & 63) == 0) fetch_rec(j);
+                    column(std::true_type{}, j, cA, dA, 0, q);
+                    cA = fetch(j + 2);
+                    dA = fetch_damp(j + 2);
+                    column(std::true_type{}, j + 1, cB, dB, 1, q);
+                    cB = fetch(j + 3);
+                    dB = fetch_damp(j + 3);
+                    j += 2;
+                } while (j < jend && damped_pair(j));
+            }
+            const Damp2 d{};
+            Late2 q{};
+            for (; j < jend && !damped_pair(j); j += 2) {
+                if (((j - j0) & 63) == 0) fetch_rec(j);
+                column(std::false_type{}, j, cA, d, 0, q);
+                cA = fetch(j + 2);
+                column(std::false_type{}, j + 1, cB, d, 1, q);
+                cB = fetch(j + 3);
+            }
+        }
+    } else {
+        const Damp2 d{};
+        Late2 q{};
+        for (int j = j0; j < jend; j += 2) {
+            if (((j - j0) & 63) == 0) fetch_rec(j);
+            column(std::false_type{}, j, cA, d, 0, q);
+            cA = fetch(j + 2);
+            column(std::false_type{}, j + 1, cB, d, 1, q);
+            cB = fetch(j + 3);
+        }
     }
 }
 
