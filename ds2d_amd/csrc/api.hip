@@ -1370,9 +1370,10 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
     if ((rc = h->fbuf("armap", std::max<long long>(B.total_rmap, 1), &w.rmap))) return rc;
     HIP_TRY(hipMemsetAsync(w.rmap, 0xff, B.total_rmap * 4, h->st));
     launch_fast_rmap(h->st, B.shape, w.rmap);
-    // fused steps: store mode, 32-bit cell indices within a field (from one window to the largest batches
-    // faster than the per-cell kernels: 5.3 against 8 us a step on 331x181, 33 against 92 on 3.2 M cells)
-    w.fused = w.store && n <= FUSED_MAX_CELLS && h->acou_fused != 0;
+    // fused steps: store mode, 32-bit byte offsets within a window's doubles (from one window to the largest
+    // batches faster than the per-cell kernels: 5 against 8 us a step on 331x181, 26 against 92 on 3.2 M cells)
+    w.fused = w.store && n <= FUSED_MAX_CELLS && (long long)B.shape.max_nxp * B.shape.nzp < (1LL << 29) &&
+              h->acou_fused != 0;
     if (w.fused && h->fbuf("acoubg2", (size_t)n * 3, &w.bg2)) {  // no room for the second background state
         w.fused = false;
         (void)hipGetLastError();

@@ -22,69 +22,18 @@
 // columns are computed again by every strip.
 #include "common.hpp"
 #include "kernels.hpp"
-#include "wave.hpp"
+#include "tile_lanes.hpp"
 
 namespace ds2d {
 
 namespace {
 
-// A tile: RX = K * NW columns of 64 rows, one wave per column at a time
-// (column = unit * NW + wave); it owns all but the eight outer ones.
 constexpr int NW = 8, K = ACOU_TILE_COLS / NW + 2 * WAVE_HALO / NW;
-struct Tile {
-    static constexpr int RX = K * NW;
-    StepTile T;
-    int lane, wv, z, ix0;
-    bool zu, zown;
-    __device__ __forceinline__ bool init(const StepTile* tiles, int ntiles, int per_xcd) {
-        const int ch = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if (ch >= ntiles) return false;
-        T = tiles[ch];
-        lane = threadIdx.x & 63;
-        wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        z = T.z0 - WAVE_HALO + lane;
-        ix0 = T.x0 - WAVE_HALO;
-        zu = z >= NOP && z < T.nzp - NOP;
-        zown = zu && lane >= WAVE_HALO && lane < 64 - WAVE_HALO;
-        return true;
-    }
-    __device__ __forceinline__ int row(int k) const { return k * NW + wv; }  // uniform over the wave
-    __device__ __forceinline__ bool row_upd(int k) const {
-        const int ix = ix0 + row(k);
-        return ix >= NOP && ix < T.nxp - NOP;
-    }
-    __device__ __forceinline__ bool upd(int k) const { return zu && row_upd(k); }
-    // whether the wave's column k is at least m columns inside the tile
-    __device__ __forceinline__ bool inside(int k, int m) const {
-        return (k * NW >= m || row(k) >= m) && (k * NW + NW <= RX - m || row(k) < RX - m);
-    }
-    __device__ __forceinline__ bool own(int k) const { return inside(k, WAVE_HALO) && row_upd(k) && zown; }
-    __device__ __forceinline__ uint32_t cell(int k) const {
-        return (uint32_t)(T.off + (long long)(ix0 + row(k)) * T.nzp + z);
-    }
-    // history cell of the window, or -1
-    __device__ __forceinline__ long long hist(int k, int it) const {
-        const int lx = ix0 + row(k) - T.pml, lz = z - T.pml;
-        if (lx < 0 || lx >= T.nx || lz < 0 || lz >= T.nz) return -1;
-        return T.hist_off + ((long long)it * T.nx + lx) * T.nz + lz;
-    }
-};
-// x taps of the wave's column k from an LDS copy with four spare columns on
-// each side: the seven other columns of a forward (backward) difference.
+using Tile = TileLanes<K, NW>;
+
 template <typename R>
-__device__ __forceinline__ R dplus_x(const R* f, int k, int wv, int lane, R own) {
-    const R* X = f + (k * NW + wv + 4) * 64 + lane;
-    return taps(X[64], own, X[128], X[-64], X[192], X[-128], X[256], X[-192]);
-}
-template <typename R>
-__device__ __forceinline__ R dminus_x(const R* f, int k, int wv, int lane, R own) {
-    const R* X = f + (k * NW + wv + 4) * 64 + lane;
-    return taps(own, X[-64], X[64], X[-128], X[128], X[-192], X[192], X[-256]);
-}
-template <typename R>
-__device__ __forceinline__ void publish(R* f, int wv, int lane, const R (&v)[K]) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) f[(k * NW + wv + 4) * 64 + lane] = v[k];
+__device__ __forceinline__ void publish(R* f, const Tile& g, const R (&v)[K]) {
+    g.put(f, v);
     __syncthreads();
 }
 
@@ -101,19 +50,16 @@ __global__ __launch_bounds__(NW * 64) void k_acou_born_tile(AcouFusedArgs a, con
     float p[K], vx[K], vz[K], bu[K], kk[K], src[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        p[k] = vx[k] = vz[k] = bu[k] = kk[k] = src[k] = 0.f;
-        if (!g.upd(k)) continue;
-        const uint32_t c = g.cell(k);
-        p[k] = (a.A + 2 * n)[c];
+        vx[k] = vz[k] = bu[k] = kk[k] = src[k] = 0.f;
+        p[k] = g.at(a.A + 2 * n, k);
         if (g.inside(k, 4)) {
-            vx[k] = a.A[c];
-            vz[k] = (a.A + n)[c];
-            bu[k] = a.b[c];
+            vx[k] = g.at(a.A, k);
+            vz[k] = g.at(a.A + n, k);
+            bu[k] = g.at(a.b, k);
         }
-        if (g.inside(k, 8) && g.zown) {
-            kk[k] = a.k[c];
-            const long long h = g.hist(k, it);
-            if (h >= 0) src[k] = 2 * a.m[c] * a.hist[h];
+        if (g.inside(k, 8)) {
+            kk[k] = g.at(a.k, k);
+            src[k] = 2 * g.at(a.m, k) * g.hist(a.hist, k, it);  // m is zero outside the physical window
         }
     }
     int rec = -1;  // traces of the wave's columns: lane k holds column k's
@@ -121,24 +67,23 @@ __global__ __launch_bounds__(NW * 64) void k_acou_born_tile(AcouFusedArgs a, con
         const int ix = g.ix0 + g.lane * NW + g.wv;
         if (ix >= NOP && ix < g.T.nxp - NOP) rec = rmap[g.T.rmap_off + ix];
     }
-    publish(lp, g.wv, g.lane, p);
+    publish(lp, g, p);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         if (!g.inside(k, 4)) continue;
-        vx[k] += a.ax * bu[k] * dplus_x(lp, k, g.wv, g.lane, p[k]);
+        vx[k] += a.ax * bu[k] * g.dplus_x(lp, k, p[k]);
         vz[k] += a.az * bu[k] * dplus_z(p[k]);
     }
-    publish(lv, g.wv, g.lane, vx);
+    publish(lv, g, vx);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         if (!g.inside(k, 8)) continue;
-        const float dvx = dminus_x(lv, k, g.wv, g.lane, vx[k]), dvz = dminus_z(vz[k]);
+        const float dvx = g.dminus_x(lv, k, vx[k]), dvz = dminus_z(vz[k]);
         const float pn = p[k] + (kk[k] * (a.ax * dvx + a.az * dvz) + src[k]);
         if (!(g.row_upd(k) && g.zown)) continue;
-        const uint32_t c = g.cell(k);
-        a.B[c] = vx[k];
-        (a.B + n)[c] = vz[k];
-        (a.B + 2 * n)[c] = pn;
+        g.at(a.B, k) = vx[k];
+        g.at(a.B + n, k) = vz[k];
+        g.at(a.B + 2 * n, k) = pn;
         const int r = __builtin_amdgcn_readlane(rec, k);
         if (r >= 0 && g.z == g.T.igz) a.rec[g.T.rec_off + (long long)r * nt + it] = pn;
     }
@@ -158,22 +103,17 @@ __global__ __launch_bounds__(NW * 64) void k_acou_adj_tile(AcouFusedArgs a, cons
     float lp[K], w[K], vx[K], vz[K], ux[K], uz[K], gr[K], dp[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        lp[k] = w[k] = vx[k] = vz[k] = ux[k] = uz[k] = gr[k] = dp[k] = 0.f;
-        if (!g.upd(k)) continue;
-        const uint32_t c = g.cell(k);
-        lp[k] = (a.A + 2 * n)[c];
-        w[k] = a.k[c];
+        vx[k] = vz[k] = ux[k] = uz[k] = gr[k] = dp[k] = 0.f;
+        lp[k] = g.at(a.A + 2 * n, k);
+        w[k] = g.at(a.k, k);
         if (g.inside(k, 4)) {
-            vx[k] = a.A[c];
-            vz[k] = (a.A + n)[c];
-            ux[k] = a.b[c];
+            vx[k] = g.at(a.A, k);
+            vz[k] = g.at(a.A + n, k);
+            ux[k] = g.at(a.b, k);
         }
-        if (g.inside(k, 8) && g.zown) {
-            const long long h = g.hist(k, it);
-            if (h >= 0) {
-                dp[k] = a.hist[h];
-                gr[k] = a.grad[c];
-            }
+        if (g.inside(k, 8)) {
+            dp[k] = g.hist(a.hist, k, it);
+            gr[k] = g.at(a.grad, k);
         }
     }
     float res = 0.f;  // residuals of the wave's columns: lane k holds column k's
@@ -184,28 +124,27 @@ __global__ __launch_bounds__(NW * 64) void k_acou_adj_tile(AcouFusedArgs a, cons
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) w[k] *= lp[k];
-    publish(lw, g.wv, g.lane, w);
+    publish(lw, g, w);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         uz[k] = ux[k];
         if (!g.inside(k, 4)) continue;
-        vx[k] += -(a.ax * dplus_x(lw, k, g.wv, g.lane, w[k]));
+        vx[k] += -(a.ax * g.dplus_x(lw, k, w[k]));
         vz[k] += -(a.az * dplus_z(w[k]));
-        ux[k] *= vx[k];  // zero outside the update region, where b was not loaded
+        ux[k] *= vx[k];  // zero on the frame, as b
         uz[k] *= vz[k];
     }
-    publish(lu, g.wv, g.lane, ux);
+    publish(lu, g, ux);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         if (!g.inside(k, 8)) continue;
-        const float gx = dminus_x(lu, k, g.wv, g.lane, ux[k]), gz = dminus_z(uz[k]);
+        const float gx = g.dminus_x(lu, k, ux[k]), gz = dminus_z(uz[k]);
         const float rk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(res), k));
         if (!(g.row_upd(k) && g.zown)) continue;
-        const uint32_t c = g.cell(k);
-        a.B[c] = vx[k];
-        (a.B + n)[c] = vz[k];
-        (a.B + 2 * n)[c] = lp[k] + -(a.ax * gx + a.az * gz) + (g.z == g.T.igz ? rk : 0.f);
-        if (g.hist(k, it) >= 0) a.grad[c] = gr[k] + 2 * dp[k] * lp[k];
+        g.at(a.B, k) = vx[k];
+        g.at(a.B + n, k) = vz[k];
+        g.at(a.B + 2 * n, k) = lp[k] + -(a.ax * gx + a.az * gz) + (g.z == g.T.igz ? rk : 0.f);
+        if (g.phys(k)) g.at(a.grad, k) = gr[k] + 2 * dp[k] * lp[k];
     }
 }
 
@@ -224,25 +163,23 @@ __global__ __launch_bounds__(NW * 64) void k_acou_bg_tile(const double* __restri
     float b[K], m[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        p[k] = vx[k] = vz[k] = 0.;
+        vx[k] = vz[k] = 0.;
         b[k] = m[k] = 0.f;
-        if (!g.upd(k)) continue;
-        const uint32_t c = g.cell(k);
-        p[k] = (A + 2 * n)[c];
+        p[k] = g.at(A + 2 * n, k);
         if (g.inside(k, 4)) {
-            vx[k] = A[c];
-            vz[k] = (A + n)[c];
-            b[k] = bu[c];
+            vx[k] = g.at(A, k);
+            vz[k] = g.at(A + n, k);
+            b[k] = g.at(bu, k);
         }
-        if (g.inside(k, 8)) m[k] = kk[c];
+        if (g.inside(k, 8)) m[k] = g.at(kk, k);
     }
     const double w = wav[it];
     const double wz = w * src_tap<double>(g.T.isz - g.z);
-    publish(lp, g.wv, g.lane, p);
+    publish(lp, g, p);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         if (!g.inside(k, 4)) continue;
-        double dx = dplus_x(lp, k, g.wv, g.lane, p[k]), dz = dplus_z(p[k]);
+        double dx = g.dplus_x(lp, k, p[k]), dz = dplus_z(p[k]);
         const int d = g.T.isx - g.ix0 - g.row(k);
         if ((unsigned)(d + 3) < 8u) {
             if (g.z == g.T.isz) dx += w * src_tap<double>(d);
@@ -252,19 +189,17 @@ __global__ __launch_bounds__(NW * 64) void k_acou_bg_tile(const double* __restri
         vz[k] += az * b[k] * dz;
     }
     __syncthreads();
-    publish(lp, g.wv, g.lane, vx);
+    publish(lp, g, vx);
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         if (!g.inside(k, 8)) continue;
-        const double dvx = dminus_x(lp, k, g.wv, g.lane, vx[k]), dvz = dminus_z(vz[k]);
+        const double dvx = g.dminus_x(lp, k, vx[k]), dvz = dminus_z(vz[k]);
         if (!(g.row_upd(k) && g.zown)) continue;
         const double d = (double)m[k] * (ax * dvx + az * dvz);
-        const uint32_t c = g.cell(k);
-        B[c] = vx[k];
-        (B + n)[c] = vz[k];
-        (B + 2 * n)[c] = p[k] + d;
-        const long long h = g.hist(k, it);
-        if (h >= 0) hist[h] = (float)d;
+        g.at(B, k) = vx[k];
+        g.at(B + n, k) = vz[k];
+        g.at(B + 2 * n, k) = p[k] + d;
+        if (g.phys(k)) g.hist(hist, k, it) = (float)d;
     }
 }
 

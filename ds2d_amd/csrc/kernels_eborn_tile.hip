@@ -18,8 +18,8 @@
 // 36 in two per-cell kernels before); one of 141x101 54.9 -> 5.3 ms; forward on
 // 16 windows of 440-1240 x 1080 392 -> 350 us a step (4.3 TB/s of the 100 B),
 // adjoint with reversal on 8 of them 208 -> 193 us.
-// Width: 32 owned columns (six units) leave one workgroup of 221-248 VGPRs a
-// CU and less halo; 16 (four units) leave two.  Narrow: 24.0 against 25.1 ms on
+// Width: 32 owned columns (six units, two workgroups of 126 registers a CU)
+// have less halo, 16 (four units) more workgroups.  Narrow: 24.0 against 25.1 ms on
 // the 8 windows (1064 wide tiles), 5.3 against 6.7 on one; wide: 56.1 against
 // 59.3 ms on the 16 large windows (9900 tiles), 41.8 against 55.3 for the
 // adjoint of 8 (5000).  Hence the line at 2048 wide tiles.
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NW * 64) void k_eb_tile(EbFusedArgs a, const StepTi
             (a.B + 3 * n)[c] = gzz[k] + ebm::inc_zz(m, cax, caz, dvx, dvz);
             (a.B + 4 * n)[c] = gxz[k] + ebm::inc_xz(m, cax, caz, dvzx, dvxz);
             if (hist_mode == 1 && phys) {
-                const size_t h = g.hist(k, it);
+                const size_t h = g.hist_cell(k, it);
                 a.hist[h] = exx;
                 a.hist[h + a.hstride] = ezz;
                 a.hist[h + 2 * a.hstride] = exz;
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(NW * 64) void k_eb_tile(EbFusedArgs a, const StepTi
             float txz = sxz[k] + ebm::inc_xz(m, cax, caz, bvzx, bvxz);
             if (phys) {
                 if (!BG) {
-                    const size_t h = g.hist(k, it);
+                    const size_t h = g.hist_cell(k, it);
                     exx = a.hist[h];
                     ezz = a.hist[h + a.hstride];
                     exz = a.hist[h + 2 * a.hstride];
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(NW * 64) void k_eb_adj_tile(EbAdjArgs a, const Step
             (a.Bbg + 3 * n)[c] = gzz[k] - ebm::inc_zz(m, cax, caz, dvx, dvz);
             (a.Bbg + 4 * n)[c] = gxz[k] - ebm::inc_xz(m, cax, caz, dvzx, dvxz);
         } else if (phys) {
-            const size_t h = g.hist(k, it);
+            const size_t h = g.hist_cell(k, it);
             exx = a.hist[h];
             ezz = a.hist[h + a.hstride];
             exz = a.hist[h + 2 * a.hstride];

@@ -15,7 +15,7 @@
 // more in the strips), against 56 B with the four velocity parts kept apart and
 // 120 B for k_rot_v + k_rot_p.  On tiles (tile_lanes.hpp) the next bound is the
 // issue of vector operations, 280 per 64 owned cells with the halo.  Measured
-// on 16 windows of 440-1240 x 640: 115 us a step (344 MB of fields, 73 us at
+// on 16 windows of 440-1240 x 640: 105 us a step (344 MB of fields, 73 us at
 // the rate of a large copy), against 196 us for a march along x with LDS
 // columns; one 141x101 window 8.6 us against 84.  Errors against 64 bits fall
 // from 5.4e-7 to 4.8e-7 with the fewer sums.

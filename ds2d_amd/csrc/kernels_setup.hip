@@ -73,7 +73,9 @@ __global__ __launch_bounds__(256) void k_setup(SetupArgs a, Med m, float* bu, fl
     m.dmp[c] = a.img_pp ? a.img_pp[gidx] : 0.f;
     m.dms[c] = a.img_ps ? a.img_ps[gidx] : 0.f;
     if (bu) {
-        bu[c] = 1.f / rho;
+        // no buoyancy on the outermost cells, which are never updated: the tile kernels rely on it
+        const bool fixed = ix < NOP || ix >= S.nxp - NOP || iz < NOP || iz >= S.nzp - NOP;
+        bu[c] = fixed ? 0.f : 1.f / rho;
         kk[c] = rho * vp * vp;
         refl[c] = (!frame && a.img_pp) ? a.img_pp[gidx] : 0.f;
     }
