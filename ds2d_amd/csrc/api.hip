@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "chunk_plan.hpp"
+#include "record_copy.hpp"
 #include "wave.hpp"
 #include "unet.hpp"
 
@@ -68,6 +69,7 @@ struct ds2d_ctx {
     float *d_vp = nullptr, *d_vs = nullptr, *d_rho = nullptr;  // global model
     float *d_ipp = nullptr, *d_ips = nullptr;                  // global image
     float* d_grad7 = nullptr;                                  // accumulated gradients
+    RecordCopy records;                                        // records to the caller's memory
     bool have_model = false, have_image = false, have_shot = false;
     // current single shot (ds2d_set_shot)
     ds2d_shot cur{};
@@ -141,6 +143,12 @@ struct Batch {
     int total_traces = 0;
     bool any_pml = false;
 };
+
+// The caller's record buffers, while the device still computes.
+void prepare_records(const Batch& B, float* z, float* x) {
+    RecordCopy::prepare(z, B.total_rec * 4);
+    RecordCopy::prepare(x, B.total_rec * 4);
+}
 
 int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     const ds2d_geom& g = h->g;
@@ -611,8 +619,8 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     }
     if (!full) {
         if (B.total_rec > 0) {
-            HIP_TRY(hipMemcpyAsync(out_z, rs_z, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-            HIP_TRY(hipMemcpyAsync(out_x, rs_x, B.total_rec * 4, hipMemcpyDeviceToHost, st));
+            prepare_records(B, out_z, out_x);
+            HIP_TRY(h->records.fetch(st, B.total_rec, out_z, rs_z, out_x, rs_x));
         }
         HIP_TRY(hipStreamSynchronize(st));
         HIP_TRY(hipGetLastError());
@@ -1028,6 +1036,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         bytes_v = (double)B.total_cells * 8 * 4 + pml_cells * 10 * 4;
         bytes_s = (double)B.total_cells * 10 * 4 + pml_cells * 14 * 4;
     }
+    prepare_records(B, rec_z, rec_x);
     if ((rc = stats_end(h, stats, cu, launches, 0))) return rc;
     {
         double kv, ks;
@@ -1048,9 +1057,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         }
         if (stats) *stats = h->last;
     }
-    if (rec_z) HIP_TRY(hipMemcpyAsync(rec_z, rz, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-    if (rec_x) HIP_TRY(hipMemcpyAsync(rec_x, rx, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(h->records.fetch(st, B.total_rec, rec_z, rz, rec_x, rx));
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -1595,10 +1602,9 @@ int ds2d_born_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, const float
     stats_loop_begin(h);
     acou_fwd(h, B, w, true, true, true);
     stats_loop_end(h);
+    prepare_records(B, rec_bg, rec_born);
     if ((rc = stats_end(h, stats, padded_cells(B) * h->g.nt * 2, h->g.nt, 0))) return rc;
-    if (rec_bg) HIP_TRY(hipMemcpyAsync(rec_bg, w.rec, B.total_rec * 4, hipMemcpyDeviceToHost, h->st));
-    if (rec_born) HIP_TRY(hipMemcpyAsync(rec_born, w.rec2, B.total_rec * 4, hipMemcpyDeviceToHost, h->st));
-    HIP_TRY(hipStreamSynchronize(h->st));
+    HIP_TRY(h->records.fetch(h->st, B.total_rec, rec_bg, w.rec, rec_born, w.rec2));
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -1963,6 +1969,7 @@ int ds2d_eborn_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, const floa
     stats_loop_begin(h);
     eb_fwd(h, B, w, true);
     stats_loop_end(h);
+    prepare_records(B, rec_z, rec_x);
     if ((rc = stats_end(h, stats, 2 * eb_cells(B, h->g.nt), 2LL * h->g.nt, 0))) return rc;
     // the fused forward step (first launch group): 100 B per padded cell (both states in and out, rho,
     // lambda, mu, the two image samples)
@@ -1977,9 +1984,7 @@ int ds2d_eborn_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, const floa
     }
     h->last.alg_bytes = w.alt ? (double)cells0 * 25 * 4 : 0;
     if (stats) *stats = h->last;
-    HIP_TRY(hipMemcpyAsync(rec_z, w.rec, B.total_rec * 4, hipMemcpyDeviceToHost, h->st));
-    HIP_TRY(hipMemcpyAsync(rec_x, w.rec + w.R, B.total_rec * 4, hipMemcpyDeviceToHost, h->st));
-    HIP_TRY(hipStreamSynchronize(h->st));
+    HIP_TRY(h->records.fetch(h->st, B.total_rec, rec_z, w.rec, rec_x, w.rec + w.R));
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -2528,6 +2533,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
             std::swap(a, b);
         }
         stats_loop_end(h);
+        prepare_records(B, rec_z, rec_x);
         if ((rc = stats_end(h, stats, padded_cells(B) * nt, nt, 0))) return rc;
         double kf, unused;
         smp.averages(&kf, &unused);
@@ -2544,9 +2550,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
         h->last.aux_alg_bytes = 0;
         h->last.kernel_samples = smp.n;
         if (stats) *stats = h->last;
-        if (rec_z) HIP_TRY(hipMemcpyAsync(rec_z, rs, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-        if (rec_x) HIP_TRY(hipMemcpyAsync(rec_x, rs + R, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+        HIP_TRY(h->records.fetch(st, B.total_rec, rec_z, rs, rec_x, rs + R));
         HIP_TRY(hipGetLastError());
         return 0;
     }
@@ -2579,9 +2583,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
     h->last.aux_alg_bytes = p_dom ? bv : bp;
     h->last.kernel_samples = smp.n;
     if (stats) *stats = h->last;
-    if (rec_z) HIP_TRY(hipMemcpyAsync(rec_z, rs, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-    if (rec_x) HIP_TRY(hipMemcpyAsync(rec_x, rs + R, B.total_rec * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(h->records.fetch(st, B.total_rec, rec_z, rs, rec_x, rs + R));
     HIP_TRY(hipGetLastError());
     return 0;
 }
