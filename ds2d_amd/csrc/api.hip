@@ -827,6 +827,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         tp = plan_tiles(nxp, sh.nzp, device_cus());
         const bool untuned = !h->fwd_two && !h->chunk_w && !h->chunk_t && !h->chunk_d && h->tblock == 1;
         tile = h->fwd_two == 2 ? tp.rounds <= TILE_MAX_ROUNDS : untuned && tp.rounds <= 8;
+        tile = tile && n < (1LL << 26);  // 32-bit byte offsets over the 15 fields (always so at these rounds)
     }
     long long launches = 0;
     StepSampler smp;
