@@ -154,12 +154,18 @@ struct GradTile {
         return *reinterpret_cast<float*>(reinterpret_cast<char*>(w + S.win_off) + c * 4u);
     }
     __device__ __forceinline__ int place() const { return (wv + NOP) * 64 + lane; }
-    __device__ __forceinline__ bool upd() const { return zupd && own(); }
+    // One mask each, without branches, and what a cell's kind decides is a
+    // value and not an address: of loads of one register in both arms of an if
+    // behind such a chain of conditions the compiler (ROCm 7.2) made one load of
+    // a selected address, and lost the choice of the lanes above and below the
+    // physical window. So the total is loaded by every cell of the region and
+    // replaced where the state is another one.
+    __device__ __forceinline__ bool upd() const { return zupd & own(); }
     __device__ __forceinline__ bool interior() const {
-        return col() >= S.pml && col() < S.nxp - S.pml && z >= S.pml && z < S.nzp - S.pml;
+        return (col() >= S.pml) & (col() < S.nxp - S.pml) & (z >= S.pml) & (z < S.nzp - S.pml);
     }
     __device__ __forceinline__ bool damped() const {
-        return S.boundary == 0 && (col() < S.pml || col() > S.nxp - S.pml || z < S.pml || z > S.nzp - S.pml);
+        return (S.boundary == 0) & ((col() < S.pml) | (col() > S.nxp - S.pml) | (z < S.pml) | (z > S.nzp - S.pml));
     }
     // values of the wave's own column, of its halo column
     template <typename T>
@@ -290,14 +296,13 @@ struct VelState {
     __device__ __forceinline__ void load(const GradTile& g, const EFieldT<T>& f) {
         p = q = pz = qz = T(0);
         if (!g.upd()) return;
+        p = g.at(f.vx);
+        q = g.at(f.vz);
         if (g.damped()) {
             p = g.at(f.vx_x);
             q = g.at(f.vz_x);
             pz = g.at(f.vx_z);
             qz = g.at(f.vz_z);
-        } else {
-            p = g.at(f.vx);
-            q = g.at(f.vz);
         }
     }
 };
@@ -332,6 +337,9 @@ struct StressState {
     __device__ __forceinline__ void load(const GradTile& g, const EFieldT<T>& f) {
         a = b = e = az = bz = ez = T(0);
         if (!g.upd()) return;
+        a = g.at(BARE ? f.txx_x : f.txx);
+        b = g.at(BARE ? f.tzz_z : f.tzz);
+        e = g.at(BARE ? f.txz_x : f.txz);
         if (g.damped()) {
             a = g.at(f.txx_x);
             b = g.at(f.tzz_x);
@@ -339,10 +347,6 @@ struct StressState {
             az = g.at(f.txx_z);
             bz = g.at(f.tzz_z);
             ez = g.at(f.txz_z);
-        } else {
-            a = g.at(BARE ? f.txx_x : f.txx);
-            b = g.at(BARE ? f.tzz_z : f.tzz);
-            e = g.at(BARE ? f.txz_x : f.txz);
         }
     }
 };
@@ -535,11 +539,10 @@ struct AdjStress {
         if (!g.upd()) return;
         a = g.at(f.txx);
         b = g.at(f.tzz);
+        e = g.at(f.txz);
         if (g.damped()) {
             e = g.at(f.txz_x);
             ez = g.at(f.txz_z);
-        } else {
-            e = g.at(f.txz);
         }
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
@@ -686,17 +689,15 @@ struct AdjVel {
     __device__ __forceinline__ void load(const GradTile& g, const EField& f, bool held) {
         p = q = pz = qz = 0.f;
         if (!g.upd()) return;
+        const float* const hx = held ? f.vx_x : f.vx;  // one select per lane, not two arms
+        const float* const hz = held ? f.vz_z : f.vz;
+        p = g.at(hx);
+        q = g.at(hz);
         if (g.damped()) {
             p = g.at(f.vx_x);
             q = g.at(f.vz_x);
             pz = g.at(f.vx_z);
             qz = g.at(f.vz_z);
-        } else if (held) {
-            p = g.at(f.vx_x);
-            q = g.at(f.vz_z);
-        } else {
-            p = g.at(f.vx);
-            q = g.at(f.vz);
         }
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
@@ -805,18 +806,14 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m
         MedState rho;
         TB* l = (TB*)lf;
         Stress3<TB> s;
-        TB vx = 0, vz = 0;
+        TB vx = 0, vz = 0, lx = 0, lz = 0;
         s.load(g, F.bg.txx, F.bg.tzz, F.bg.txz);
         rho.load(g, m.rho);
-        // bg itself goes on without the bands (its splits do), lv takes them
         if (g.upd()) {
-            if (g.interior()) {
-                vx = g.at(F.bg.vx);
-                vz = g.at(F.bg.vz);
-            } else {
-                vx = g.at(F.lvx);
-                vz = g.at(F.lvz);
-            }
+            vx = g.at(F.bg.vx);
+            vz = g.at(F.bg.vz);
+            lx = g.at(F.lvx);
+            lz = g.at(F.lvz);
         }
         s.put(g, l);
         __syncthreads();
@@ -826,13 +823,12 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m
         if (!g.own()) return;
         const Grad4<TB> t(g, s, l);
         if (!g.zupd) return;
+        // bg itself goes on without the bands (its splits do), lv takes them; outside the physical
+        // window bg has step k's bands, which the source strains of this step still see
         const bool in = g.interior();
-        if (in) {
-            const TB br = TB(1) / (TB)rho.v;
-            vx -= br * kx * t.a + br * kz * t.b;
-            vz -= br * kx * t.e + br * kz * t.d;
-        }
-        // outside the physical window: step k's bands, which the source strains of this step still see
+        const TB br = TB(1) / (TB)rho.v;
+        vx = in ? vx - (br * kx * t.a + br * kz * t.b) : lx;
+        vz = in ? vz - (br * kx * t.e + br * kz * t.d) : lz;
         if (in || F.edges) {
             g.at(F.bg.vx) = vx;
             g.at(F.bg.vz) = vz;

@@ -62,6 +62,14 @@ def test_gradient_at_the_edges_of_tiles(allnx, allnz, boundary):
     test_gradient_matches_oracle(allnx, allnz, 4, [allnx], [boundary], 160)
 
 
+def test_background_beside_the_window(monkeypatch):
+    """The rows above and below the physical window, of which the background's Born source of b
+    (images 3 and 4) sees the velocities a step late.  4e-6: rounding of the FP32 fields of 2 * 400
+    steps, sqrt(800) * 2^-24 = 1.7e-6, and twice that; stale velocities there give 6.9e-6 and 1.0e-5."""
+    monkeypatch.setitem(globals(), "TOL", 4e-6)
+    test_gradient_matches_oracle(60, 30, 20, [60], [0], 400)
+
+
 def test_born_records_of_traces_on_one_column():
     allnx, allnz, pml, nt = 40, 30, 20, 150
     vp, vs, _ = elastic_model(allnx, allnz, 21)
