@@ -76,7 +76,7 @@ def parse():
                     help="c5: the elastic Born forward pass with two kernels per step instead of one fused launch")
     ap.add_argument("--no-fused-rot", action="store_true",
                     help="rot: k_rot_v + k_rot_p per step instead of the fused rotation step")
-    ap.add_argument("--born-tile", default=None, help="c5: x-chunk width,lanes of the fused Born step (e.g. 64,256)")
+    ap.add_argument("--born-tile", default=None, help="c5: width,lanes given to set_fused_born (checked; the steps run on tiles)")
     ap.add_argument("--no-chunk-plan", action="store_true",
                     help="two steps per launch: fixed-width chunks instead of the balanced chunk plan")
     ap.add_argument("--no-cpu-baseline", action="store_true")
@@ -189,7 +189,8 @@ def roofline(stats):
     return out
 
 
-KERNELS = {2: "fused single kernel per step (x-marching, LDS z taps, unsplit interior)",
+KERNELS = {3: "two time steps per launch on tiles (small batches)",
+           2: "fused single kernel per step (x-marching, LDS z taps, unsplit interior)",
            1: "two fast kernels per step (unsplit interior, split PML strips)",
            0: "reference split layout, two kernels per step"}
 
@@ -234,7 +235,8 @@ def run_forward(a, cfg):
         "data": f"synthetic: seeded layered+faulted elastic model (seed {cfg['seed']}), Gardner density",
         "config": {
             "workload": cfg["desc"], "shots": len(cfg["shots"]), "nt": cfg["nt"], "cell_updates_per_step": cu,
-            "kernels": KERNELS[1 if (a.mode == 2 and chunk == 0) else a.mode] +
+            "kernels": KERNELS[a.mode if a.mode != 2 or chunk != 0 else
+                               3 if stats[0].get("blocked_bytes", 0.0) > 0 else 1] +
                        (", two time steps per launch (temporal blocking)" if tblock == 2 else "") +
                        (" (autotuned)" if a.mode == 2 and not a.tile else ""), "parallelism": "shots batched on one GPU",
             "autotuned_tile": None if chunk is None else {"x_width": None if plan else chunk, "threads": threads,
@@ -639,7 +641,7 @@ def run_c5(a):
                        "born_data_s": round(t_fwd, 2), "solvers": runs, "elastic_unet_training": train,
                        "note": "a step = one CG iteration over all shots; 1e-2 is not reached in this many "
                                "iterations (see resid)"},
-            # the fused forward step of the Born data pass (k_eb_tile, 100 B per padded cell and step)
+            # the forward step of the Born data pass (k_eb_tile, 100 B per padded cell and step)
             "roofline": roofline([stf]) if stf.get("kernel_avg_ms", 0) > 0 else None}
 
 
@@ -688,7 +690,8 @@ def run_compat(a):
             "config": {"workload": f"compat_gradient: 251x101, dx=dz=10 m, pml 20, dt 0.8 ms, {nt} steps, "
                                    f"{len(shots)} shots 10 nodes apart, reference ELSRTM gradient (iteration 1)",
                        "shots": len(shots), "nt": nt, "cell_updates_per_step": cu,
-                       "kernels": "reference split-PML layout, per-cell kernels (ds2d_batch_gradient)",
+                       "kernels": "k_grad_*: two launches per forward step and three per backward step "
+                                  "(ds2d_batch_gradient)",
                        "parallelism": "shots batched on one GPU"}}
 
 
