@@ -385,9 +385,13 @@ __device__ __forceinline__ int wg_chunk(int c, int j) { return j < 8 ? j ^ ((c >
 // Block = (TCO/32) x (TCI/32) x DS waves; wave (cot, cit, dsel) accumulates the
 // 32x32 (co, ci) tile of the taps dx = d - 1 with d = dsel, dsel + DS, ... < 3.
 // Input rows live in a 4-slot LDS ring (row r in slot r & 3, r >= -1) and dy
-// rows in two buffers, so the global loads of rows x + 2 (input) and x + 1
-// (dy) are issued before the MFMAs of row x and land in LDS after them, with
-// one barrier per row.  Each thread moves two pixels x 8 channels per item
+// rows in two buffers; the global loads of rows x + 3 (input) and x + 2 (dy)
+// are issued before the MFMAs of row x, stay in registers for a row, and land
+// in LDS after the MFMAs of row x + 1, with one barrier per row.  Bound by the
+// latency of a row's loads and by first loads and last stores (a round of
+// 64x64 tiles takes 1.1-1.2 us a row and 12-13 more; the products alone 0.5 us
+// a row): with one row in flight and addresses formed per pixel 55.0 us a
+// layer of 8 images of 512x256 on average, 50.0 now (32x32 tiles 59.4, 56.6).  Each thread moves two pixels x 8 channels per item
 // (two 16-byte loads, eight 4-byte LDS writes of a channel's pixel pair).
 template <int TCO, int TCI, int DS>
 __global__ __launch_bounds__(64 * (TCO / 32) * (TCI / 32) * DS) __attribute__((amdgpu_waves_per_eu(4))) void k_wgrad(WgradArgs a) {
@@ -426,49 +430,89 @@ __global__ __launch_bounds__(64 * (TCO / 32) * (TCI / 32) * DS) __attribute__((a
             *reinterpret_cast<unsigned*>(&rows[c + 1][e]) = (v0[k] >> 16) | (v1[k] & 0xFFFF0000u);
         }
     };
-    // input row x: item q = (pair p, g) holds in[n][x][zs + 2p - 1 .. + 1][ci0 + 8g .. + 8], zero outside the image
-    u32x4 ri[NI][2], ro[NO][2];
-    auto in_px = [&](int x, int z, int c) -> u32x4 {
-        if (x < 0 || x >= a.h || z < 0 || z >= a.w) return zero;
-        return c < a.c1 ? ld16(a.x1 + (((long long)n * a.h + x) * a.w + z) * a.c1 + c)
-                        : ld16(a.x2 + (((long long)n * h2 + (x >> a.up)) * w2 + (z >> a.up)) * a.c2 + (c - a.c1));
+    // input row x: item q = (pair p, g) holds in[n][x][zs + 2p - 1 .. + 1][ci0 + 8g .. + 8], zero outside the image;
+    // dy row x: item q = (pair p, g) holds dy[n][x][zs + 2p .. + 1][co0 + 8g .. + 8], zero beyond the image.
+    // What a thread reads of a row is fixed, so its address in row 0 is formed
+    // once.  Every load is issued, from an address inside the image, and what
+    // lies outside is zeroed on its way to LDS: behind a condition the wait for
+    // one row's loads would be a wait for the next row's too.
+    struct InItem {
+        const bf16_t* p;
+        int next;  // from the first pixel to the second, 0 where the second is clamped
+        bool one, z0, z1;
     };
-    auto fetch_in = [&](int x) {
+    struct DyItem {
+        int p, next;
+        bool z0, z1;
+    };
+    InItem ii[NI];
+    DyItem io[NO];
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+        const int q = min(tid + k * NT, QI - 1), p = q / GI, g = q % GI;
+        const int z = zs + 2 * p - 1, c = ci0 + g * 8;
+        ii[k].one = c < a.c1;
+        const int cc = ii[k].one ? a.c1 : a.c2, up = ii[k].one ? 0 : a.up;
+        const int z0 = max(min(z, a.w - 1), 0) >> up, z1 = min(z + 1, a.w - 1) >> up;
+        const bf16_t* base = ii[k].one ? a.x1 + (long long)n * a.h * a.w * a.c1 + c
+                                       : a.x2 + (long long)n * h2 * w2 * a.c2 + (c - a.c1);
+        ii[k].p = base + (long long)z0 * cc;
+        ii[k].next = (z1 - z0) * cc;
+        ii[k].z0 = z >= 0 && z < a.w;
+        ii[k].z1 = z + 1 < a.w;
+    }
+#pragma unroll
+    for (int k = 0; k < NO; ++k) {
+        const int q = min(tid + k * NT, QO - 1), p = q / GO, g = q % GO;
+        const int z = zs + 2 * p;
+        io[k].p = (min(z, a.w - 1) - zs) * a.cout + g * 8;
+        io[k].next = (min(z + 1, a.w - 1) - min(z, a.w - 1)) * a.cout;
+        io[k].z0 = z < a.w;
+        io[k].z1 = z + 1 < a.w;
+    }
+    struct Row {
+        u32x4 in[NI][2], dy[NO][2];
+    };
+    const int xlast = min(xe, a.h - 1);
+    auto fetch_in = [&](Row& r, int x) {
+        const int xc = max(min(x, xlast), 0);
+        const long long o1 = (long long)xc * a.w * a.c1, o2 = (long long)(xc >> a.up) * w2 * a.c2;
 #pragma unroll
         for (int k = 0; k < NI; ++k) {
-            const int q = tid + k * NT, p = q / GI, g = q % GI;
-            const int z = zs + 2 * p - 1, c = ci0 + g * 8;
-            ri[k][0] = ri[k][1] = zero;
-            if (q < QI) {
-                ri[k][0] = in_px(x, z, c);
-                ri[k][1] = in_px(x, z + 1, c);
-            }
+            const bf16_t* src = ii[k].p + (ii[k].one ? o1 : o2);
+            r.in[k][0] = ld16(src);
+            r.in[k][1] = ld16(src + ii[k].next);
         }
     };
-    auto store_in = [&](int slot) {
+    auto fetch_dy = [&](Row& r, int x) {
+        const bf16_t* row = a.dy + (((long long)n * a.h + min(x, xe - 1)) * a.w + zs) * a.cout + co0;
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+            r.dy[k][0] = ld16(row + io[k].p);
+            r.dy[k][1] = ld16(row + io[k].p + io[k].next);
+        }
+    };
+    // Every wave waits for a row before its store, those without an item to
+    // store too: else the wait moves behind the loads that overwrite the row,
+    // and is then one for the other row as well.
+    auto store_in = [&](const Row& r, int x) {
+        const bool row = x >= 0 && x < a.h;
 #pragma unroll
         for (int k = 0; k < NI; ++k) {
+            asm volatile("" ::"v"(r.in[k][0]), "v"(r.in[k][1]));
             const int q = tid + k * NT, p = q / GI, g = q % GI;
-            if (q < QI) put_pair(Bs[slot], g, 2 * p, ri[k][0], ri[k][1]);
+            if (q < QI)
+                put_pair(Bs[(x + 4) & 3], g, 2 * p, row && ii[k].z0 ? r.in[k][0] : zero,
+                         row && ii[k].z1 ? r.in[k][1] : zero);
         }
     };
-    // dy row x: item q = (pair p, g) holds dy[n][x][zs + 2p .. + 1][co0 + 8g .. + 8], zero beyond the image
-    auto fetch_dy = [&](int x) {
+    auto store_dy = [&](const Row& r, int x) {
 #pragma unroll
         for (int k = 0; k < NO; ++k) {
+            asm volatile("" ::"v"(r.dy[k][0]), "v"(r.dy[k][1]));
             const int q = tid + k * NT, p = q / GO, g = q % GO;
-            const int z = zs + 2 * p;
-            const bf16_t* src = a.dy + (((long long)n * a.h + x) * a.w + z) * a.cout + co0 + g * 8;
-            ro[k][0] = ro[k][1] = zero;
-            if (q < QO && z < a.w) ro[k][0] = ld16(src);
-            if (q < QO && z + 1 < a.w) ro[k][1] = ld16(src + a.cout);
-        }
-    };
-    auto store_dy = [&](int buf) {
-#pragma unroll
-        for (int k = 0; k < NO; ++k) {
-            const int q = tid + k * NT, p = q / GO, g = q % GO;
-            if (q < QO) put_pair(As[buf], g, 2 * p, ro[k][0], ro[k][1]);
+            if (q < QO)
+                put_pair(As[x & 1], g, 2 * p, io[k].z0 ? r.dy[k][0] : zero, io[k].z1 ? r.dy[k][1] : zero);
         }
     };
 
@@ -484,19 +528,23 @@ __global__ __launch_bounds__(64 * (TCO / 32) * (TCI / 32) * DS) __attribute__((a
     const int bco = tid % TCO, bpart = tid / TCO;
     float bacc = 0.f;
 
-    for (int r = xa - 1; r <= xa + 1; ++r) {
-        fetch_in(r);
-        store_in((r + 4) & 3);
-    }
-    fetch_dy(xa);
-    store_dy(xa & 1);
+    Row ra, rb;
+    fetch_in(rb, xa - 1);
+    fetch_dy(rb, xa);
+    fetch_in(ra, xa);
+    store_in(rb, xa - 1);
+    store_dy(rb, xa);
+    fetch_in(rb, xa + 1);
+    store_in(ra, xa);
+    fetch_in(ra, xa + 2);
+    fetch_dy(ra, xa + 1);
+    store_in(rb, xa + 1);
     __syncthreads();
-    for (int x = xa; x < xe; ++x) {
-        const bool more = x + 1 < xe;
-        if (more) {
-            fetch_in(x + 2);
-            fetch_dy(x + 1);
-        }
+    // row x: cur holds (or waits for) input row x + 2 and dy row x + 1, next takes the ones after
+    auto row_step = [&](int x, const Row& cur, Row& next) {
+        fetch_in(next, x + 3);
+        fetch_dy(next, x + 2);
+#pragma unroll 1
         for (int s = 0; s < nks; ++s) {
             const int base = 16 * s + 8 * kh;
             const int ca = cot * 32 + li, cb = cit * 32 + li, jb = base >> 3;
@@ -528,12 +576,16 @@ __global__ __launch_bounds__(64 * (TCO / 32) * (TCI / 32) * DS) __attribute__((a
                 }
             }
         }
-        if (more) {
-            store_in((x + 2) & 3);
-            store_dy((x + 1) & 1);
-        }
+        store_in(cur, x + 2);
+        store_dy(cur, x + 1);
         __syncthreads();
+    };
+    int x = xa;
+    for (; x + 1 < xe; x += 2) {
+        row_step(x, ra, rb);
+        row_step(x + 1, rb, ra);
     }
+    if (x < xe) row_step(x, ra, rb);
     const long long rec = 9LL * a.cout * cin;
     float* out = a.part + (long long)chunk * (rec + (a.bias ? a.cout : 0));
     if (do_bias) {  // the ring is free after the last barrier

@@ -101,6 +101,13 @@ def test_conv_weight_gradient_matches_oracle(c1, c2, up, cout, h, w):
     assert e <= 1e-5
 
 
+@pytest.mark.parametrize("c1,c2,up,cout,h,w", [(128, 256, 1, 128, 64, 64), (64, 0, 0, 64, 139, 260), (32, 64, 0, 32, 45, 70)])
+def test_conv_weight_gradient_of_many_rows_a_workgroup(c1, c2, up, cout, h, w):
+    """Odd and even numbers of rows, rounds of workgroups that just fit.  FP32 sums of at most 9 * 64 products and
+    128 partials: sqrt(576 + 128) * 2^-24 = 1.6e-6, held to the 1e-5 of the other shapes."""
+    test_conv_weight_gradient_matches_oracle(c1, c2, up, cout, h, w)
+
+
 @pytest.mark.parametrize("levels,base,n,h,w", [(4, 32, 2, 32, 16), (3, 32, 1, 24, 40), (2, 64, 2, 16, 16)])
 def test_unet_loss_and_gradient_match_oracle(levels, base, n, h, w):
     from ds2d_amd.lib import Unet
