@@ -618,10 +618,23 @@ void wgrad_plan(int n, int h, int w, int cout, int cin, long long max_part, int*
     // workgroups for one full round of the GPU: 256 CUs x the workgroups of this tile shape that fit on a CU
     // (64x64: 12 waves, one per CU; 64x32 and 32x64: 6 waves, two; 32x32: 3 waves, five)
     const long long target = tco == 64 && tci == 64 ? 256 : tco == 32 && tci == 32 ? 1280 : 512;
-    const long long want = std::max<long long>(1, (target + tiles - 1) / tiles);
-    long long per = std::max<long long>(1, (want + (long long)n * nseg - 1) / ((long long)n * nseg));
-    int r = (int)std::max<long long>(1, (h + per - 1) / per);
-    r = std::max(r, std::min(4, h));
+    // Chunks of rows per image and segment: as many as fit into k rounds, k <= 4.  A round lasts its rows and about 11
+    // more (first loads, partial sums; 1.1 and 12 us of a 64x64 tile), so an overfull one is dear: 288 workgroups
+    // of 43 rows took 117 us where 240 of 52 take 69.
+    const long long base = (long long)n * nseg;
+    int r = h;
+    long long best = 0;
+    for (int k = 1; k <= 4; ++k) {
+        const long long per = std::min<long long>(h, k * target / (tiles * base));
+        if (per < 1) continue;
+        const int rows_k = std::max((int)((h + per - 1) / per), std::min(4, h));
+        const long long wgs = tiles * base * ((h + rows_k - 1) / rows_k);
+        const long long cost = (wgs + target - 1) / target * (rows_k + 11);
+        if (best == 0 || cost < best) {
+            best = cost;
+            r = rows_k;
+        }
+    }
     const long long per_chunk = 9LL * cout * cin + cout;
     for (;;) {
         const long long nc = (long long)n * nseg * ((h + r - 1) / r);
