@@ -391,7 +391,8 @@ __device__ __forceinline__ int wg_chunk(int c, int j) { return j < 8 ? j ^ ((c >
 // latency of a row's loads and by first loads and last stores (a round of
 // 64x64 tiles takes 1.1-1.2 us a row and 12-13 more; the products alone 0.5 us
 // a row): with one row in flight and addresses formed per pixel 55.0 us a
-// layer of 8 images of 512x256 on average, 50.0 now (32x32 tiles 59.4, 56.6).  Each thread moves two pixels x 8 channels per item
+// layer of 8 images of 512x256 on average, 50.0 so (32x32 tiles 59.4, 56.6),
+// and 42.3 (52.1) in rounds that fit (wgrad_plan).  Each thread moves two pixels x 8 channels per item
 // (two 16-byte loads, eight 4-byte LDS writes of a channel's pixel pair).
 template <int TCO, int TCI, int DS>
 __global__ __launch_bounds__(64 * (TCO / 32) * (TCI / 32) * DS) __attribute__((amdgpu_waves_per_eu(4))) void k_wgrad(WgradArgs a) {
