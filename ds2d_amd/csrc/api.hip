@@ -142,6 +142,7 @@ struct Batch {
     long long total_cells = 0, total_rec = 0, total_win = 0, total_edge = 0, total_rmap = 0, total_hist = 0;
     int total_traces = 0;
     bool any_pml = false;
+    std::vector<int> rnext;  // trace -> the one before it on its column (-1: none); empty when no column has several
 };
 
 // The caller's record buffers, while the device still computes.
@@ -157,6 +158,8 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     B.slots.resize(nshots);
     long long off = 0, roff = 0, woff = 0, eoff = 0, moff = 0;
     int rixo = 0, max_nxp = 0, max_ntr = 0;
+    bool repeated = false;
+    std::vector<int> last;  // last trace of each column of a window
     for (int s = 0; s < nshots; ++s) {
         const ds2d_shot& q = shots[s];
         if (q.nx <= 0 || q.ngx_min < 0 || q.ngx_min + q.nx > g.allnx)
@@ -204,7 +207,14 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
         B.total_hist += (long long)g.nt * q.nx * g.allnz;
         B.tbase.push_back(B.total_traces);
         B.total_traces += q.ntr;
-        for (int r = 0; r < q.ntr; ++r) B.rix.push_back(q.rec_ix[r]);
+        last.assign(nxp, -1);
+        for (int r = 0; r < q.ntr; ++r) {
+            int& t = last[q.rec_ix[r]];
+            repeated = repeated || t >= 0;
+            B.rix.push_back(q.rec_ix[r]);
+            B.rnext.push_back(t);
+            t = r;
+        }
         rixo += q.ntr;
         max_nxp = std::max(max_nxp, nxp);
         max_ntr = std::max(max_ntr, q.ntr);
@@ -228,6 +238,15 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     BatchShape& sh = B.shape;
     sh.slots = d_slots;
     sh.rix = d_rix;
+    sh.rnext = nullptr;
+    if (repeated) {
+        int* d_next;
+        if ((rc = h->fbuf("rnext", B.rnext.size(), &d_next))) return rc;
+        HIP_TRY(hipMemcpyAsync(d_next, B.rnext.data(), B.rnext.size() * sizeof(int), hipMemcpyHostToDevice, h->st));
+        sh.rnext = d_next;
+    } else {
+        B.rnext.clear();
+    }
     sh.nslots = nshots;
     sh.max_nxp = max_nxp;
     sh.nzp = nzp;
@@ -238,6 +257,16 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     sh.dt = g.dt;
     sh.dx = g.dx;
     sh.dz = g.dz;
+    return 0;
+}
+
+// Every window's columns -> the last trace that records each (-1: none).
+int column_traces(ds2d_ctx* h, const Batch& B, const char* name, int** map) {
+    const size_t n = std::max<long long>(B.total_rmap, 1);
+    int rc;
+    if ((rc = h->fbuf(name, n, map))) return rc;
+    HIP_TRY(hipMemsetAsync(*map, 0xff, n * sizeof(int), h->st));
+    launch_fast_rmap(h->st, B.shape, *map);
     return 0;
 }
 
@@ -552,18 +581,8 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     float* win;
     if ((rc = h->fbuf("win7", (size_t)W * 7, &win))) return rc;
     HIP_TRY(hipMemsetAsync(win, 0, (size_t)W * 7 * 4, st));
-    // column -> a trace that records it, trace -> the next one on its column (a column may have several)
-    std::vector<int> map(std::max<long long>(B.total_rmap, 1), -1), next(std::max<size_t>(B.rix.size(), 1), -1);
-    for (const SlotDesc& S : B.slots)
-        for (int r = 0; r < S.ntr; ++r) {
-            int& head = map[S.rmap_off + B.rix[S.rix_off + r]];
-            next[S.rix_off + r] = head;
-            head = r;
-        }
-    int *d_map, *d_next;
-    if ((rc = h->fbuf("gmap", map.size(), &d_map)) || (rc = h->fbuf("gnext", next.size(), &d_next))) return rc;
-    HIP_TRY(hipMemcpyAsync(d_map, map.data(), map.size() * 4, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(d_next, next.data(), next.size() * 4, hipMemcpyHostToDevice, st));
+    int* d_map;
+    if ((rc = column_traces(h, B, "gmap", &d_map))) return rc;
     const int nt = h->g.nt;
     GradArgs ga{};
     ga.n = n;
@@ -583,7 +602,7 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     ga.nt = nt;
     ga.wav = h->d_wav;
     ga.rmap = d_map;
-    ga.rnext = d_next;
+    ga.rnext = sh.rnext;
     ga.rs_z = rs_z;
     ga.rs_x = rs_x;
     ga.rs2_z = rs2_z;
@@ -808,6 +827,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
     launch_setup(st, sh, setup_args(h, false), m);
     HIP_TRY(hipMemsetAsync(f.vx, 0, (size_t)n * 15 * 4, st));
     double bytes_v = 0, bytes_s = 0, blocked = 0;
+    int* rmap = nullptr;  // of the kernels that record one trace a column
     // cells of the update region that carry split PML memory (PML windows only)
     double pml_cells = 0;
     for (auto& S : B.slots)
@@ -852,11 +872,8 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
     } else if (mode == 2 && (tile || !h->fwd_two) && n <= FUSED_MAX_CELLS) {
         // fused kernels, ping-pong state
         float* par;
-        int* rmap;
-        if ((rc = h->fbuf("fpar", (size_t)n * 3, &par)) || (rc = h->fbuf("rmap", B.total_rmap, &rmap))) return rc;
+        if ((rc = h->fbuf("fpar", (size_t)n * 3, &par)) || (rc = column_traces(h, B, "rmap", &rmap))) return rc;
         launch_fast_params(st, m.rho, m.lam, m.mu, par, par + n, par + 2 * n, n, h->g.dt);
-        HIP_TRY(hipMemsetAsync(rmap, 0xff, B.total_rmap * 4, st));
-        launch_fast_rmap(st, sh, rmap);
         EField g2;
         if ((rc = alloc_efield(h, "b", n, g2, true))) return rc;
         std::vector<ChunkDesc> ch;
@@ -1007,11 +1024,8 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         }
     } else {
         float* par;
-        int* rmap;
-        if ((rc = h->fbuf("fpar", (size_t)n * 3, &par)) || (rc = h->fbuf("rmap", B.total_rmap, &rmap))) return rc;
+        if ((rc = h->fbuf("fpar", (size_t)n * 3, &par)) || (rc = column_traces(h, B, "rmap", &rmap))) return rc;
         launch_fast_params(st, m.rho, m.lam, m.mu, par, par + n, par + 2 * n, n, h->g.dt);
-        HIP_TRY(hipMemsetAsync(rmap, 0xff, B.total_rmap * 4, st));
-        launch_fast_rmap(st, sh, rmap);
         FastArgs a{};
         a.vx = f.vx; a.vz = f.vz; a.txx = f.txx; a.tzz = f.tzz; a.txz = f.txz;
         a.vx_x = f.vx_x; a.vx_z = f.vx_z; a.vz_x = f.vz_x; a.vz_z = f.vz_z;
@@ -1037,6 +1051,7 @@ static int batch_forward_n(ds2d_t* h, int nshots, const ds2d_shot* shots, float*
         bytes_v = (double)B.total_cells * 8 * 4 + pml_cells * 10 * 4;
         bytes_s = (double)B.total_cells * 10 * 4 + pml_cells * 14 * 4;
     }
+    if (rmap) launch_share_records(st, sh, rmap, rz, rx);
     prepare_records(B, rec_z, rec_x);
     if ((rc = stats_end(h, stats, cu, launches, 0))) return rc;
     {
@@ -1375,9 +1390,7 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
     w.store = h->g.bg_mode == 1 || (h->g.bg_mode == 0 && hist_gb <= budget);
     if (w.store && (rc = h->fbuf("hist", (size_t)B.total_hist, &w.hist))) return rc;
     // receiver map (column -> trace) of every slot, for the in-kernel recorder and injection
-    if ((rc = h->fbuf("armap", std::max<long long>(B.total_rmap, 1), &w.rmap))) return rc;
-    HIP_TRY(hipMemsetAsync(w.rmap, 0xff, B.total_rmap * 4, h->st));
-    launch_fast_rmap(h->st, B.shape, w.rmap);
+    if ((rc = column_traces(h, B, "armap", &w.rmap))) return rc;
     // fused steps: store mode, 32-bit byte offsets within a window's doubles (from one window to the largest
     // batches faster than the per-cell kernels: 5 against 8 us a step on 331x181, 26 against 92 on 3.2 M cells)
     w.fused = w.store && n <= FUSED_MAX_CELLS && (long long)B.shape.max_nxp * B.shape.nzp < (1LL << 29) &&
@@ -1461,6 +1474,7 @@ void acou_fwd(ds2d_ctx* h, const Batch& B, AcouWS& w, bool do_bg, bool do_born, 
             for (const std::pair<int, int>& gc : w.groups)
                 for (int it = 0; it < h->g.nt; ++it)
                     launch_acou_born_tile(st, B.shape, (it & 1) ? odd : even, w.tiles + gc.first, gc.second, w.rmap, it);
+            launch_share_records(st, B.shape, w.rmap, w.rec2, nullptr);
         }
         return;
     }
@@ -1473,28 +1487,31 @@ void acou_fwd(ds2d_ctx* h, const Batch& B, AcouWS& w, bool do_bg, bool do_born, 
             launch_acou_p(st, sh, w.bg, w.bn, w.m, w.hist, rec_bg ? w.rec : nullptr, do_born ? w.rec2 : nullptr, it,
                           do_bg, do_born, hmode, w.rmap);
         }
+    launch_share_records(st, B.shape, w.rmap, do_born ? w.rec2 : nullptr, rec_bg ? w.rec : nullptr);
 }
 
-// Backward pass (residual in w.rec2): the gradient is accumulated in
+// Backward pass (residual in w.rec2, whose traces on one column are summed
+// into the last of them here): the gradient is accumulated in
 // w.grad_pad from the stored increment, or from the background rebuilt by
 // reversal from the state acou_fwd left at t = nt.
 void acou_bwd(ds2d_ctx* h, const Batch& B, AcouWS& w) {
     hipStream_t st = h->st;
     (void)hipMemsetAsync(w.lm.vx, 0, (size_t)w.n * 3 * 4, st);
     (void)hipMemsetAsync(w.grad_pad, 0, (size_t)w.n * 4, st);
+    launch_fold_residuals(st, B.shape, w.rmap, w.rec2, nullptr);
     if (w.fused) {
         (void)hipMemsetAsync(w.lm2.vx, 0, (size_t)w.n * 3 * 4, st);
         AcouFusedArgs even = acou_fused_args(h, w, w.lm, w.lm2), odd = acou_fused_args(h, w, w.lm2, w.lm);
         even.grad = odd.grad = w.grad_pad;
         even.res = odd.res = w.rec2;
-        launch_acou_inj(st, B.shape, w.lm.p, w.rec2, h->g.nt - 1);
+        launch_acou_inj(st, B.shape, w.lm.p, w.rec2, w.rmap, h->g.nt - 1);
         for (const std::pair<int, int>& gc : w.groups)
             for (int it = h->g.nt - 1, k = 0; it >= 0; --it, ++k)
                 launch_acou_adj_tile(st, B.shape, (k & 1) ? odd : even, w.tiles + gc.first, gc.second, w.rmap, it);
         return;
     }
     for (const BatchShape& sh : launch_groups(h, B)) {
-        launch_acou_inj(st, sh, w.lm.p, w.rec2, h->g.nt - 1);
+        launch_acou_inj(st, sh, w.lm.p, w.rec2, w.rmap, h->g.nt - 1);
         for (int it = h->g.nt - 1; it >= 0; --it) {
             launch_acou_adj_p(st, sh, w.bg, w.lm, w.m, w.grad_pad, w.store ? w.hist : nullptr, it);
             launch_acou_adj_v(st, sh, w.bg, w.lm, w.m, h->d_wav, it, w.store ? 0 : 1, w.rmap, w.rec2);
@@ -1806,9 +1823,7 @@ int eb_prepare(ds2d_ctx* h, const Batch& B, const float* pp_dev, const float* ps
     const double budget = h->g.hbm_budget_gb > 0 ? h->g.hbm_budget_gb : 64.0;
     w.store = want_store && (h->g.bg_mode == 1 || (h->g.bg_mode == 0 && hist_gb <= budget));
     if (w.store && (rc = h->fbuf("ehist", (size_t)w.H * 3, &w.hist))) return rc;
-    if ((rc = h->fbuf("ebrmap", std::max<long long>(B.total_rmap, 1), &w.rmap))) return rc;
-    HIP_TRY(hipMemsetAsync(w.rmap, 0xff, B.total_rmap * 4, h->st));
-    launch_fast_rmap(h->st, B.shape, w.rmap);
+    if ((rc = column_traces(h, B, "ebrmap", &w.rmap))) return rc;
     // fused steps (32-bit cell indices within a field); when the second state does
     // not fit, the per-cell kernels (one state) run instead
     w.alt = nullptr;
@@ -1861,6 +1876,7 @@ void eb_fwd(ds2d_ctx* h, const Batch& B, EbWS& w, bool do_bg) {
     const int hmode = do_bg ? (w.store ? 1 : 0) : 2;
     if (w.alt) {
         eb_tile_steps(h, B, w, do_bg, true, hmode);
+        launch_share_records(st, B.shape, w.rmap, w.rec, w.rec + w.R);
         return;
     }
     for (const BatchShape& sh : launch_groups(h, B))
@@ -1868,6 +1884,7 @@ void eb_fwd(ds2d_ctx* h, const Batch& B, EbWS& w, bool do_bg) {
             launch_eb_v(st, sh, w.bg, w.bn, w.m.rho, h->wav[it], 1.f, do_bg, 1);
             launch_eb_s(st, sh, w.bg, w.bn, w.m, w.hist, w.H, it, 1.f, do_bg, 1, hmode, w.rmap, w.rec, w.rec + w.R);
         }
+    launch_share_records(st, B.shape, w.rmap, w.rec, w.rec + w.R);
 }
 
 // Background only (fills the strain history), from rest to t = nt.
@@ -1886,12 +1903,14 @@ void eb_bg(ds2d_ctx* h, const Batch& B, EbWS& w) {
         }
 }
 
-// Backward pass (residual in w.res): gradients in w.gpp / w.gps.  Without the
+// Backward pass (residual in w.res, whose traces on one column are summed into
+// the last of them here): gradients in w.gpp / w.gps.  Without the
 // history the background, left at t = nt by the forward pass, is reversed.
 void eb_bwd(ds2d_ctx* h, const Batch& B, EbWS& w) {
     hipStream_t st = h->st;
     (void)hipMemsetAsync(w.lm.vx, 0, (size_t)w.n * 12 * 4, st);  // lm + gpp + gps + adjoint products
     if (w.alt) (void)hipMemsetAsync(w.alt, 0, (size_t)w.n * 10 * 4, st);
+    launch_fold_residuals(st, B.shape, w.rmap, w.res, w.res + w.R);
     const int nt = h->g.nt, undo = w.store ? 0 : 1;
     int g = 0;
     for (const BatchShape& sh : launch_groups(h, B)) {
@@ -2510,11 +2529,9 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
     if (fa) {
         // one fused launch per step on tiles, state ping-ponged between two sets of 6 fields
         int* rmap;
-        if ((rc = h->fbuf("rmap", B.total_rmap, &rmap))) return rc;
+        if ((rc = column_traces(h, B, "rmap", &rmap))) return rc;
         HIP_TRY(hipMemsetAsync(fa, 0, (size_t)n * 12 * 4, st));
-        HIP_TRY(hipMemsetAsync(rmap, 0xff, B.total_rmap * 4, st));
         HIP_TRY(hipMemsetAsync(rs, 0, R * 2 * 4, st));
-        launch_fast_rmap(st, sh, rmap);
         const StepTiles tp = plan_rot_tiles(widths(B), sh.nzp);
         StepTile* tiles;
         std::vector<std::pair<int, int>> gr;
@@ -2534,6 +2551,7 @@ int ds2d_rot_forward(ds2d_t* h, int nshots, const ds2d_shot* shots, float* rec_z
             std::swap(a, b);
         }
         stats_loop_end(h);
+        launch_share_records(st, sh, rmap, rs, rs + R);
         prepare_records(B, rec_z, rec_x);
         if ((rc = stats_end(h, stats, padded_cells(B) * nt, nt, 0))) return rc;
         double kf, unused;

@@ -11,6 +11,7 @@ namespace ds2d {
 struct BatchShape {
     const SlotDesc* slots;  // device
     const int* rix;         // device, receiver columns (padded)
+    const int* rnext;       // device, trace -> the one before it on its column (-1: none); null: no column has several
     int nslots, max_nxp, nzp, nz, max_ntr, nt;
     long long total_cells;  // sum of nxp*nzp
     float dt, dx, dz;
@@ -40,7 +41,7 @@ struct GradArgs {
     double kx64, kz64, ix64, iz64;
     int nt;
     const float* wav;
-    const int *rmap, *rnext;          // column -> a trace, trace -> the next on its column (-1: none)
+    const int *rmap, *rnext;          // column -> its last trace, trace -> the one before on its column (-1: none; null: none at all)
     float *rs_z, *rs_x, *rs2_z, *rs2_x;
     float *g, *wk, *pk, *wb, *cs;     // bg strains, products of bk (two sets) and bb, 3 arrays of n each; 2 mu (-dms)
     float* w7;                        // window images pp, ps, illum, b_pp, b_ps, b2_pp, b2_ps
@@ -111,7 +112,7 @@ void launch_acou_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField
 // Backward step it: (injection of res[it] already in lam.p) adj_p, then adj_v,
 // which also injects res[it - 1] for the next step.  Step nt - 1 is injected
 // by launch_acou_inj.
-void launch_acou_inj(hipStream_t st, const BatchShape& b, float* lp, const float* res, int it);
+void launch_acou_inj(hipStream_t st, const BatchShape& b, float* lp, const float* res, const int* rmap, int it);
 // hist != null: gradient from the stored increment, background untouched
 void launch_acou_adj_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField lam, AcouMed m, float* grad,
                        const float* hist, int it);
@@ -173,7 +174,14 @@ void launch_fast_v(hipStream_t st, const BatchShape& b, const FastArgs& a, const
 void launch_fast_s(hipStream_t st, const BatchShape& b, const FastArgs& a);
 void launch_fast_params(hipStream_t st, const float* rho, const float* lam, const float* mu, float* bx, float* ldt,
                         float* mdt, long long n, float dt);
+// Column -> the last trace that records it (rmap holds -1 before).
 void launch_fast_rmap(hipStream_t st, const BatchShape& b, int* rmap);
+// The step kernels record and inject one trace a column, rmap's.  Records are
+// handed on to the column's other traces after the loop, and residuals summed
+// into that trace before it (the others are cleared); z or x may be null, and
+// nothing is launched when no column has several.
+void launch_share_records(hipStream_t st, const BatchShape& b, const int* rmap, float* z, float* x);
+void launch_fold_residuals(hipStream_t st, const BatchShape& b, const int* rmap, float* z, float* x);
 
 // --- plain-L2 elastic Born pair (kernels_eborn.hip) --------------------------
 // Unsplit elastic wavefield (random boundary, no damping).

@@ -186,12 +186,13 @@ __global__ __launch_bounds__(256) void k_acou_adj_v(AcouFieldD bg, AcouField lm,
     }
 }
 
-// lp[rec] += res[r][it] (first backward step; later steps inject inside k_acou_adj_v).
+// lp[rec] += res[r][it] (first backward step; later steps inject inside k_acou_adj_v),
+// one trace a column: the others hold nothing (launch_fold_residuals).
 __global__ void k_acou_inj(float* lp, const float* __restrict__ res, const int* __restrict__ rix,
-                           const SlotDesc* __restrict__ slots, int nt, int it) {
+                           const int* __restrict__ rmap, const SlotDesc* __restrict__ slots, int nt, int it) {
     const SlotDesc S = slots[blockIdx.y];
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= S.ntr) return;
+    if (r >= S.ntr || rmap[S.rmap_off + rix[S.rix_off + r]] != r) return;
     const size_t c = (size_t)S.off + (size_t)rix[S.rix_off + r] * S.nzp + S.igz;
     lp[c] += res[(size_t)S.rec_off + (size_t)r * nt + it];
 }
@@ -212,9 +213,9 @@ void launch_acou_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField
     hipLaunchKernelGGL(k_acou_p, cgrid(b), dim3(BZ, BX), 0, st, bg, born, m, hist, b.slots, b.dt / b.dx, b.dt / b.dz,
                        dxd(b), dzd(b), it, do_bg, do_born, hist_mode, rmap, rec_bg, rec_born, b.nt);
 }
-void launch_acou_inj(hipStream_t st, const BatchShape& b, float* lp, const float* res, int it) {
+void launch_acou_inj(hipStream_t st, const BatchShape& b, float* lp, const float* res, const int* rmap, int it) {
     hipLaunchKernelGGL(k_acou_inj, dim3(ceil_div(b.max_ntr, 64), b.nslots), dim3(64), 0, st, lp, res, b.rix,
-                       b.slots, b.nt, it);
+                       rmap, b.slots, b.nt, it);
 }
 void launch_acou_adj_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField lam, AcouMed m, float* grad,
                        const float* hist, int it) {

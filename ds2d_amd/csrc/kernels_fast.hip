@@ -130,12 +130,40 @@ __global__ void k_fast_params(const float* __restrict__ rho, const float* __rest
     mdt[i] = mu[i] * dt;
 }
 
-// Receiver map: rmap[pad0 + ix] = trace index recording column ix, else -1.
+// Receiver map: rmap[pad0 + ix] = last trace recording column ix, else -1.
 __global__ void k_fast_rmap(int* rmap, const int* __restrict__ rix, const SlotDesc* __restrict__ slots) {
     const SlotDesc S = slots[blockIdx.y];
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= S.ntr) return;
-    rmap[S.rmap_off + rix[S.rix_off + r]] = r;
+    atomicMax(&rmap[S.rmap_off + rix[S.rix_off + r]], r);
+}
+
+// Rows of the traces that share a column with rmap's: copies of its row.
+__global__ __launch_bounds__(64) void k_share_records(float* rec, const int* __restrict__ rmap,
+                                                      const int* __restrict__ rix, const SlotDesc* __restrict__ slots,
+                                                      int nt) {
+    const SlotDesc S = slots[blockIdx.z];
+    const int r = blockIdx.x, it = blockIdx.y * 64 + threadIdx.x;
+    if (r >= S.ntr || it >= nt) return;
+    const int from = rmap[S.rmap_off + rix[S.rix_off + r]];
+    float* row = rec + S.rec_off + it;
+    if (from != r) row[(size_t)r * nt] = row[(size_t)from * nt];
+}
+
+// The row of rmap's trace: the sum over the traces of its column, whose own rows are cleared.
+__global__ __launch_bounds__(64) void k_fold_residuals(float* res, const int* __restrict__ rmap,
+                                                       const int* __restrict__ rnext, const int* __restrict__ rix,
+                                                       const SlotDesc* __restrict__ slots, int nt) {
+    const SlotDesc S = slots[blockIdx.z];
+    const int r = blockIdx.x, it = blockIdx.y * 64 + threadIdx.x;
+    if (r >= S.ntr || it >= nt || rmap[S.rmap_off + rix[S.rix_off + r]] != r) return;
+    float* row = res + S.rec_off + it;
+    float sum = row[(size_t)r * nt];
+    for (int q = rnext[S.rix_off + r]; q >= 0; q = rnext[S.rix_off + q]) {
+        sum += row[(size_t)q * nt];
+        row[(size_t)q * nt] = 0.f;
+    }
+    row[(size_t)r * nt] = sum;
 }
 
 static dim3 fgrid(const BatchShape& b) { return dim3(ceil_div(b.nzp, BZ), ceil_div(b.max_nxp, BX), b.nslots); }
@@ -153,6 +181,19 @@ void launch_fast_params(hipStream_t st, const float* rho, const float* lam, cons
 }
 void launch_fast_rmap(hipStream_t st, const BatchShape& b, int* rmap) {
     hipLaunchKernelGGL(k_fast_rmap, dim3(ceil_div(b.max_ntr, 64), b.nslots), dim3(64), 0, st, rmap, b.rix, b.slots);
+}
+void launch_share_records(hipStream_t st, const BatchShape& b, const int* rmap, float* z, float* x) {
+    if (!b.rnext) return;
+    const dim3 grid(b.max_ntr, ceil_div(b.nt, 64), b.nslots);
+    for (float* rec : {z, x})
+        if (rec) hipLaunchKernelGGL(k_share_records, grid, dim3(64), 0, st, rec, rmap, b.rix, b.slots, b.nt);
+}
+void launch_fold_residuals(hipStream_t st, const BatchShape& b, const int* rmap, float* z, float* x) {
+    if (!b.rnext) return;
+    const dim3 grid(b.max_ntr, ceil_div(b.nt, 64), b.nslots);
+    for (float* res : {z, x})
+        if (res)
+            hipLaunchKernelGGL(k_fold_residuals, grid, dim3(64), 0, st, res, rmap, b.rnext, b.rix, b.slots, b.nt);
 }
 
 }  // namespace ds2d

@@ -410,7 +410,7 @@ __device__ __forceinline__ void stress_cell(const GradTile& g, const EFieldT<T>&
 template <typename T>
 __device__ __forceinline__ void record_cell(const SlotDesc& S, const int* rmap, const int* rnext, int ix, int nt,
                                             int it, T vz, T vx, float* rz, float* rx) {
-    for (int r = rmap[S.rmap_off + ix]; r >= 0; r = rnext[S.rix_off + r]) {
+    for (int r = rmap[S.rmap_off + ix]; r >= 0; r = rnext ? rnext[S.rix_off + r] : -1) {
         const size_t o = (size_t)S.rec_off + (size_t)r * nt + it;
         rz[o] = (float)vz;
         rx[o] = (float)vx;
@@ -753,7 +753,8 @@ __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* 
         hx = g.halo(F.bk.txz);
     }
     if (!BORN && g.upd() && g.z == g.S.igz) {
-        for (int r = a.rmap[g.S.rmap_off + g.col()]; r >= 0; r = a.rnext[g.S.rix_off + r]) {
+        for (int r = a.rmap[g.S.rmap_off + g.col()]; r >= 0;
+             r = a.rnext ? a.rnext[g.S.rix_off + r] : -1) {
             held = true;
             if (k > 0) {
                 const size_t o = (size_t)g.S.rec_off + (size_t)r * a.nt + (k - 1);
@@ -968,7 +969,7 @@ __global__ __launch_bounds__(256) void k_grad_bwd_0(GradFields<TB> F, Med m, Gra
         F.lvz[c] = F.bg.vz[c];
     }
     if (iz == S.igz)
-        for (int r = a.rmap[S.rmap_off + ix]; r >= 0; r = a.rnext[S.rix_off + r]) {
+        for (int r = a.rmap[S.rmap_off + ix]; r >= 0; r = a.rnext ? a.rnext[S.rix_off + r] : -1) {
             const size_t o = (size_t)S.rec_off + (size_t)r * a.nt + (a.nt - 1);
             F.bk.vz[c] += a.rs_z[o];
             F.bk.vx[c] += a.rs_x[o];
