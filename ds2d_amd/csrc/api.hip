@@ -611,10 +611,9 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
     F.lvx = bg.vx;
     F.lvz = bg.vz;
     if (full) {
-        // strains of bg, two sets of products of bk, one of bb, the Born adjoint's modulus
-        float* prod;
-        if ((rc = h->fbuf("gradprod", (size_t)n * 13, &prod))) return rc;
-        HIP_TRY(hipMemsetAsync(prod, 0, (size_t)n * 13 * 4, st));
+        // strains of bg, two sets of products of bk, one of bb, the Born adjoint's modulus: 13 arrays of the
+        // backward loop in the 15 of b2, which only the forward loop has
+        float* prod = b2.vx;
         ga.g = prod;
         ga.wk = prod + 3 * n;
         ga.pk = prod + 6 * n;
@@ -675,6 +674,7 @@ int batch_gradient_impl(ds2d_t* h, int nshots, const ds2d_shot* shots, const flo
             }
         }
     }
+    HIP_TRY(hipMemsetAsync(ga.g, 0, (size_t)n * 13 * 4, st));
     launch_grad_backward<TB>(st, sh, F, m, ga);
     const long long A = (long long)h->g.allnx * h->g.allnz;
     launch_slot_nonfinite(st, sh, win, W, 7, 1, d_bad);
