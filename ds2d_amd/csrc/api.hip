@@ -1307,7 +1307,7 @@ namespace {
 
 struct AcouWS {
     AcouFieldD bg;              // FP64 background
-    double* bg2 = nullptr;      // its second state in the fused background pass (3 n doubles)
+    double* bg2 = nullptr;      // its second state in the fused background pass: 3 n doubles, in bn2 and lm2
     AcouField bn, lm;
     AcouField bn2, lm2;         // second state of the fused (ping-pong) Born / adjoint steps
     AcouMed m;
@@ -1375,6 +1375,7 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
     float *bu = base + 7 * n, *kk = base + 8 * n, *refl = base + 9 * n;
     w.bn2 = AcouField{base + 10 * n, base + 11 * n, base + 12 * n};
     w.lm2 = AcouField{base + 13 * n, base + 14 * n, base + 15 * n};
+    w.bg2 = (double*)w.bn2.vx;
     Med m;
     if ((rc = alloc_med(h, n, m))) return rc;
     SetupArgs a = setup_args(h, false);
@@ -1395,10 +1396,6 @@ int acou_prepare(ds2d_ctx* h, const Batch& B, const float* refl_glob_dev, AcouWS
     // batches faster than the per-cell kernels: 5 against 8 us a step on 331x181, 26 against 92 on 3.2 M cells)
     w.fused = w.store && n <= FUSED_MAX_CELLS && (long long)B.shape.max_nxp * B.shape.nzp < (1LL << 29) &&
               h->acou_fused != 0;
-    if (w.fused && h->fbuf("acoubg2", (size_t)n * 3, &w.bg2)) {  // no room for the second background state
-        w.fused = false;
-        (void)hipGetLastError();
-    }
     return w.fused ? step_tiles(h, B, "atiles", ACOU_TILE_COLS, group_size(h, B), &w.tiles, w.groups) : 0;
 }
 AcouFusedArgs acou_fused_args(ds2d_ctx* h, AcouWS& w, const AcouField& A, const AcouField& Bf) {
@@ -1455,8 +1452,8 @@ std::vector<BatchShape> launch_groups(const ds2d_ctx* h, const Batch& B) {
 void acou_fwd(ds2d_ctx* h, const Batch& B, AcouWS& w, bool do_bg, bool do_born, bool rec_bg) {
     hipStream_t st = h->st;
     if (w.fused && w.store && !rec_bg) {
-        // the background pass fills the history, the Born pass reads it: one fused launch per step each;
-        // chunk lists hold absolute slot indices: launch with the whole slot table
+        // the background pass fills the history, the Born pass reads it: one fused launch per step each,
+        // the background's second state in arrays that only the passes after it use
         if (do_bg) {
             (void)hipMemsetAsync(w.bg.vx, 0, (size_t)w.n * 3 * 8, st);
             (void)hipMemsetAsync(w.bg2, 0, (size_t)w.n * 3 * 8, st);

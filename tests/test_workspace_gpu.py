@@ -4,6 +4,7 @@ A batch that fits a card has to go on fitting it, so what a call takes is held
 to what its wavefields, media and histories need:
   gradient        two FP64 and three FP32 split wavefields (15 arrays each),
                   9 medium arrays, and 8 floats of products or velocity copies
+  acoustic Born   16 FP32 and 3 FP64 arrays, 9 medium arrays, and the history
 plus images and records.  64 MB on top: some 30 allocations, each rounded up
 to 2 MB.  What the library keeps by itself is there before the measurement,
 from a small call of the same kind."""
@@ -54,5 +55,18 @@ def test_gradient(boundary):
     used = _used(call, nx, nz, 0, boundary)
     cells = (nx + 2 * PML) * (nz + 2 * PML)
     bound = cells * (2 * 15 * 8 + 3 * 15 * 4 + 9 * 4 + 8 * 4) + 7 * 4 * nx * nz + SLACK
+    print(f"{used / cells:.1f} B a cell, at most {bound / cells:.1f}")
+    assert used <= bound
+
+
+def test_acoustic_adjoint():
+    def call(s, shot, d):
+        s.born_adjoint([shot], d)
+
+    nx, nz = 4000, 1960
+    _used(call, 60, 40, 1, 1)
+    used = _used(call, nx, nz, 1, 1)
+    cells = (nx + 2 * PML) * (nz + 2 * PML)
+    bound = cells * (16 * 4 + 3 * 8 + 9 * 4) + 4 * nx * nz * (NT + 2) + SLACK
     print(f"{used / cells:.1f} B a cell, at most {bound / cells:.1f}")
     assert used <= bound
