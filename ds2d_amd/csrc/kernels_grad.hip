@@ -36,6 +36,7 @@
 // workgroup, sharing strains, 93 ms (145-227 VGPRs, one workgroup a CU).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "slot_address.hpp"
 #include "wave.hpp"
 
 namespace ds2d {
@@ -110,6 +111,7 @@ struct GradTile {
     static constexpr int COLS = 8, FS = (COLS + 2 * NOP) * 64;
     SlotDesc S;
     int lane, wv, x0, z, layer;
+    long long start, halo_start;  // of the wave's own and halo column
     bool zin, zupd;
     // Tile of this workgroup among zt x xt of each slot and layer; each XCD
     // (workgroups go round them) takes one range of them, so that the halo it
@@ -129,29 +131,26 @@ struct GradTile {
         z = zi * GROWS + lane;
         zin = z < S.nzp;
         zupd = lane >= NOP && lane < 64 - NOP && z < S.nzp - NOP;
+        start = uniform(column_start(S.off, col(), S.nzp));
+        halo_start = uniform(column_start(S.off, halo_col(), S.nzp));
         return x0 < S.nxp - NOP;
     }
+    // kept in scalar registers: else the compiler adds a lane's offset to it first, in 64-bit vector arithmetic
+    static __device__ __forceinline__ long long uniform(long long v) {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+        return (long long)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32)) << 32 | lo);
+    }
     __device__ __forceinline__ int col() const { return x0 + wv; }
+    __device__ __forceinline__ int halo_col() const { return wv < NOP ? x0 - NOP + wv : x0 + COLS + wv - NOP; }
     __device__ __forceinline__ bool own() const { return col() < S.nxp - NOP; }
-    // f at the lane's cell: the slot's start in scalar registers, 32 bits of
-    // byte offset within the slot (a slot of 2^29 cells would not fit the card)
-    template <typename T>
-    __device__ __forceinline__ T& in_slot(T* f, int ix) const {
-        const uint32_t c = (uint32_t)(ix * S.nzp + z);
-        return *reinterpret_cast<T*>(reinterpret_cast<char*>(f + S.off) + c * (uint32_t)sizeof(T));
-    }
-    template <typename T>
-    __device__ __forceinline__ const T& in_slot(const T* f, int ix) const {
-        return in_slot(const_cast<T*>(f), ix);
-    }
+    // f at the lane's cell
     template <typename T>
     __device__ __forceinline__ T& at(T* f) const {
-        return in_slot(f, col());
+        return column_cell(f, start, z);
     }
     // the lane's cell in an image window
     __device__ __forceinline__ float& window(float* w) const {
-        const uint32_t c = (uint32_t)((col() - S.pml) * S.nz + z - S.pml);
-        return *reinterpret_cast<float*>(reinterpret_cast<char*>(w + S.win_off) + c * 4u);
+        return column_cell(w, column_start(S.win_off, col() - S.pml, S.nz), z - S.pml);
     }
     __device__ __forceinline__ int place() const { return (wv + NOP) * 64 + lane; }
     // One mask each, without branches, and what a cell's kind decides is a
@@ -174,8 +173,7 @@ struct GradTile {
     }
     template <typename T>
     __device__ __forceinline__ T halo(const T* f) const {
-        const int ix = wv < NOP ? x0 - NOP + wv : x0 + COLS + wv - NOP;
-        return zin && ix < S.nxp ? in_slot(f, ix) : T(0);
+        return zin && halo_col() < S.nxp ? column_cell(f, halo_start, z) : T(0);
     }
     template <typename T>
     __device__ __forceinline__ void put(T* lds, const T& r, T h) const {
