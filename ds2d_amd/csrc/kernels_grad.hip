@@ -15,9 +15,10 @@
 //     (3) b stress and source, bb stress, the images.
 // Split PML memory is touched only where a damping profile can be non-zero;
 // elsewhere the split update equals the unsplit one.  A field that other
-// terms are added to (Born sources, Born adjoint, residuals: the next update
-// drops them, because it rebuilds the sum from the splits) keeps the bare
-// value of such cells in a split array and the sum in the field itself.
+// terms are added to (Born sources, Born adjoint: the next update drops them,
+// because it rebuilds the sum from the splits) keeps the bare value of such
+// cells in a split array and the sum in the field itself; a residual is added
+// where the stress reads the velocity, and kept nowhere.
 // The receiver side's derivatives of (moduli x stress) are taken of products
 // that the stress kernel writes once per cell instead of at all 8 taps.
 //
@@ -565,11 +566,31 @@ struct AdjStress {
     }
 };
 
+// The residuals of step it on top of the velocity of the lanes on the receiver
+// row: the sum over a column's traces, for the wave's own column and its halo one.
+__device__ __forceinline__ void add_residual(const GradTile& g, const GradArgs& a, int it, Vel2<float>& v) {
+    if (g.z != g.S.igz) return;
+#pragma unroll 1  // one copy of the loop's scalars: two take the kernel past 100 SGPRs and cost a workgroup a CU
+    for (int halo = 0; halo < 2; ++halo) {
+        const int ix = halo ? g.halo_col() : g.col();
+        if (ix >= g.S.nxp) continue;
+        float x = 0.f, z = 0.f;
+        for (int r = a.rmap[g.S.rmap_off + ix]; r >= 0; r = a.rnext ? a.rnext[g.S.rix_off + r] : -1) {
+            const size_t o = (size_t)g.S.rec_off + (size_t)r * a.nt + it;
+            z += a.rs_z[o];
+            x += a.rs_x[o];
+        }
+        (halo ? v.hx : v.vx) += x;
+        (halo ? v.hz : v.vz) += z;
+    }
+}
+
 // Backward launch 1 of step k: (0) bg stress one step back on the physical
 // window (FD2DGPU.cu:993-1082) with its strains, from the velocities that hold
 // step k's edge bands; (1) b velocity of step k+1 one step back
-// (FD2DGPU.cu:903-989), then step k's edge bands; (2) receiver-side stress and
-// the products the velocities differentiate.
+// (FD2DGPU.cu:903-989), then step k's edge bands; (2) receiver-side stress,
+// from the velocity with step k's residual on top, and the products that the
+// velocities differentiate.
 template <typename TB>
 __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m, GradArgs a,
                                                      const SlotDesc* __restrict__ slots, GradGrid gg, int k) {
@@ -660,6 +681,7 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
         dms.load(g, m.dms);
         cs.load(g, a.cs);
         ds.load(g, m);
+        add_residual(g, a, k, v);
         v.put(g, lf);
         __syncthreads();
         if (!g.own()) return;
@@ -679,64 +701,65 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
     }
 }
 
-// Receiver-side velocity (FD2DGPU.cu:591-682) from the products of its stress;
-// add_x and add_z go on top of the sum, and undamped cells that have such a
-// term (held) keep the bare velocity in vx_x and vz_z.
+// Receiver-side velocity (FD2DGPU.cu:591-682) from the products of its stress.
+// BORN: add_x and add_z go on top of the sum, and undamped cells keep the bare
+// velocity in vx_x and vz_z.
+template <bool BORN>
 struct AdjVel {
-    float p, q, pz, qz;
-    __device__ __forceinline__ void load(const GradTile& g, const EField& f, bool held) {
-        p = q = pz = qz = 0.f;
+    float x, z;            // the components of undamped cells, or (BORN) vx_x and vz_z of all
+    float xx, zz, xz, zx;  // vx_x, vz_z, vx_z, vz_x of damped cells
+    __device__ __forceinline__ void load(const GradTile& g, const EField& f) {
+        x = z = xx = zz = xz = zx = 0.f;
         if (!g.upd()) return;
-        const float* const hx = held ? f.vx_x : f.vx;  // one select per lane, not two arms
-        const float* const hz = held ? f.vz_z : f.vz;
-        p = g.at(hx);
-        q = g.at(hz);
+        x = g.at(BORN ? f.vx_x : f.vx);
+        z = g.at(BORN ? f.vz_z : f.vz);
         if (g.damped()) {
-            p = g.at(f.vx_x);
-            q = g.at(f.vz_x);
-            pz = g.at(f.vx_z);
-            qz = g.at(f.vz_z);
+            if (!BORN) {
+                xx = g.at(f.vx_x);
+                zz = g.at(f.vz_z);
+            }
+            xz = g.at(f.vx_z);
+            zx = g.at(f.vz_x);
         }
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
-                                         float kx, float kz, const Grad4<float>& t, bool held, float add_x,
-                                         float add_z) const {
+                                         float kx, float kz, const Grad4<float>& t, float add_x, float add_z) const {
         const float ax = kx * t.a, az = kz * t.b, bx = kx * t.e, bz = kz * t.d;
         float vx, vz;
         if (g.damped()) {
             const Damp<float> d(ds.x, ds.z, dt);
-            const float xx = (d.d1 * p - ax) * d.r2, xz = (d.d3 * pz - az) * d.r4;
-            const float zx = (d.d1 * q - bx) * d.r2, zz = (d.d3 * qz - bz) * d.r4;
-            g.at(f.vx_x) = xx;
-            g.at(f.vx_z) = xz;
-            g.at(f.vz_x) = zx;
-            g.at(f.vz_z) = zz;
-            vx = xx + xz;
-            vz = zx + zz;
+            const float nxx = (d.d1 * (BORN ? x : xx) - ax) * d.r2, nxz = (d.d3 * xz - az) * d.r4;
+            const float nzx = (d.d1 * zx - bx) * d.r2, nzz = (d.d3 * (BORN ? z : zz) - bz) * d.r4;
+            g.at(f.vx_x) = nxx;
+            g.at(f.vx_z) = nxz;
+            g.at(f.vz_x) = nzx;
+            g.at(f.vz_z) = nzz;
+            vx = nxx + nxz;
+            vz = nzx + nzz;
         } else {
-            vx = p - (ax + az);
-            vz = q - (bx + bz);
-            if (held) {
+            vx = x - (ax + az);
+            vz = z - (bx + bz);
+            if (BORN) {
                 g.at(f.vx_x) = vx;
                 g.at(f.vz_z) = vz;
             }
         }
-        g.at(f.vx) = vx + add_x;
-        g.at(f.vz) = vz + add_z;
+        g.at(f.vx) = BORN ? vx + add_x : vx;
+        g.at(f.vz) = BORN ? vz + add_z : vz;
     }
 };
 
 // Layers 1 and 2 of backward launch 2 (see there).
 template <bool BORN, typename TB>
 __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* lf, const EField& f, const float* w,
-                                                      const GradFields<TB>& F, const Med& m, const GradArgs& a, int k) {
+                                                      const GradFields<TB>& F, const Med& m, const GradArgs& a) {
     constexpr int FS = GradTile::FS;
     const long long n = a.n;
     Stress3<float> s;
-    AdjVel v;
+    AdjVel<BORN> v;
     DampState ds;
     float p0, p1, p2, cs, xz, hp, hc, hx, add_x = 0.f, add_z = 0.f;
-    bool held = BORN && g.interior();
+    const bool in = g.interior();  // formed here: after the barrier it takes the kernel from 61 to 74 VGPRs
     s.load(g, w, w + n, w + 2 * n);
     MedState rho;
     rho.load(g, m.rho);
@@ -750,18 +773,7 @@ __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* 
         hc = g.halo(a.cs);
         hx = g.halo(F.bk.txz);
     }
-    if (!BORN && g.upd() && g.z == g.S.igz) {
-        for (int r = a.rmap[g.S.rmap_off + g.col()]; r >= 0;
-             r = a.rnext ? a.rnext[g.S.rix_off + r] : -1) {
-            held = true;
-            if (k > 0) {
-                const size_t o = (size_t)g.S.rec_off + (size_t)r * a.nt + (k - 1);
-                add_z += a.rs_z[o];
-                add_x += a.rs_x[o];
-            }
-        }
-    }
-    v.load(g, f, held);
+    v.load(g, f);
     ds.load(g, m);
     s.put(g, lf);
     if constexpr (BORN) {
@@ -778,21 +790,20 @@ __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* 
         const float *C = lf + 3 * FS + g.place(), *X = lf + 4 * FS + g.place();
         const float odd = DS2D_C1 * (C[0] * (X[0] - X[-64])) + DS2D_C2 * (C[64] * (X[64] - X[-128])) +
                           DS2D_C3 * (C[128] * (X[128] - X[-192])) + DS2D_C4 * (C[192] * (X[192] - X[-256]));
-        if (held) {
+        if (in) {
             add_x = -br * (px * a.ix + p2z * a.iz);
             add_z = -br * (p1z * a.iz + odd * a.ix);
         }
     }
     if (!g.zupd) return;
-    v.step(g, f, ds, a.dt, br * a.kx, br * a.kz, t, held, add_x, add_z);
+    v.step(g, f, ds, a.dt, br * a.kx, br * a.kz, t, add_x, add_z);
 }
 
 // Backward launch 2 of step k: (0) bg velocity one step back, and in PML
 // windows the copy of it that holds step k-1's edge bands; (1) receiver-side
-// velocity with the residual of step k-1 on top; (2) the receiver-side Born
-// field's velocity with the Born adjoint (born.cu:408-527) on top.  txz's x
-// derivative there weights both taps with the modulus of the upper one
-// (born.cu:514-515), as in the reference.
+// velocity; (2) the receiver-side Born field's velocity with the Born adjoint
+// (born.cu:408-527) on top.  txz's x derivative there weights both taps with
+// the modulus of the upper one (born.cu:514-515), as in the reference.
 template <typename TB>
 __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m, GradArgs a,
                                                      const SlotDesc* __restrict__ slots, GradGrid gg, int k) {
@@ -844,9 +855,9 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m
         return;
     }
     if (layer == 1)
-        adjoint_velocity_tile<false, TB>(g, lf, F.bk, a.wk, F, m, a, k);
+        adjoint_velocity_tile<false, TB>(g, lf, F.bk, a.wk, F, m, a);
     else
-        adjoint_velocity_tile<true, TB>(g, lf, F.bb, a.wb, F, m, a, k);
+        adjoint_velocity_tile<true, TB>(g, lf, F.bb, a.wb, F, m, a);
 }
 
 // Backward launch 3 of step k: (0) b stress one step back with its strains and
@@ -951,9 +962,9 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_3(GradFields<TB> F, Med m
     }
 }
 
-// Start of the backward loop: the modulus of the Born adjoint's txz, the copy
-// of bg's velocity that holds the edge bands (PML windows; the last step's are
-// its own values), and the last step's residual on bk's receivers (at rest).
+// Start of the backward loop: the modulus of the Born adjoint's txz, and the
+// copy of bg's velocity that holds the edge bands (PML windows; the last step's
+// are its own values).
 template <typename TB>
 __global__ __launch_bounds__(256) void k_grad_bwd_0(GradFields<TB> F, Med m, GradArgs a,
                                                     const SlotDesc* __restrict__ slots) {
@@ -966,12 +977,6 @@ __global__ __launch_bounds__(256) void k_grad_bwd_0(GradFields<TB> F, Med m, Gra
         F.lvx[c] = F.bg.vx[c];
         F.lvz[c] = F.bg.vz[c];
     }
-    if (iz == S.igz)
-        for (int r = a.rmap[S.rmap_off + ix]; r >= 0; r = a.rnext ? a.rnext[S.rix_off + r] : -1) {
-            const size_t o = (size_t)S.rec_off + (size_t)r * a.nt + (a.nt - 1);
-            F.bk.vz[c] += a.rs_z[o];
-            F.bk.vx[c] += a.rs_x[o];
-        }
 }
 
 // ---------------------------------------------------------------------------
