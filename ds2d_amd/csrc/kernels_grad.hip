@@ -18,7 +18,12 @@
 // terms are added to (Born sources, Born adjoint: the next update drops them,
 // because it rebuilds the sum from the splits) keeps the bare value of such
 // cells in a split array and the sum in the field itself; a residual is added
-// where the stress reads the velocity, and kept nowhere.
+// where the stress reads the velocity, and kept nowhere.  The receiver side's
+// undamped sums of FP32 keep what they round off in a split array and take it
+// along in the next step (compensated summation): as one plain total instead of
+// two splits they were 4-6 % further from 64 bits in the images of the
+// receiver-side Born field (12 inputs each of 8 windows of 291x141 and one of
+// 141x101), so they are 4-7 % nearer than two splits, for 1 % of the time.
 // The receiver side's derivatives of (moduli x stress) are taken of products
 // that the stress kernel writes once per cell instead of at all 8 taps.
 //
@@ -530,7 +535,8 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_fwd_s(GradFields<TB> F, Med m
         stress_tile<float, TB, true>(g, (float*)(l + 2 * FS), l, F.b2, m, a, step, src, F.b.vx, F.b.vz);
 }
 
-// Receiver-side stress (FD2DGPU.cu:725-761, 860-895) of an updated cell.
+// Receiver-side stress (FD2DGPU.cu:725-761, 860-895) of an updated cell; txz_z of
+// an undamped one holds what the last sum of txz rounded off.
 struct AdjStress {
     float a, b, e, ez;
     __device__ __forceinline__ void load(const GradTile& g, const EField& f) {
@@ -539,10 +545,8 @@ struct AdjStress {
         a = g.at(f.txx);
         b = g.at(f.tzz);
         e = g.at(f.txz);
-        if (g.damped()) {
-            e = g.at(f.txz_x);
-            ez = g.at(f.txz_z);
-        }
+        ez = g.at(f.txz_z);
+        if (g.damped()) e = g.at(f.txz_x);
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
                                          float kx, float kz, const Taps<float>& t, float& xx, float& zz,
@@ -558,7 +562,9 @@ struct AdjStress {
         } else {
             xx = a - kx * t.xx;
             zz = b - kz * t.zz;
-            xz = e - (kx * t.xz + kz * t.zx);
+            const float d = -(kx * t.xz + kz * t.zx) - ez;
+            xz = e + d;
+            g.at(f.txz_z) = (xz - e) - d;
         }
         g.at(f.txx) = xx;
         g.at(f.tzz) = zz;
@@ -707,19 +713,20 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
 template <bool BORN>
 struct AdjVel {
     float x, z;            // the components of undamped cells, or (BORN) vx_x and vz_z of all
-    float xx, zz, xz, zx;  // vx_x, vz_z, vx_z, vz_x of damped cells
+    float xx, zz;          // vx_x and vz_z of damped cells
+    float xz, zx;          // vx_z and vz_x; of undamped cells, what the last sums of x and z rounded off
     __device__ __forceinline__ void load(const GradTile& g, const EField& f) {
         x = z = xx = zz = xz = zx = 0.f;
         if (!g.upd()) return;
         x = g.at(BORN ? f.vx_x : f.vx);
         z = g.at(BORN ? f.vz_z : f.vz);
-        if (g.damped()) {
-            if (!BORN) {
+        xz = g.at(f.vx_z);
+        zx = g.at(f.vz_x);
+        if (!BORN) {
+            if (g.damped()) {
                 xx = g.at(f.vx_x);
                 zz = g.at(f.vz_z);
             }
-            xz = g.at(f.vx_z);
-            zx = g.at(f.vz_x);
         }
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
@@ -737,8 +744,11 @@ struct AdjVel {
             vx = nxx + nxz;
             vz = nzx + nzz;
         } else {
-            vx = x - (ax + az);
-            vz = z - (bx + bz);
+            const float dx = -(ax + az) - xz, dz = -(bx + bz) - zx;
+            vx = x + dx;
+            vz = z + dz;
+            g.at(f.vx_z) = (vx - x) - dx;
+            g.at(f.vz_x) = (vz - z) - dz;
             if (BORN) {
                 g.at(f.vx_x) = vx;
                 g.at(f.vz_z) = vz;
