@@ -117,7 +117,16 @@ class RecordCopy {
                 share(i, t, of.load(std::memory_order_relaxed));
             }
         };
+        const auto start = [&](int i) {
+            const hipError_t e = hipMemcpyAsync(pin_ + (i & 1) * kPiece, todo[i].src, todo[i].bytes, hipMemcpyDeviceToHost, st);
+            return e != hipSuccess ? e : hipEventRecord(ev_[i & 1], st);
+        };
+        hipError_t e = start(0);
+        if (e == hipSuccess && n > 1) e = start(1);
+        // threads start once the first piece is there: until then the stream may have seconds of work before it
+        if (e == hipSuccess) e = hipEventSynchronize(ev_[0]);
         std::vector<std::thread> pool;
+        if (e != hipSuccess) helpers = 0;
         try {
             pool.reserve(helpers);
             for (; started < helpers; ++started) pool.emplace_back(help, started + 1);
@@ -125,15 +134,9 @@ class RecordCopy {
         }
         const int all = started + 1;
         of.store(all, std::memory_order_release);
-        const auto start = [&](int i) {
-            const hipError_t e = hipMemcpyAsync(pin_ + (i & 1) * kPiece, todo[i].src, todo[i].bytes, hipMemcpyDeviceToHost, st);
-            return e != hipSuccess ? e : hipEventRecord(ev_[i & 1], st);
-        };
-        hipError_t e = start(0);
         for (int i = 0; i < n && e == hipSuccess; ++i) {
-            if (i + 1 < n) {
-                if (i > 0)  // the other half still holds piece i - 1
-                    while (left[i - 1].load(std::memory_order_acquire) < all) std::this_thread::yield();
+            if (i > 0 && i + 1 < n) {  // the other half still holds piece i - 1
+                while (left[i - 1].load(std::memory_order_acquire) < all) std::this_thread::yield();
                 e = start(i + 1);
             }
             if (e == hipSuccess) e = hipEventSynchronize(ev_[i & 1]);
