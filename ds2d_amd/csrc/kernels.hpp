@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "tile_plan.hpp"
 
 namespace ds2d {
 
@@ -339,6 +340,7 @@ void launch_fused2_step(hipStream_t st, const BatchShape& b, const FusedArgs& a,
                         bool pml);
 
 // --- elastic step on tiles, two time steps per launch (kernels_tile.hip) ----
+static_assert(TILE_FRAME == NOP, "frame of the tile plan");
 // One tile: all that a workgroup needs of its window (one 64-byte load).
 struct TileDesc {
     long long off, rec_off;
@@ -349,14 +351,6 @@ struct TileDesc {
     int rmap_off;
     int pad[3];
 };
-constexpr int TILE_HALO = 16, TILE_ROWS = 64 - 2 * TILE_HALO, TILE_KINDS = 4;
-struct TilePlan {
-    int kind, cols;    // tile and its owned columns
-    long long rounds;  // rounds of one workgroup per CU
-    float us;          // estimate of one launch
-};
-// The tile whose rounds of the chip cost least for windows of nxp columns and nzp rows.
-TilePlan plan_tiles(const std::vector<int>& nxp, int nzp, int ncu);
 // Steps it .. it + ns - 1 (ns 1 or 2), state A -> B.
 void launch_tile_steps(hipStream_t st, const BatchShape& b, const FusedArgs& a, const TileDesc* tiles, int ntiles,
                        const int* rmap, int it, int ns, int kind, bool pml);

@@ -30,7 +30,6 @@
 #include "kernels.hpp"
 #include "wave.hpp"
 
-#include <algorithm>
 #include <type_traits>
 
 namespace ds2d {
@@ -269,29 +268,6 @@ __global__ __launch_bounds__(NW * 64) void k_tile_steps(FusedArgs a, const TileD
     }
 }
 
-// Columns per wave and waves of the four tiles, and what one round of one
-// workgroup per CU costs per launch of two steps (us, PML windows; measured
-// on 251x101 windows, 1 to 26 of them).
-struct TileKind {
-    int k, nw;
-    float us;
-};
-static const TileKind kTiles[TILE_KINDS] = {{3, 14, 9.2f}, {4, 12, 10.2f}, {4, 14, 12.1f}, {5, 12, 12.5f}};
-
-TilePlan plan_tiles(const std::vector<int>& nxp, int nzp, int ncu) {
-    TilePlan best{0, 0, 0, 0.f};
-    const long long zt = (std::max(nzp - 2 * NOP, 0) + TILE_ROWS - 1) / TILE_ROWS;
-    for (int v = 0; v < TILE_KINDS; ++v) {
-        const int cols = kTiles[v].k * kTiles[v].nw - 2 * TILE_HALO;
-        long long t = 0;
-        for (int w : nxp) t += (std::max(w - 2 * NOP, 0) + cols - 1) / cols * zt;
-        const long long rounds = (t + ncu - 1) / ncu;
-        const float us = rounds * kTiles[v].us;
-        if (v == 0 || us < best.us) best = TilePlan{v, cols, rounds, us};
-    }
-    return best;
-}
-
 void launch_tile_steps(hipStream_t st, const BatchShape& b, const FusedArgs& a, const TileDesc* tiles, int ntiles,
                        const int* rmap, int it, int ns, int kind, bool pml) {
     const int per_xcd = (ntiles + 7) / 8;
@@ -299,12 +275,13 @@ void launch_tile_steps(hipStream_t st, const BatchShape& b, const FusedArgs& a, 
 #define DS2D_TILE_LAUNCH(K, NW, MM)                                                                           \
     hipLaunchKernelGGL((k_tile_steps<K, NW, MM>), dim3(per_xcd * 8), dim3(NW * 64), 0, st, a, tiles, ntiles,  \
                        per_xcd, rmap, idx, idz, b.dt, b.nt, it, ns)
-#define DS2D_TILE_KIND(V, K, NW)                   \
-    case V:                                        \
-        if (pml)                                   \
-            DS2D_TILE_LAUNCH(K, NW, true);         \
-        else                                       \
-            DS2D_TILE_LAUNCH(K, NW, false);        \
+#define DS2D_TILE_KIND(V, K, NW)                                  \
+    case V:                                                       \
+        static_assert(kTiles[V].k == K && kTiles[V].nw == NW, ""); \
+        if (pml)                                                  \
+            DS2D_TILE_LAUNCH(K, NW, true);                        \
+        else                                                      \
+            DS2D_TILE_LAUNCH(K, NW, false);                       \
         break;
     switch (kind) {
         DS2D_TILE_KIND(0, 3, 14)
