@@ -7,7 +7,7 @@
 // pages are made while the device still computes (prepare), and the copy goes
 // through two pinned pieces, each emptied by several threads while the next
 // one arrives: 3.8 ms.  Below 8 MB the plain copy (17 GB/s, 0.5 ms) is kept: the
-// threads' start would cost as much.
+// threads' start would cost as much, and for destinations that HIP knows.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <sys/mman.h>
@@ -50,7 +50,7 @@ class RecordCopy {
     // n floats to each destination that is not null, complete on return.
     hipError_t fetch(hipStream_t st, size_t n, float* z, const float* dz, float* x, const float* dx) {
         const Piece whole[2] = {{(char*)z, (const char*)dz, z ? n * 4 : 0}, {(char*)x, (const char*)dx, x ? n * 4 : 0}};
-        if (whole[0].bytes + whole[1].bytes < kStaged || !staging()) {
+        if (whole[0].bytes + whole[1].bytes < kStaged || known(z) || known(x) || !staging()) {
             for (const Piece& q : whole) {
                 const hipError_t e = q.bytes ? hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, st) : hipSuccess;
                 if (e != hipSuccess) return e;
@@ -73,6 +73,15 @@ class RecordCopy {
     static constexpr size_t kPiece = 4u << 20;
     char* pin_ = nullptr;
     hipEvent_t ev_[2] = {nullptr, nullptr};
+
+    // Memory that HIP knows, which the runtime copies to at full rate by itself
+    // (pinned) and a host thread may not be able to write (device).
+    static bool known(const void* p) {
+        hipPointerAttribute_t a;
+        if (p && hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return false;
+    }
 
     bool staging() {
         for (hipEvent_t& e : ev_)

@@ -22,9 +22,16 @@ typedef int hipError_t;
 typedef void* hipStream_t;
 struct Event { size_t upto = 0; };
 typedef Event* hipEvent_t;
+enum { hipMemoryTypeUnregistered = 0, hipMemoryTypeDevice = 2 };
+struct hipPointerAttribute_t { int type; };
 enum { hipSuccess = 0, hipEventDisableTiming = 2, hipHostMallocDefault = 0, hipMemcpyDeviceToHost = 2 };
 struct Copy { void* d; const void* s; size_t n; };
 inline std::vector<Copy> queue_;
+inline const void* device_ = nullptr;
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    a->type = p == device_ ? hipMemoryTypeDevice : hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
 inline size_t done_ = 0;
 inline double busy_s = 0;
 inline hipError_t reach(size_t upto) {
@@ -50,6 +57,18 @@ inline hipError_t hipStreamSynchronize(hipStream_t) { return reach(queue_.size()
 SHIM = r'''
 #include <ctime>
 #include "record_copy.hpp"
+// copies straight to the caller's memory, of records whose z lies on the device
+extern "C" int direct(size_t n, float* z, const float* dz, float* x, const float* dx) {
+    queue_.clear();
+    done_ = 0;
+    device_ = z;
+    ds2d::RecordCopy rc;
+    const int e = rc.fetch(nullptr, n, z, dz, x, dx);
+    device_ = nullptr;
+    int k = 0;
+    for (const Copy& c : queue_) k += c.n == 4 * n && (c.d == z || c.d == x);
+    return e == hipSuccess && k == (int)queue_.size() ? k : -1;
+}
 // seconds of processor time of all threads
 extern "C" double fetch(size_t n, float* z, const float* dz, float* x, const float* dx, double busy) {
     busy_s = busy;
@@ -62,7 +81,7 @@ extern "C" double fetch(size_t n, float* z, const float* dz, float* x, const flo
 
 
 @pytest.fixture(scope="module")
-def fetch(tmp_path_factory):
+def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("copy")
     (d / "hip").mkdir()
     (d / "hip" / "hip_runtime.h").write_text(HIP)
@@ -70,7 +89,11 @@ def fetch(tmp_path_factory):
     so = d / "libcopy.so"
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-I", str(d), "-I",
                     os.path.join(ROOT, "ds2d_amd", "csrc"), str(d / "shim.cpp"), "-o", str(so)], check=True)
-    lib = C.CDLL(str(so))
+    return C.CDLL(str(so))
+
+
+@pytest.fixture(scope="module")
+def fetch(lib):
     lib.fetch.restype = C.c_double
     fp = C.POINTER(C.c_float)
     lib.fetch.argtypes = [C.c_size_t, fp, fp, fp, fp, C.c_double]
@@ -97,3 +120,13 @@ def test_nothing_spins_while_the_device_computes(fetch):
     cpu = fetch(2 << 20, True, 0.5)
     print(f"{cpu:.3f} s of processor time")
     assert cpu < 0.25
+
+
+def test_memory_that_hip_knows_is_left_to_it(lib):
+    """No thread writes to a destination on the device: one copy for each component, whole."""
+    n = 3 << 20
+    src = np.arange(2 * n, dtype=np.float32).reshape(2, n)
+    dst = np.zeros((2, n), np.float32)
+    p = lambda a: a.ctypes.data_as(C.POINTER(C.c_float))
+    assert lib.direct(C.c_size_t(n), p(dst[0]), p(src[0]), p(dst[1]), p(src[1])) == 2
+    assert np.array_equal(dst, src)
