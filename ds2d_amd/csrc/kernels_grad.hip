@@ -15,10 +15,10 @@
 //     (3) b stress and source, bb stress, the images.
 // Split PML memory is touched only where a damping profile can be non-zero;
 // elsewhere the split update equals the unsplit one.  A field that other
-// terms are added to (Born sources, Born adjoint: the next update drops them,
-// because it rebuilds the sum from the splits) keeps the bare value of such
-// cells in a split array and the sum in the field itself; a residual is added
-// where the stress reads the velocity, and kept nowhere.  The receiver side's
+// terms are added to (Born sources, Born adjoint, residuals: the next update
+// drops them, because it rebuilds the sum from the splits) keeps the bare
+// value of such cells in a split array and the sum in the field itself.  The
+// receiver side's
 // undamped sums of FP32 keep what they round off in a split array and take it
 // along in the next step (compensated summation): as one plain total instead of
 // two splits they were 4-6 % further from 64 bits in the images of the
@@ -572,31 +572,11 @@ struct AdjStress {
     }
 };
 
-// The residuals of step it on top of the velocity of the lanes on the receiver
-// row: the sum over a column's traces, for the wave's own column and its halo one.
-__device__ __forceinline__ void add_residual(const GradTile& g, const GradArgs& a, int it, Vel2<float>& v) {
-    if (g.z != g.S.igz) return;
-#pragma unroll 1  // one copy of the loop's scalars: two take the kernel past 100 SGPRs and cost a workgroup a CU
-    for (int halo = 0; halo < 2; ++halo) {
-        const int ix = halo ? g.halo_col() : g.col();
-        if (ix >= g.S.nxp) continue;
-        float x = 0.f, z = 0.f;
-        for (int r = a.rmap[g.S.rmap_off + ix]; r >= 0; r = a.rnext ? a.rnext[g.S.rix_off + r] : -1) {
-            const size_t o = (size_t)g.S.rec_off + (size_t)r * a.nt + it;
-            z += a.rs_z[o];
-            x += a.rs_x[o];
-        }
-        (halo ? v.hx : v.vx) += x;
-        (halo ? v.hz : v.vz) += z;
-    }
-}
-
 // Backward launch 1 of step k: (0) bg stress one step back on the physical
 // window (FD2DGPU.cu:993-1082) with its strains, from the velocities that hold
 // step k's edge bands; (1) b velocity of step k+1 one step back
-// (FD2DGPU.cu:903-989), then step k's edge bands; (2) receiver-side stress,
-// from the velocity with step k's residual on top, and the products that the
-// velocities differentiate.
+// (FD2DGPU.cu:903-989), then step k's edge bands; (2) receiver-side stress and
+// the products the velocities differentiate.
 template <typename TB>
 __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m, GradArgs a,
                                                      const SlotDesc* __restrict__ slots, GradGrid gg, int k) {
@@ -632,7 +612,7 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
     } else if (layer == 1) {
         if (k + 1 >= a.nt) return;  // the velocities are step k's already
         Stress3<TB> s;
-        TB vx = 0, vz = 0;
+        TB vx = 0, vz = 0, hx = 0, hz = 0;
         MedState rho;
         s.load(g, F.b.txx, F.b.tzz, F.b.txz);
         rho.load(g, m.rho);
@@ -641,13 +621,12 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
         // the physical window inside a band keep the bare velocity in vx_x and vz_z
         const bool held = band >= 0 && k + 2 < a.nt;
         if (g.upd()) {
-            if (held) {
-                vx = g.at(F.b.vx_x);
-                vz = g.at(F.b.vz_z);
-            } else {
-                vx = g.at(F.b.vx);
-                vz = g.at(F.b.vz);
-            }
+            vx = g.at(F.b.vx);
+            vz = g.at(F.b.vz);
+        }
+        if (held) {
+            hx = g.at(F.b.vx_x);
+            hz = g.at(F.b.vz_z);
         }
         s.put(g, l);
         __syncthreads();
@@ -658,8 +637,8 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
         const bool in = g.interior();
         if (in) {
             const TB br = TB(1) / (TB)rho.v;
-            vx -= br * kx * t.a + br * kz * t.b;
-            vz -= br * kx * t.e + br * kz * t.d;
+            vx = (held ? hx : vx) - (br * kx * t.a + br * kz * t.b);
+            vz = (held ? hz : vz) - (br * kx * t.e + br * kz * t.d);
         }
         if (band >= 0) {
             if (in) {
@@ -687,7 +666,6 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
         dms.load(g, m.dms);
         cs.load(g, a.cs);
         ds.load(g, m);
-        add_residual(g, a, k, v);
         v.put(g, lf);
         __syncthreads();
         if (!g.own()) return;
@@ -707,30 +685,35 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_1(GradFields<TB> F, Med m
     }
 }
 
-// Receiver-side velocity (FD2DGPU.cu:591-682) from the products of its stress.
-// BORN: add_x and add_z go on top of the sum, and undamped cells keep the bare
-// velocity in vx_x and vz_z.
+// Receiver-side velocity (FD2DGPU.cu:591-682) from the products of its stress;
+// add_x and add_z go on top of the sum, and undamped cells that may have such a
+// term (held: all with the Born adjoint, else receivers) keep the bare velocity
+// in vx_x and vz_z.
 template <bool BORN>
 struct AdjVel {
-    float x, z;            // the components of undamped cells, or (BORN) vx_x and vz_z of all
-    float xx, zz;          // vx_x and vz_z of damped cells
-    float xz, zx;          // vx_z and vz_x; of undamped cells, what the last sums of x and z rounded off
-    __device__ __forceinline__ void load(const GradTile& g, const EField& f) {
-        x = z = xx = zz = xz = zx = 0.f;
+    float x, z;    // the components of undamped cells, or (BORN) vx_x and vz_z of all
+    float hx, hz;  // vx_x and vz_z on a tile that has the receiver row
+    float xx, zz;  // vx_x and vz_z of damped cells
+    float xz, zx;  // vx_z and vz_x; of undamped cells, what the last sums of x and z rounded off
+    __device__ __forceinline__ void load(const GradTile& g, const EField& f, bool receivers) {
+        x = z = hx = hz = xx = zz = xz = zx = 0.f;
         if (!g.upd()) return;
         x = g.at(BORN ? f.vx_x : f.vx);
         z = g.at(BORN ? f.vz_z : f.vz);
         xz = g.at(f.vx_z);
         zx = g.at(f.vz_x);
-        if (!BORN) {
-            if (g.damped()) {
-                xx = g.at(f.vx_x);
-                zz = g.at(f.vz_z);
-            }
+        if (!BORN && receivers) {
+            hx = g.at(f.vx_x);
+            hz = g.at(f.vz_z);
+        }
+        if (!BORN && g.damped()) {
+            xx = g.at(f.vx_x);
+            zz = g.at(f.vz_z);
         }
     }
     __device__ __forceinline__ void step(const GradTile& g, const EField& f, const DampState& ds, float dt,
-                                         float kx, float kz, const Grad4<float>& t, float add_x, float add_z) const {
+                                         float kx, float kz, const Grad4<float>& t, bool held, float add_x,
+                                         float add_z) const {
         const float ax = kx * t.a, az = kz * t.b, bx = kx * t.e, bz = kz * t.d;
         float vx, vz;
         if (g.damped()) {
@@ -744,25 +727,26 @@ struct AdjVel {
             vx = nxx + nxz;
             vz = nzx + nzz;
         } else {
+            const float x0 = !BORN && held ? hx : x, z0 = !BORN && held ? hz : z;
             const float dx = -(ax + az) - xz, dz = -(bx + bz) - zx;
-            vx = x + dx;
-            vz = z + dz;
-            g.at(f.vx_z) = (vx - x) - dx;
-            g.at(f.vz_x) = (vz - z) - dz;
-            if (BORN) {
+            vx = x0 + dx;
+            vz = z0 + dz;
+            g.at(f.vx_z) = (vx - x0) - dx;
+            g.at(f.vz_x) = (vz - z0) - dz;
+            if (held) {
                 g.at(f.vx_x) = vx;
                 g.at(f.vz_z) = vz;
             }
         }
-        g.at(f.vx) = BORN ? vx + add_x : vx;
-        g.at(f.vz) = BORN ? vz + add_z : vz;
+        g.at(f.vx) = vx + add_x;
+        g.at(f.vz) = vz + add_z;
     }
 };
 
 // Layers 1 and 2 of backward launch 2 (see there).
 template <bool BORN, typename TB>
 __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* lf, const EField& f, const float* w,
-                                                      const GradFields<TB>& F, const Med& m, const GradArgs& a) {
+                                                      const GradFields<TB>& F, const Med& m, const GradArgs& a, int k) {
     constexpr int FS = GradTile::FS;
     const long long n = a.n;
     Stress3<float> s;
@@ -783,7 +767,26 @@ __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* 
         hc = g.halo(a.cs);
         hx = g.halo(F.bk.txz);
     }
-    v.load(g, f);
+    // whether the tile has the receiver row: uniform, so that what such a cell starts from is chosen by value
+    const int row = g.S.igz - (g.z - g.lane);
+    const bool receivers = !BORN && g.own() && row >= 0 && row < 64;
+    bool held = BORN;
+    v.load(g, f, receivers);
+    if (receivers) {
+        float x = 0.f, z = 0.f;
+        bool any = false;
+        for (int r = a.rmap[g.S.rmap_off + g.col()]; r >= 0; r = a.rnext ? a.rnext[g.S.rix_off + r] : -1) {
+            any = true;
+            if (k > 0) {
+                const size_t o = (size_t)g.S.rec_off + (size_t)r * a.nt + (k - 1);
+                z += a.rs_z[o];
+                x += a.rs_x[o];
+            }
+        }
+        held = any && g.z == g.S.igz;
+        add_x = held ? x : 0.f;
+        add_z = held ? z : 0.f;
+    }
     ds.load(g, m);
     s.put(g, lf);
     if constexpr (BORN) {
@@ -806,14 +809,15 @@ __device__ __forceinline__ void adjoint_velocity_tile(const GradTile& g, float* 
         }
     }
     if (!g.zupd) return;
-    v.step(g, f, ds, a.dt, br * a.kx, br * a.kz, t, add_x, add_z);
+    v.step(g, f, ds, a.dt, br * a.kx, br * a.kz, t, held, add_x, add_z);
 }
 
 // Backward launch 2 of step k: (0) bg velocity one step back, and in PML
 // windows the copy of it that holds step k-1's edge bands; (1) receiver-side
-// velocity; (2) the receiver-side Born field's velocity with the Born adjoint
-// (born.cu:408-527) on top.  txz's x derivative there weights both taps with
-// the modulus of the upper one (born.cu:514-515), as in the reference.
+// velocity with the residual of step k-1 on top; (2) the receiver-side Born
+// field's velocity with the Born adjoint (born.cu:408-527) on top.  txz's x
+// derivative there weights both taps with the modulus of the upper one
+// (born.cu:514-515), as in the reference.
 template <typename TB>
 __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m, GradArgs a,
                                                      const SlotDesc* __restrict__ slots, GradGrid gg, int k) {
@@ -865,9 +869,9 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_2(GradFields<TB> F, Med m
         return;
     }
     if (layer == 1)
-        adjoint_velocity_tile<false, TB>(g, lf, F.bk, a.wk, F, m, a);
+        adjoint_velocity_tile<false, TB>(g, lf, F.bk, a.wk, F, m, a, k);
     else
-        adjoint_velocity_tile<true, TB>(g, lf, F.bb, a.wb, F, m, a);
+        adjoint_velocity_tile<true, TB>(g, lf, F.bb, a.wb, F, m, a, k);
 }
 
 // Backward launch 3 of step k: (0) b stress one step back with its strains and
@@ -972,9 +976,9 @@ __global__ __launch_bounds__(GTHREADS) void k_grad_bwd_3(GradFields<TB> F, Med m
     }
 }
 
-// Start of the backward loop: the modulus of the Born adjoint's txz, and the
-// copy of bg's velocity that holds the edge bands (PML windows; the last step's
-// are its own values).
+// Start of the backward loop: the modulus of the Born adjoint's txz, the copy
+// of bg's velocity that holds the edge bands (PML windows; the last step's are
+// its own values), and the last step's residual on bk's receivers (at rest).
 template <typename TB>
 __global__ __launch_bounds__(256) void k_grad_bwd_0(GradFields<TB> F, Med m, GradArgs a,
                                                     const SlotDesc* __restrict__ slots) {
@@ -987,6 +991,12 @@ __global__ __launch_bounds__(256) void k_grad_bwd_0(GradFields<TB> F, Med m, Gra
         F.lvx[c] = F.bg.vx[c];
         F.lvz[c] = F.bg.vz[c];
     }
+    if (iz == S.igz)
+        for (int r = a.rmap[S.rmap_off + ix]; r >= 0; r = a.rnext ? a.rnext[S.rix_off + r] : -1) {
+            const size_t o = (size_t)S.rec_off + (size_t)r * a.nt + (a.nt - 1);
+            F.bk.vz[c] += a.rs_z[o];
+            F.bk.vx[c] += a.rs_x[o];
+        }
 }
 
 // ---------------------------------------------------------------------------
