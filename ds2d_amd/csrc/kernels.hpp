@@ -119,7 +119,6 @@ void launch_acou_adj_p(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouF
                        const float* hist, int it);
 void launch_acou_adj_v(hipStream_t st, const BatchShape& b, AcouFieldD bg, AcouField lam, AcouMed m,
                        const float* wav, int it, int do_bg, const int* rmap, const float* res);
-struct ChunkDesc;
 // Fused plain acoustic steps (kernels_acoustic_tile.hip): state A -> B, each
 // 3 fields (vx, vz, p) of n floats from the base pointer.
 struct AcouFusedArgs {

@@ -13,10 +13,10 @@
 // (32 columns of 64 rows, four columns a wave), so a step is one memory
 // latency, two LDS exchanges of x neighbours and wave shifts for z.  Eight
 // columns and rows on each side are halo (four for the velocity, four for the
-// pressure).  Measured per step: 26 windows of 331x181 Born 19.3 -> 15.9 us,
-// adjoint 21.1 -> 17.8, background 49 (two per-cell kernels) -> 18.6; 16 of
-// 592x336 adjoint 92 (per-cell) -> 32.6, background 56 -> 31.7; one of 331x181
-// 5.3 us a step.  Tiles of 48 and 64 columns have less halo but measured up to
+// pressure).  Measured per step: 26 windows of 331x181 Born 19.3 -> 14.2 us,
+// adjoint 21.1 -> 16.4, background 49 (two per-cell kernels) -> 18.0; 16 of
+// 592x336 adjoint 92 (per-cell) -> 30.2, background 56 -> 30.8; one of 331x181
+// about 5 us a step.  40-58 registers and 20 KB of LDS: four workgroups a CU.  Tiles of 48 and 64 columns have less halo but measured up to
 // 40 % slower below 1 M cells and 0-10 % faster above (FP64: slower throughout);
 // one wave per strip without LDS marched no faster (18.7-21 us): its halo
 // columns are computed again by every strip.

@@ -14,15 +14,18 @@
 // rows per wave and unit, exchanges x neighbours through LDS (twice a step) and
 // reads z neighbours with wave shifts; eight columns and rows on each side are
 // halo.  Measured per pass: PP/PS CG on 8 windows of 592x336 with the history
-// 77.8 -> 24 ms (adjoint step 116 -> 32 us, forward 118 -> 35, background alone
-// 36 in two per-cell kernels before); one of 141x101 54.9 -> 5.3 ms; forward on
+// 77.8 -> 24 ms (adjoint step 116 -> 29 us, forward 118 -> 34, scattered field
+// alone 25); one of 141x101 54.9 -> 5.3 ms; forward on
 // 16 windows of 440-1240 x 1080 392 -> 350 us a step (4.3 TB/s of the 100 B),
 // adjoint with reversal on 8 of them 208 -> 193 us.
 // Width: 32 owned columns (six units, two workgroups of 126 registers a CU)
 // have less halo, 16 (four units) more workgroups.  Narrow: 24.0 against 25.1 ms on
 // the 8 windows (1064 wide tiles), 5.3 against 6.7 on one; wide: 56.1 against
 // 59.3 ms on the 16 large windows (9900 tiles), 41.8 against 55.3 for the
-// adjoint of 8 (5000).  Hence the line at 2048 wide tiles.
+// adjoint of 8 (5000).  Hence the line at 2048 wide tiles; between 1100 and
+// 5000 it is not measured.  The narrow adjoint with the reversal takes 129
+// registers, and so one workgroup a CU: still 22 us a step on one window of
+// 592x336 and 124 on 16 against 139 and 238 with the march.
 #include <algorithm>
 
 #include "common.hpp"

@@ -21,9 +21,9 @@
 // receiver side's
 // undamped sums of FP32 keep what they round off in a split array and take it
 // along in the next step (compensated summation): as one plain total instead of
-// two splits they were 4-6 % further from 64 bits in the images of the
+// two splits they were 5-6 % further from 64 bits in the images of the
 // receiver-side Born field (12 inputs each of 8 windows of 291x141 and one of
-// 141x101), so they are 4-7 % nearer than two splits, for 1 % of the time.
+// 141x101), so they are 4-7 % nearer than two splits, for 0.5 % of the time.
 // The receiver side's derivatives of (moduli x stress) are taken of products
 // that the stress kernel writes once per cell instead of at all 8 taps.
 //
@@ -33,10 +33,10 @@
 // cell a thread with all eight taps from memory (35 loads a cell and field) took
 // 20.6-37.5 us a launch there, 126 a step of both loops.  Here a wave holds a
 // column of 64 rows, loads every operand once and ahead, and takes x taps from
-// LDS and z taps by wave shifts; slots are addressed by 32-bit offsets from
-// scalar bases, and neighbouring tiles share an XCD's L2: 16.0-26.1 us, 95 a
-// step.  8 shots x 700 steps 89.7 -> 70 ms (148 with a launch per operation),
-// one 141x101 window x 400 steps 11.0 -> 10.0, 26 shots x 100 steps 33.  Two
+// LDS and z taps by wave shifts; columns are addressed by 32-bit offsets from
+// scalar bases, and neighbouring tiles share an XCD's L2: 16.6-27.2 us, 99 a
+// step.  8 shots x 700 steps 89.7 -> 70.4 ms (148 with a launch per operation),
+// one 141x101 window x 400 steps 11.0 -> 10.1, 26 shots x 100 steps 34.  Two
 // columns a wave lose more to occupancy (76 ms) than they save in halo columns,
 // 16 waves to a workgroup likewise (81 ms); all fields of a launch in one
 // workgroup, sharing strains, 93 ms (145-227 VGPRs, one workgroup a CU).

@@ -25,7 +25,10 @@
 // Vector operations bound the PML step (1700 a wave of three columns), so the
 // addresses are 32-bit offsets from scalar bases and cells beyond the update
 // region rest for want of a medium instead of being masked: 10.3 -> 9.4 us from
-// launch to launch on 291x141, 16 such windows 49.8 -> 45.7.
+// launch to launch on 291x141, 16 such windows 49.8 -> 45.7.  (A state that has
+// overflowed reaches the frame that way a step before it would by the taps.)
+// The PML tiles of 24 and 28 columns spill 36 and 44 bytes a lane at the 128 and
+// 168 registers that their 14 and 12 waves leave.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "wave.hpp"

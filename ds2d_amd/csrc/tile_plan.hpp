@@ -12,7 +12,8 @@ constexpr int TILE_HALO = 16, TILE_ROWS = 64 - 2 * TILE_HALO, TILE_KINDS = 4, TI
 
 // Columns per wave and waves of the four tiles, and what one round of one
 // workgroup per CU costs per launch of two steps (us, PML windows; measured
-// on 251x101 windows, 1 to 26 of them).
+// on 251x101 windows, 1 to 26 of them; windows with the random boundary, whose
+// launches take three quarters of that, are planned by the same costs).
 struct TileKind {
     int k, nw;
     float us;

@@ -88,7 +88,8 @@ typedef struct {
     int isx, isz;           /* source cell, padded-window coordinates           */
     int igz;                /* receiver row, padded coordinates (pml + gy)      */
     int ntr;                /* number of traces                                 */
-    const int* rec_ix;      /* [ntr] receiver columns, padded coordinates       */
+    const int* rec_ix;      /* [ntr] receiver columns, padded coordinates; a column
+                               may have several traces                          */
     int shot_id;            /* seeds the random boundary of this shot           */
     int boundary;           /* 0 PML, 1 random boundary                         */
 } ds2d_shot;
