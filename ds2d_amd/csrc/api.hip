@@ -159,7 +159,7 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     long long off = 0, roff = 0, woff = 0, eoff = 0, moff = 0;
     int rixo = 0, max_nxp = 0, max_ntr = 0;
     bool repeated = false;
-    std::vector<int> last;  // last trace of each column of a window
+    std::vector<int> seen;  // last shot with a trace on a column
     for (int s = 0; s < nshots; ++s) {
         const ds2d_shot& q = shots[s];
         if (q.nx <= 0 || q.ngx_min < 0 || q.ngx_min + q.nx > g.allnx)
@@ -207,13 +207,11 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
         B.total_hist += (long long)g.nt * q.nx * g.allnz;
         B.tbase.push_back(B.total_traces);
         B.total_traces += q.ntr;
-        last.assign(nxp, -1);
+        seen.resize(std::max<size_t>(seen.size(), nxp), -1);
         for (int r = 0; r < q.ntr; ++r) {
-            int& t = last[q.rec_ix[r]];
-            repeated = repeated || t >= 0;
             B.rix.push_back(q.rec_ix[r]);
-            B.rnext.push_back(t);
-            t = r;
+            repeated = repeated || seen[q.rec_ix[r]] == s;
+            seen[q.rec_ix[r]] = s;
         }
         rixo += q.ntr;
         max_nxp = std::max(max_nxp, nxp);
@@ -240,12 +238,19 @@ int build_batch(ds2d_ctx* h, int nshots, const ds2d_shot* shots, Batch& B) {
     sh.rix = d_rix;
     sh.rnext = nullptr;
     if (repeated) {
+        std::vector<int> last;  // last trace of each column of a window
+        for (const SlotDesc& S : B.slots) {
+            last.assign(S.nxp, -1);
+            for (int r = 0; r < S.ntr; ++r) {
+                int& t = last[B.rix[S.rix_off + r]];
+                B.rnext.push_back(t);
+                t = r;
+            }
+        }
         int* d_next;
         if ((rc = h->fbuf("rnext", B.rnext.size(), &d_next))) return rc;
         HIP_TRY(hipMemcpyAsync(d_next, B.rnext.data(), B.rnext.size() * sizeof(int), hipMemcpyHostToDevice, h->st));
         sh.rnext = d_next;
-    } else {
-        B.rnext.clear();
     }
     sh.nslots = nshots;
     sh.max_nxp = max_nxp;
