@@ -2632,6 +2632,8 @@ int ds2d_rot_rtm(ds2d_t* h, int nshots, const ds2d_shot* shots, const float* rec
     if ((rc = upload_records(h, B, "obs_z", rec_z, &dz)) || (rc = upload_records(h, B, "obs_x", rec_x, &dx)))
         return rc;
     if ((rc = h->fbuf("rot_win", (size_t)B.total_win * 2, &w2))) return rc;
+    int* rmap;
+    if ((rc = column_traces(h, B, "rmap", &rmap))) return rc;
     HIP_TRY(hipMemsetAsync(w2, 0, (size_t)B.total_win * 2 * 4, st));
     stats_begin(h);
     stats_loop_begin(h);
@@ -2646,7 +2648,7 @@ int ds2d_rot_rtm(ds2d_t* h, int nshots, const ds2d_shot* shots, const float* rec
         launch_rot_src(st, sh, f.th, h->d_wav, it);
         launch_rot_v(st, sh, f, m, -1.f);
         launch_rot_v(st, sh, b, m, 1.f);
-        launch_rot_inject(st, sh, b.vz, b.vx, dz, dx, it);
+        launch_rot_inject(st, sh, b.vz, b.vx, dz, dx, rmap, it);
         launch_rot_p(st, sh, b, m, 1.f);
         launch_rot_image(st, sh, f, b, w2, B.total_win);
     }
@@ -2674,6 +2676,8 @@ int ds2d_decomp_rtm(ds2d_t* h, int nshots, const ds2d_shot* shots, int kind, con
     if ((rc = h->fbuf("decomp_hist", (size_t)nt * W * K, &hist))) return rc;
     if ((rc = h->fbuf("rot_win", (size_t)W, &win))) return rc;
     if ((rc = upload_records(h, B, "obs_z", rec_z, &dz))) return rc;
+    int* rmap;
+    if ((rc = column_traces(h, B, "rmap", &rmap))) return rc;
     float *VP = vps, *VS = vps + n;
     HIP_TRY(hipMemsetAsync(vps, 0, (size_t)n * 2 * 4, st));
     HIP_TRY(hipMemsetAsync(win, 0, (size_t)W * 4, st));
@@ -2690,7 +2694,7 @@ int ds2d_decomp_rtm(ds2d_t* h, int nshots, const ds2d_shot* shots, int kind, con
     HIP_TRY(hipMemsetAsync(f.vx, 0, (size_t)n * 15 * 4, st));
     HIP_TRY(hipMemsetAsync(vps, 0, (size_t)n * 2 * 4, st));
     for (int it = nt - 1; it >= 0; --it) {
-        launch_assign_rec(st, sh, f.txx, f.tzz, dz, it);
+        launch_assign_rec(st, sh, f.txx, f.tzz, dz, rmap, it);
         launch_ref_v(st, sh, f, m);
         launch_helmholtz(st, sh, f.vx, f.vz, VP, VS);
         if (it < nt - 1) launch_decomp(st, sh, kind, VP, VS, f, hist + (size_t)it * W * K, win, 0);

@@ -286,7 +286,7 @@ void launch_rot_src(hipStream_t st, const BatchShape& b, double* th, const float
 void launch_rot_image(hipStream_t st, const BatchShape& b, RotFieldD src, RotFieldD rcv, float* w2, long long wstride);
 // vz += rec_z, vx += rec_x at the receivers (FP64 receiver field of the rotation RTM).
 void launch_rot_inject(hipStream_t st, const BatchShape& b, double* vz, double* vx, const float* rz, const float* rx,
-                       int it);
+                       const int* rmap, int it);
 void launch_helmholtz(hipStream_t st, const BatchShape& b, const float* vx, const float* vz, float* VP, float* VS);
 // Floats per window cell and step of a decomposed image kind (0..6).
 int decomp_floats(int kind);
@@ -296,7 +296,8 @@ int decomp_floats(int kind);
 void launch_decomp(hipStream_t st, const BatchShape& b, int kind, const float* VP, const float* VS, EField f,
                    float* hist, float* win, int store);
 // txx = tzz = rec_z[tr][it] at each receiver (assignment).
-void launch_assign_rec(hipStream_t st, const BatchShape& b, float* txx, float* tzz, const float* rz, int it);
+void launch_assign_rec(hipStream_t st, const BatchShape& b, float* txx, float* tzz, const float* rz, const int* rmap,
+                       int it);
 
 // --- fused single-kernel elastic step (kernels_fused.hip) -------------------
 struct ChunkDesc {

@@ -150,17 +150,24 @@ __global__ __launch_bounds__(256) void k_rot_image(const TS* __restrict__ spx, c
 }
 
 // GPUapplysource_backward_from_record with stack (FD2DGPU.cu:3306-3327):
-// vz += rec_z[tr][it], vx += rec_x[tr][it] at each receiver.
+// vz += rec_z[tr][it], vx += rec_x[tr][it] at each receiver; a column's last
+// trace takes all of them.
 template <typename T>
 __global__ void k_rot_inject(T* vz, T* vx, const float* __restrict__ rz, const float* __restrict__ rx,
-                             const int* __restrict__ rix, const SlotDesc* __restrict__ slots, int nt, int it) {
+                             const int* __restrict__ rix, const int* __restrict__ rmap, const int* __restrict__ rnext,
+                             const SlotDesc* __restrict__ slots, int nt, int it) {
     const SlotDesc S = slots[blockIdx.y];
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= S.ntr) return;
+    if (r >= S.ntr || rmap[S.rmap_off + rix[S.rix_off + r]] != r) return;
     const size_t c = (size_t)S.off + (size_t)rix[S.rix_off + r] * S.nzp + S.igz;
-    const size_t o = (size_t)S.rec_off + (size_t)r * nt + it;
-    vz[c] += (T)rz[o];
-    vx[c] += (T)rx[o];
+    T z = vz[c], x = vx[c];
+    for (int q = r; q >= 0; q = rnext ? rnext[S.rix_off + q] : -1) {
+        const size_t o = (size_t)S.rec_off + (size_t)q * nt + it;
+        z += (T)rz[o];
+        x += (T)rx[o];
+    }
+    vz[c] = z;
+    vx[c] = x;
 }
 
 // FD2DGPU.cu:1963-1986: VP = div v, VS = d(vx)/dz - d(vz)/dx on the
@@ -267,12 +274,13 @@ __global__ __launch_bounds__(256) void k_decomp(const float* __restrict__ VP, co
 }
 
 // FD2DGPU.cu:2128-2134 GPUapplysource_backward: the receiver records are
-// assigned (not added) to txx and tzz at each receiver.
+// assigned (not added) to txx and tzz at each receiver, of several traces on a
+// column the last one's.
 __global__ void k_assign_rec(float* txx, float* tzz, const float* __restrict__ rz, const int* __restrict__ rix,
-                             const SlotDesc* __restrict__ slots, int nt, int it) {
+                             const int* __restrict__ rmap, const SlotDesc* __restrict__ slots, int nt, int it) {
     const SlotDesc S = slots[blockIdx.y];
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= S.ntr) return;
+    if (r >= S.ntr || rmap[S.rmap_off + rix[S.rix_off + r]] != r) return;
     const size_t c = (size_t)S.off + (size_t)rix[S.rix_off + r] * S.nzp + S.igz;
     const float v = rz[(size_t)S.rec_off + (size_t)r * nt + it];
     txx[c] = v;
@@ -316,9 +324,9 @@ void launch_rot_image(hipStream_t st, const BatchShape& b, RotFieldD src, RotFie
                        rcv.vpz, rcv.vsx, rcv.vsz, w2, wstride, b.slots);
 }
 void launch_rot_inject(hipStream_t st, const BatchShape& b, double* vz, double* vx, const float* rz, const float* rx,
-                       int it) {
+                       const int* rmap, int it) {
     hipLaunchKernelGGL(k_rot_inject<double>, dim3(ceil_div(b.max_ntr, 64), b.nslots), dim3(64), 0, st, vz, vx, rz, rx,
-                       b.rix, b.slots, b.nt, it);
+                       b.rix, rmap, b.rnext, b.slots, b.nt, it);
 }
 void launch_helmholtz(hipStream_t st, const BatchShape& b, const float* vx, const float* vz, float* VP, float* VS) {
     hipLaunchKernelGGL(k_helmholtz, rot_grid(b), dim3(BZ, BX), 0, st, vx, vz, VP, VS, b.slots, b.dx, b.dz);
@@ -340,9 +348,10 @@ void launch_decomp(hipStream_t st, const BatchShape& b, int kind, const float* V
     }
 #undef DS2D_DECOMP
 }
-void launch_assign_rec(hipStream_t st, const BatchShape& b, float* txx, float* tzz, const float* rz, int it) {
+void launch_assign_rec(hipStream_t st, const BatchShape& b, float* txx, float* tzz, const float* rz, const int* rmap,
+                       int it) {
     hipLaunchKernelGGL(k_assign_rec, dim3(ceil_div(b.max_ntr, 64), b.nslots), dim3(64), 0, st, txx, tzz, rz, b.rix,
-                       b.slots, b.nt, it);
+                       rmap, b.slots, b.nt, it);
 }
 
 }  // namespace ds2d

@@ -143,3 +143,28 @@ def test_least_squares_migration_of_repeated_traces():
     assert np.abs(resid[1] - want) <= 2 * NT * 2.0 ** -23 * max(1.0, want)
     assert np.linalg.norm(img - step * g) <= 2 * NT * 2.0 ** -23 * np.linalg.norm(step * g)
     s.close()
+
+
+def test_rotation_rtm():
+    """The receiver side adds every trace's sample."""
+    twice, once, _ = _pair(1)
+    (rz, tz), (rx, tx) = _residuals(6), _residuals(7)
+    s = _solver()
+    a, b = s.rot_rtm(once, tz, tx), s.rot_rtm(twice, rz, rx)
+    for i in range(2):
+        assert np.abs(a[i]).max() > 0 and np.array_equal(a[i], b[i])
+    s.close()
+
+
+@pytest.mark.parametrize("boundary", [0, 1])
+def test_decomposed_rtm(boundary):
+    """The receiver side assigns the samples, of several on a cell the last trace's, as one after another would."""
+    twice, once, place = _pair(boundary)
+    r = np.random.default_rng(4).standard_normal((place.size, NT)).astype(np.float32)
+    last = np.zeros((sum(sh.ntr for sh in once), NT), np.float32)
+    for t, p in enumerate(place):
+        last[p] = r[t]
+    s = _solver()
+    a, b = s.decomp_rtm(once, 0, last.ravel()), s.decomp_rtm(twice, 0, r.ravel())
+    assert np.abs(a).max() > 0 and np.array_equal(a, b)
+    s.close()
